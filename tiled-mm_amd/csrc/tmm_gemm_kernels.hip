@@ -542,6 +542,31 @@ __global__ __launch_bounds__(256, 2) void gemm_cplx_kernel(GemmParams<R> prm) {
 
 
 // ---------------------------------------------------------------------------------------------
+// The last k-step of the pipelined kernels. Their ring reads whole k-steps of BK values in 16-byte
+// chunks; a partial last step, or (for a row-contiguous operand whose row count is no multiple of
+// the chunk's CH rows) a last step whose final column has no room for a whole chunk behind it, is
+// instead read element by element, straight from global memory into fragments, and multiplied
+// first, while the ring's first stages are on their way. One launch then takes any k and any row
+// count; before, a remainder of k was a launch of its own (a second pass over C) and odd row
+// counts ran on the register-staged kernel (FP64 TT 6222 x 6255 x 3501: 4.97 ms).
+// ---------------------------------------------------------------------------------------------
+__device__ __forceinline__ int ring_steps(int k, int bk, bool ragged) { return ragged ? (k - 1) / bk : k / bk; }
+
+// KV consecutive k values of one row from k on, zero from k_end on; W reals per element.
+template <bool KC, int KV, int W, typename V, typename R>
+__device__ __forceinline__ V last_frag(const R* __restrict__ p, long ld, int row, int nrows, int k, int k_end) {
+  V v;
+  const int r = min(row, nrows - 1);
+#pragma unroll
+  for (int e = 0; e < KV; ++e) {
+    const R* q = p + (KC ? (long)(k + e) + (long)r * ld : (long)r + (long)(k + e) * ld) * W;
+#pragma unroll
+    for (int w = 0; w < W; ++w) v[e * W + w] = k + e < k_end ? q[w] : R(0);
+  }
+  return v;
+}
+
+// ---------------------------------------------------------------------------------------------
 // FP64 GEMM with direct global->LDS loads (global_load_lds_dwordx4) into an S-stage LDS ring.
 // WG tile 128x128, 2x2 waves of 64x64, k-step 8 per stage, S stages of 16 KB (S = 3, three
 // workgroups per CU).
@@ -739,10 +764,10 @@ struct SdldsOperand {
         src = p + (long)(4 * q + k0) + (long)row * ld;
       } else if (ROWS == 128) {  // 128 rows at two k
         const int kk = 2 * inst + (lane >> 5);
-        const int row = min(r0 + 4 * (lane & 31), nrows - 4);
+        const int row = min(r0 + 4 * (lane & 31), (nrows - 1) & ~3);
         src = p + (long)row + (long)(k0 + kk) * ld;
       } else {  // 256 rows at one k
-        const int row = min(r0 + 4 * lane, nrows - 4);
+        const int row = min(r0 + 4 * lane, (nrows - 1) & ~3);
         src = p + (long)row + (long)(k0 + inst) * ld;
       }
       __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
@@ -856,7 +881,8 @@ __device__ __forceinline__ void spipe_tile_at(const GemmParams<float>& prm, int 
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int wm = wave % WM, wn = wave / WM;
   const int li = lane & 15, lg = lane >> 4;
-  const int nkt = K / 16;
+  const bool ragged = K % 16 != 0 || (!A_KC && M % 4 != 0) || (!B_KC && N % 4 != 0);
+  const int nkt = ring_steps(K, 16, ragged);
 
   flt4 acc[4][TJ];
 #pragma unroll
@@ -877,6 +903,21 @@ __device__ __forceinline__ void spipe_tile_at(const GemmParams<float>& prm, int 
 #pragma unroll
     for (int j = 0; j < TJ; ++j) f.b[j] = OpB::frag(st + A_ELEMS, lg, wn * TN + j * 16 + li);
   };
+  if (ragged) {
+    Frags f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      f.a[i] = last_frag<A_KC, 4, 1, v4f>(prm.a, prm.lda, m0 + wm * 64 + i * 16 + li, M, nkt * 16 + 4 * lg, K);
+#pragma unroll
+    for (int j = 0; j < TJ; ++j)
+      f.b[j] = last_frag<B_KC, 4, 1, v4f>(prm.b, prm.ldb, n0 + wn * TN + j * 16 + li, N, nkt * 16 + 4 * lg, K);
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) acc[i][j] = mfma(f.b[j][t], f.a[i][t], acc[i][j]);
+  }
   if (nkt > 0) {
 #pragma unroll
     for (int s = 0; s < S; ++s) issue(min(s, nkt - 1), s * STAGE);
@@ -1039,7 +1080,7 @@ struct CdldsOperand {
         const int row = min(r0 + local, nrows - 1);
         src = p + 2 * ((long)(2 * q + k0) + (long)row * ld);
       } else {
-        const int row = min(r0 + 2 * lane, nrows - 2);
+        const int row = min(r0 + 2 * lane, (nrows - 1) & ~1);
         src = p + 2 * ((long)row + (long)(k0 + inst) * ld);
       }
       __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
@@ -1191,7 +1232,8 @@ __device__ __forceinline__ void cpipe_tile(const GemmParams<float>& prm, int blo
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int wm = wave & 1, wn = wave >> 1;
   const int li = lane & 15, lg = lane >> 4;
-  const int nkt = K / 8;
+  const bool ragged = K % 8 != 0 || (!A_KC && M % 2 != 0) || (!B_KC && N % 2 != 0);
+  const int nkt = ring_steps(K, 8, ragged);
 
   flt4 cre[4][4], cim[4][4];
 #pragma unroll
@@ -1215,6 +1257,32 @@ __device__ __forceinline__ void cpipe_tile(const GemmParams<float>& prm, int blo
 #pragma unroll
     for (int j = 0; j < 4; ++j) f.b[j] = CdldsOperand<B_KC>::frag(st + TILE, lg, wn * 64 + j * 16 + li);
   };
+  if (ragged) {
+    // one A fragment and one B fragment at a time: beside 128 accumulators a whole set would spill
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      v4f a = last_frag<A_KC, 2, 2, v4f>(prm.a, prm.lda, m0 + wm * 64 + i * 16 + li, M, nkt * 8 + 2 * lg, K);
+      if (A_CONJ) {
+        a[1] = -a[1];
+        a[3] = -a[3];
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        v4f b = last_frag<B_KC, 2, 2, v4f>(prm.b, prm.ldb, n0 + wn * 64 + j * 16 + li, N, nkt * 8 + 2 * lg, K);
+        if (B_CONJ) {
+          b[1] = -b[1];
+          b[3] = -b[3];
+        }
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          cre[i][j] = mfma(b[2 * t], a[2 * t], cre[i][j]);
+          cre[i][j] = mfma(b[2 * t + 1], -a[2 * t + 1], cre[i][j]);
+          cim[i][j] = mfma(b[2 * t + 1], a[2 * t], cim[i][j]);
+          cim[i][j] = mfma(b[2 * t], a[2 * t + 1], cim[i][j]);
+        }
+      }
+    }
+  }
   if constexpr (!B_KC) {
     // A row-contiguous B: two fragment sets of A but one of B, each B fragment read for stage kt+1
     // into its registers as soon as the 32 MFMAs of stage kt that use it are issued (two full sets
@@ -1480,7 +1548,8 @@ struct BigOperand {
   long kstride;  // elements per step of k: 1 (k-contiguous) or ld (row-contiguous)
   // k-contiguous: instruction i fills rows 16i..16i+15 (64 bytes each, slots XOR-permuted as in
   // DldsOperand); row-contiguous: instruction i fills the 128 rows (i % P) * 128.. at k = i / P,
-  // P = ROWS / 128, 2 rows per lane (needs an even row count).
+  // P = ROWS / 128, 2 rows per lane (of an odd row count the last lane's second row is the next
+  // column's first, or padding: see ring_steps).
   __device__ __forceinline__ BigOperand(const double* p, long ld, int r0, int nrows, int wave, int lane) {
     kstride = KC ? 1 : ld;
 #pragma unroll
@@ -1494,7 +1563,7 @@ struct BigOperand {
       } else {
         constexpr int P = ROWS / 128;
         const int kk = inst / P, part = inst % P;
-        base[t] = p + min(r0 + part * 128 + 2 * lane, nrows - 2) + (long)kk * ld;
+        base[t] = p + min(r0 + part * 128 + 2 * lane, (nrows - 1) & ~1) + (long)kk * ld;
         dst[t] = kk * ROWS + part * 128;
       }
     }
@@ -1520,8 +1589,7 @@ struct BigOperand {
   static constexpr int READS = KC ? 1 : 2;  // LDS read instructions per fragment
 };
 
-// One 128 x BN C tile at (m0, n0); K a multiple of 8 (the launcher hands a remainder to
-// gemm_real_kernel).
+// One 128 x BN C tile at (m0, n0), any m, n, k >= 1.
 template <bool A_KC, bool B_KC, int BN>
 __device__ __forceinline__ void dbig_tile_at(const GemmParams<double>& prm, int m0, int n0) {
   constexpr int BM = 128, S = 3, A_ST = BM * 8, STAGE = (BM + BN) * 8;
@@ -1538,7 +1606,8 @@ __device__ __forceinline__ void dbig_tile_at(const GemmParams<double>& prm, int 
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int wm = wave & 1, wn = wave >> 1;
   const int li = lane & 15, lg = lane >> 4;
-  const int nkt = K / 8;
+  const bool ragged = K % 8 != 0 || (!A_KC && M % 2 != 0) || (!B_KC && N % 2 != 0);
+  const int nkt = ring_steps(K, 8, ragged);
   const OA opa(prm.a, prm.lda, m0, M, wave, lane);
   const OB opb(prm.b, prm.ldb, n0, N, wave, lane);
   auto issue = [&](int kt, int so) {
@@ -1566,6 +1635,21 @@ __device__ __forceinline__ void dbig_tile_at(const GemmParams<double>& prm, int 
 #pragma unroll
     for (int j = 0; j < TJ; ++j) acc[i][j] = dbl4{0, 0, 0, 0};
 
+  if (ragged) {
+    Frags f;
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+      f.a[i] = last_frag<A_KC, 2, 1, v2d>(prm.a, prm.lda, m0 + wm * 64 + i * 16 + li, M, nkt * 8 + 2 * lg, K);
+#pragma unroll
+    for (int j = 0; j < TJ; ++j)
+      f.b[j] = last_frag<B_KC, 2, 1, v2d>(prm.b, prm.ldb, n0 + wn * (BN / 2) + j * 16 + li, N, nkt * 8 + 2 * lg, K);
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int i = 0; i < TI; ++i)
+#pragma unroll
+        for (int j = 0; j < TJ; ++j) acc[i][j] = mfma(f.b[j][h], f.a[i][h], acc[i][j]);
+  }
   if (nkt > 0) {
     // stages 0, 1, 2 in flight (clamped), stage 0 read into F0
 #pragma unroll
@@ -1922,7 +2006,8 @@ __device__ __forceinline__ void zpipe_tile(const GemmParams<double>& prm, int bl
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int wm = wave & 1, wn = wave >> 1;
   const int li = lane & 15, lg = lane >> 4;
-  const int nkt = K / 8;
+  const bool ragged = K % 8 != 0;
+  const int nkt = ring_steps(K, 8, ragged);
 
   dbl4 cre[2][2], cim[2][2];
 #pragma unroll
@@ -1949,6 +2034,31 @@ __device__ __forceinline__ void zpipe_tile(const GemmParams<double>& prm, int bl
       for (int j = 0; j < 2; ++j) f.b[kk][j] = ZdldsOperand<B_KC>::elem(st + TILE, wn * 32 + j * 16 + li, 4 * kk + lg);
     }
   };
+  if (ragged) {
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      v2d a[2], b[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        a[i] = last_frag<A_KC, 1, 2, v2d>(prm.a, prm.lda, m0 + wm * 32 + i * 16 + li, M, nkt * 8 + 4 * kk + lg, K);
+        if (A_CONJ) a[i][1] = -a[i][1];
+      }
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        b[j] = last_frag<B_KC, 1, 2, v2d>(prm.b, prm.ldb, n0 + wn * 32 + j * 16 + li, N, nkt * 8 + 4 * kk + lg, K);
+        if (B_CONJ) b[j][1] = -b[j][1];
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          cre[i][j] = mfma(b[j][0], a[i][0], cre[i][j]);
+          cre[i][j] = mfma(b[j][1], -a[i][1], cre[i][j]);
+          cim[i][j] = mfma(b[j][1], a[i][0], cim[i][j]);
+          cim[i][j] = mfma(b[j][0], a[i][1], cim[i][j]);
+        }
+    }
+  }
   if (nkt > 0) {
 #pragma unroll
     for (int s = 0; s < S; ++s) issue(min(s, nkt - 1), s * STAGE);
@@ -2156,10 +2266,13 @@ int dgemm_kind(long largest, bool big_ok, long tiles128, long tiles256) {
   return kDgemmRing3;
 }
 
+int dgemm_kind(const GemmParams<double>& p) {
+  return dgemm_kind((long)p.m * p.n, p.m > 128 && p.n > 128, dgemm_tiles(p.m, p.n, 128), dgemm_tiles(p.m, p.n, 256));
+}
+
 template <bool AKC, bool BKC>
 void launch_dlds(const GemmParams<double>& p, hipStream_t s) {
-  const int kind = dgemm_kind((long)p.m * p.n, p.m > 128 && p.n > 128, dgemm_tiles(p.m, p.n, 128),
-                              dgemm_tiles(p.m, p.n, 256));
+  const int kind = dgemm_kind(p);
   if (kind == kDgemmBig) {
     hipLaunchKernelGGL((gemm_d_big_kernel<AKC, BKC>), dim3(dgemm_tiles(p.m, p.n, 256)), dim3(256), 0, s, p);
     return;
@@ -2174,15 +2287,17 @@ void launch_dlds(const GemmParams<double>& p, hipStream_t s) {
   hipLaunchKernelGGL((gemm_d_dlds_kernel<AKC, BKC, 3, 3>), dim3(nbm * nbn), dim3(256), 0, s, p);
 }
 
-// FP64 through the direct-LDS kernel for the largest multiple of 8 in K; a remainder of K goes to
-// gemm_real_kernel, accumulating (beta only on the first part).
+// FP64 through the direct-LDS kernels. The pipelined ones take any m, n and k; the three-per-CU one
+// the largest multiple of 8 in K, a remainder going to gemm_real_kernel, accumulating (beta only on
+// the first part).
 hipError_t launch_gemm_d_direct(const GemmParams<double>& p, hipStream_t s) {
   const bool akc = is_kc_a(p.opa), bkc = is_kc_b(p.opb);
-  const int k8 = p.k / 8 * 8;
-  // a row-contiguous operand with an odd row count would need a 2-row chunk that straddles the
-  // last row: such shapes keep the register-staged kernel
+  const bool pipe = p.k > 0 && dgemm_kind(p) != kDgemmRing3;
+  const int k8 = pipe ? p.k : p.k / 8 * 8;
+  // for the three-per-CU kernel a row-contiguous operand with an odd row count would need a 2-row
+  // chunk that straddles the last row: such shapes keep the register-staged kernel
   const bool pairs_ok = (akc || p.m % 2 == 0) && (bkc || p.n % 2 == 0);
-  if (k8 == 0 || p.m < 2 || p.n < 2 || !pairs_ok) return launch_real<double>(p, s);
+  if (!pipe && (k8 == 0 || p.m < 2 || p.n < 2 || !pairs_ok)) return launch_real<double>(p, s);
   GemmParams<double> q = p;
   q.k = k8;
   if (akc && bkc) launch_dlds<true, true>(q, s);
@@ -2416,14 +2531,18 @@ hipError_t launch_gemm_d(const GemmParams<double>& p, hipStream_t s) {
   if (p.variant == 1) return launch_gemm_d_direct(p, s);
   return launch_real<double>(p, s);
 }
-// FP32 through the direct-LDS kernel for the largest multiple of 16 in K; a remainder of K goes to
-// gemm_real_kernel, accumulating (beta only on the first part).
+// FP32 through the direct-LDS kernels. The pipelined one takes any k and any row count (but not a
+// row-contiguous operand whose 4-row chunks could reach over more than one column end); the others
+// the largest multiple of 16 in K, a remainder going to gemm_real_kernel, accumulating (beta only
+// on the first part).
 hipError_t launch_gemm_s_direct(const GemmParams<float>& p, hipStream_t s) {
   const bool akc = is_kc_a(p.opa), bkc = is_kc_b(p.opb);
-  const int k16 = p.k / 16 * 16;
-  // a row-contiguous operand needs whole 4-row chunks
+  const bool chunks_ok = (akc || p.m % 4 == 0 || p.lda >= 3) && (bkc || p.n % 4 == 0 || p.ldb >= 3);
+  const bool pipe = p.k > 0 && sgemm_pipe(p.m, p.n) && chunks_ok;
+  const int k16 = pipe ? p.k : p.k / 16 * 16;
+  // the other kernels need whole 4-row chunks of a row-contiguous operand
   const bool rows_ok = (akc || p.m % 4 == 0) && (bkc || p.n % 4 == 0);
-  if (k16 == 0 || !rows_ok) return launch_real<float>(p, s);
+  if (!pipe && (k16 == 0 || !rows_ok)) return launch_real<float>(p, s);
   GemmParams<float> q = p;
   q.k = k16;
   // 256 x 256 workgroup tiles (8 waves of 64 x 128, one workgroup per CU) once m and n allow:
@@ -2431,7 +2550,7 @@ hipError_t launch_gemm_s_direct(const GemmParams<float>& p, hipStream_t s) {
   // for 256 x 128 tiles (8 waves of 64 x 64, two per CU; 32 against 48 bytes of LDS writes per
   // MFMA); 256 x 128 in turn ran NN 138.2 and TN 135.1 against 134.8 and 134.3 for 128 x 128 tiles
   // at three per CU
-  if (sgemm_pipe(p.m, p.n)) {
+  if (pipe) {
     const dim3 grid(dgemm_tiles(p.m, p.n, 128)), block(256);
     if (akc && bkc) hipLaunchKernelGGL((gemm_s_pipe_kernel<true, true>), grid, block, 0, s, q);
     else if (akc) hipLaunchKernelGGL((gemm_s_pipe_kernel<true, false>), grid, block, 0, s, q);
@@ -2475,17 +2594,17 @@ hipError_t launch_gemm_s(const GemmParams<float>& p, hipStream_t s) {
 hipError_t launch_gemm_z(const GemmParams<double>& p, hipStream_t s) {
   if (p.m <= 0 || p.n <= 0) return hipSuccess;
   if (p.variant == 0) return launch_cplx<double>(p, s);
-  // direct-LDS kernel on the largest multiple of 8 in K, the remainder through gemm_cplx_kernel
-  // accumulating (beta only on the first part)
-  const int k8 = p.k / 8 * 8;
+  const dim3 grid(((p.m + 63) / 64) * ((p.n + 63) / 64)), block(256);
+  const bool pipe = p.k > 0 && (long)grid.x >= 2L * device_cus();  // as for the groups
+  // the pipelined kernel takes any k; the other one the largest multiple of 8 in K, the remainder
+  // going through gemm_cplx_kernel, accumulating (beta only on the first part)
+  const int k8 = pipe ? p.k : p.k / 8 * 8;
   if (k8 == 0) return launch_cplx<double>(p, s);
   const bool akc = is_kc_a(p.opa), bkc = is_kc_b(p.opb);
   GemmParams<double> q = p;
   q.k = k8;
-  const dim3 grid(((p.m + 63) / 64) * ((p.n + 63) / 64)), block(256);
   const bool ca = p.opa == 'C', cb = p.opb == 'C';
   // 3-stage ring, 3 workgroups per CU: 69.7 TFLOP/s on CN 8192^3 against 67.9 for 4 stages at 2
-  const bool pipe = (long)grid.x >= 2L * device_cus();  // as for the groups
 #define TMM_ZDLDS(AK, BK, CA, CB)                                                              \
   do {                                                                                         \
     if (pipe) hipLaunchKernelGGL((gemm_z_pipe_kernel<AK, BK, CA, CB>), grid, block, 0, s, q);  \
@@ -2520,17 +2639,17 @@ hipError_t launch_gemm_z(const GemmParams<double>& p, hipStream_t s) {
 hipError_t launch_gemm_c(const GemmParams<float>& p, hipStream_t s) {
   if (p.m <= 0 || p.n <= 0) return hipSuccess;
   const bool akc = is_kc_a(p.opa), bkc = is_kc_b(p.opb);
-  const int k8 = p.k / 8 * 8;
-  // a row-contiguous operand needs whole 2-row chunks
-  const bool rows_ok = (akc || p.m % 2 == 0) && (bkc || p.n % 2 == 0);
+  const dim3 grid(((p.m + 127) / 128) * ((p.n + 127) / 128));
+  const bool pipe = p.k > 0 && sgemm_pipe((long)grid.x);  // as for the groups
+  // the pipelined kernel takes any k and any row count; the other one the largest multiple of 8 in
+  // K, the remainder going through gemm_cplx_kernel, accumulating (beta only on the first part),
+  // and whole 2-row chunks of a row-contiguous operand
+  const int k8 = pipe ? p.k : p.k / 8 * 8;
+  const bool rows_ok = pipe || ((akc || p.m % 2 == 0) && (bkc || p.n % 2 == 0));
   if (p.variant != 1 || k8 == 0 || !rows_ok) return launch_cplx<float>(p, s);
-  // direct-LDS kernel on the largest multiple of 8 in K, the remainder through gemm_cplx_kernel
-  // accumulating (beta only on the first part)
   GemmParams<float> q = p;
   q.k = k8;
-  const dim3 grid(((p.m + 127) / 128) * ((p.n + 127) / 128));
   const bool ca = p.opa == 'C', cb = p.opb == 'C';
-  const bool pipe = sgemm_pipe((long)grid.x);  // as for the groups
 #define TMM_CDLDS(AK, BK, CA, CB) launch_c1<AK, BK, CA, CB>(pipe, grid, s, q)
   if (akc && bkc) {
     if (ca) TMM_CDLDS(true, true, true, false);
