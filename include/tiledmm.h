@@ -196,13 +196,12 @@ int tmm_synchronize(tmm_handle* h);
  *                        and the tile's products start before it arrives; 0: before the tile's
  *                        own products, as for native calls. Same results.
  *   TMM_OPT_DGEMM_KERNEL tile kernels of every element type: 1 (default) = direct global->LDS
- *                        loads into a 3-stage ring (with at least two workgroup tiles per CU
- *                        software-pipelined; FP64 on 128 x 128 tiles, or 128 x 256 from 2^27
- *                        elements of C on); 0 = LDS double buffer filled through registers
- *                        (the kernel that variant 1 also uses for shapes it does not
- *                        take: K % 8 remainders (FP32: K % 16); an odd row count of a
- *                        row-contiguous operand (FP32: not a multiple of 4); for FP64 also m or
- *                        n < 2). */
+ *                        loads: small tiles that split the inner dimension over a workgroup's
+ *                        waves, or, with at least two workgroup tiles per CU and where they are
+ *                        estimated to be faster, software-pipelined 128 x 128 tiles (complex
+ *                        double 64 x 64; FP64 128 x 256 from 2^27 elements of C on); 0 = LDS
+ *                        double buffer filled through registers (the kernel that variant 1 also
+ *                        uses for k = 0 and for leading dimensions beyond 256 MB). */
 enum {
   TMM_OPT_COARSEN = 1,
   TMM_OPT_FIRST_CHUNK = 2,

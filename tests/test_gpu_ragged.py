@@ -46,3 +46,23 @@ def _ops(dtype):
 def test_pipelined_kernels_ragged(torch_gpu, dtype, m, n, k):
     """At least two workgroup tiles per CU: the software-pipelined kernels."""
     _exact(torch_gpu, dtype, m, n, k, _ops(dtype), 1)
+
+
+# each of the tile shapes (16 to 64 rows and columns) is the estimated fastest at one of these sizes
+KS_SIZES = [(1, 1, 1), (16, 16, 1), (17, 33, 5), (457, 1266, 6), (298, 397, 430), (1219, 204, 556), (1213, 416, 178),
+            (645, 1123, 536), (1186, 631, 381), (476, 1159, 214), (1316, 722, 450), (704, 710, 694), (1059, 1220, 683),
+            (1261, 1169, 697), (1302, 1305, 686), (200, 301, 5003)]
+
+
+@pytest.mark.parametrize("m,n,k", KS_SIZES)
+@pytest.mark.parametrize("dtype", [np.float64, np.float32, np.complex64, np.complex128], ids=["d", "s", "c", "z"])
+def test_split_inner_dimension_ragged(torch_gpu, dtype, m, n, k):
+    """Fewer tiles: the kernels that split the inner dimension over a workgroup's waves."""
+    _exact(torch_gpu, dtype, m, n, k, _ops(dtype), 3 if m > 16 else 2)
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32, np.complex64, np.complex128], ids=["d", "s", "c", "z"])
+def test_leading_dimension_of_one(torch_gpu, dtype):
+    """Row vectors without padding: consecutive columns lie one element apart."""
+    _exact(torch_gpu, dtype, 1, 1, 100, [("N", "T")], 0)
+    _exact(torch_gpu, dtype, 1, 70, 33, [("N", "T"), ("N", "N")], 0)

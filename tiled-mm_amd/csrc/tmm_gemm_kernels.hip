@@ -24,7 +24,9 @@
 #include <stdint.h>
 
 #include <algorithm>
+#include "tmm_group.h"
 #include "tmm_kernels.h"
+#include "tmm_ksplit.h"
 
 namespace tmm {
 namespace {
@@ -567,9 +569,9 @@ __device__ __forceinline__ V last_frag(const R* __restrict__ p, long ld, int row
 }
 
 // ---------------------------------------------------------------------------------------------
-// FP64 GEMM with direct global->LDS loads (global_load_lds_dwordx4) into an S-stage LDS ring.
-// WG tile 128x128, 2x2 waves of 64x64, k-step 8 per stage, S stages of 16 KB (S = 3, three
-// workgroups per CU).
+// FP64 tile with direct global->LDS loads (global_load_lds_dwordx4) into an S-stage LDS ring, the
+// body of the batched path. WG tile 128x128, 2x2 waves of 64x64, k-step 8 per stage, S stages of
+// 16 KB (S = 3, three workgroups per CU).
 // The loads of stage kt+S-1 are issued right after the barrier of stage kt, so S-1 stages are in
 // flight while the MFMAs run; no registers or ds_write instructions carry the operands.
 //   k-contiguous operand (A for 'T', B for 'N'): LDS [row][slot][2], a 16-byte chunk = 2
@@ -577,8 +579,7 @@ __device__ __forceinline__ V last_frag(const R* __restrict__ p, long ld, int row
 //     instruction fills 16 consecutive rows, reading 64 contiguous bytes of each.
 //   row-contiguous operand (A for 'N', B for 'T'): LDS [k][row], a 16-byte chunk = 2 consecutive
 //     rows at one k; a wave instruction fills all 128 rows of one k (coalesced in global memory).
-// Rows beyond the matrix load a clamped in-bounds row: they only feed outputs that are not
-// stored. K must be a multiple of 8 (the launcher hands a remainder to gemm_real_kernel).
+// Rows beyond the matrix load a clamped row: they only feed outputs that are not stored.
 // ---------------------------------------------------------------------------------------------
 template <bool KC>
 struct DldsOperand {
@@ -587,11 +588,10 @@ struct DldsOperand {
   // then touches 8 distinct 16-byte bank groups per 8 lanes (rows r, r+1 share a swizzle and sit
   // 64 bytes apart), i.e. it is free of bank conflicts.
   __device__ __forceinline__ static int kc_swz(int r) { return (r >> 1) & 3; }
-  // issue this wave's 2 loads of one stage (8 instructions per workgroup). ARENA: the operand lies
-  // in a device arena with at least 16 more bytes after its last column (the batched path), so a
-  // row-contiguous operand of odd row count may read its last 2-row chunk one row past the end
-  // (that row only feeds unstored outputs) instead of needing an even row count.
-  template <bool ARENA = false>
+  // issue this wave's 2 loads of one stage (8 instructions per workgroup). The operand lies in a
+  // device arena with at least 16 more bytes after its last column, so a row-contiguous operand of
+  // odd row count may read its last 2-row chunk one row past the end (that row only feeds unstored
+  // outputs).
   __device__ __forceinline__ static void issue(const double* __restrict__ p, long ld, int r0, int nrows, int k0,
                                                double* stage, int wave, int lane) {
 #pragma unroll
@@ -610,7 +610,7 @@ struct DldsOperand {
         dst = stage + inst * 128;
       } else {
         const int kk = inst;
-        const int row = min(r0 + 2 * lane, ARENA ? ((nrows + 1) & ~1) - 2 : nrows - 2);
+        const int row = min(r0 + 2 * lane, (nrows - 1) & ~1);
         src = p + (long)row + (long)(k0 + kk) * ld;
         dst = stage + kk * 128;
       }
@@ -631,10 +631,10 @@ struct DldsOperand {
   }
 };
 
-// One 128x128 C tile at (m0, n0). ARENA (the batched path): operands in the batch's device arena
-// (see DldsOperand::issue), any m, n >= 1, and K need not be a multiple of 8: the last K % 8
-// values are added in the epilogue from global memory.
-template <bool A_KC, bool B_KC, int S, bool ARENA>
+// One 128x128 C tile at (m0, n0) of a problem in the batch's device arena (see
+// DldsOperand::issue): any m, n >= 1, any K (the last K % 8 values are added in the epilogue from
+// global memory).
+template <bool A_KC, bool B_KC, int S>
 __device__ __forceinline__ void dlds_tile_at(const GemmParams<double>& prm, int m0, int n0) {
   constexpr int STAGE = 2 * 1024;  // A and B, 1024 doubles each
   __shared__ __attribute__((aligned(16))) double lds[S * STAGE];
@@ -652,8 +652,8 @@ __device__ __forceinline__ void dlds_tile_at(const GemmParams<double>& prm, int 
 
   auto issue = [&](int kt) {
     double* st = lds + (kt % S) * STAGE;
-    DldsOperand<A_KC>::template issue<ARENA>(prm.a, prm.lda, m0, M, kt * 8, st, wave, lane);
-    DldsOperand<B_KC>::template issue<ARENA>(prm.b, prm.ldb, n0, N, kt * 8, st + 1024, wave, lane);
+    DldsOperand<A_KC>::issue(prm.a, prm.lda, m0, M, kt * 8, st, wave, lane);
+    DldsOperand<B_KC>::issue(prm.b, prm.ldb, n0, N, kt * 8, st + 1024, wave, lane);
   };
 #pragma unroll
   for (int s = 0; s < S - 1; ++s)
@@ -697,12 +697,10 @@ __device__ __forceinline__ void dlds_tile_at(const GemmParams<double>& prm, int 
         const int gj = n0 + wn * 64 + j * 16 + out_col<double>(lane, r);
         if (gj >= N) continue;
         double sum = acc[i][j][r];
-        if constexpr (ARENA) {
-          for (int kk = nkt * 8; kk < K; ++kk) {
-            const double av = A_KC ? prm.a[(long)kk + (long)gi * prm.lda] : prm.a[(long)gi + (long)kk * prm.lda];
-            const double bv = B_KC ? prm.b[(long)kk + (long)gj * prm.ldb] : prm.b[(long)gj + (long)kk * prm.ldb];
-            sum = fma(av, bv, sum);
-          }
+        for (int kk = nkt * 8; kk < K; ++kk) {
+          const double av = A_KC ? prm.a[(long)kk + (long)gi * prm.lda] : prm.a[(long)gi + (long)kk * prm.lda];
+          const double bv = B_KC ? prm.b[(long)kk + (long)gj * prm.ldb] : prm.b[(long)gj + (long)kk * prm.ldb];
+          sum = fma(av, bv, sum);
         }
         double v = alpha * sum;
         double* dst = prm.c + (long)gi + (long)gj * prm.ldc;
@@ -714,35 +712,17 @@ __device__ __forceinline__ void dlds_tile_at(const GemmParams<double>& prm, int 
   }
 }
 
-template <bool A_KC, bool B_KC, int S>
-__device__ __forceinline__ void dlds_tile(const GemmParams<double>& prm, int block) {
-  const int nbm = (prm.m + 127) / 128, nbn = (prm.n + 127) / 128;
-  int bm, bn;
-  tile_coords(block, nbm, nbn, bm, bn);
-  dlds_tile_at<A_KC, B_KC, S, false>(prm, bm * 128, bn * 128);
-}
-
-template <bool A_KC, bool B_KC, int S, int OCC = 2>
-__global__ __launch_bounds__(256, OCC) void gemm_d_dlds_kernel(GemmParams<double> prm) {
-  if (prm.gate_a && (*prm.gate_a | *prm.gate_b) == 0) return;  // uniform: before any barrier
-  dlds_tile<A_KC, B_KC, S>(prm, blockIdx.x);
-}
-
 // ---------------------------------------------------------------------------------------------
 // FP32 GEMM with direct global->LDS loads: the FP64 kernel's ring with 16-byte chunks of 4 floats,
-// so a stage holds k-step 16 (64 bytes per operand row), 3 stages; workgroup tiles of 256 x 256
-// (8 waves of 64 x 128, 32 KB per stage, one workgroup per CU), 256 x 128 (8 waves of 64 x 64, 24
-// KB per stage, two per CU) or 128 x 128 (4 waves, 16 KB per stage, three per CU). A lane's
-// 16-byte fragment holds k = 4g..4g+3 of its row (g = lane / 16) and
-// feeds four v_mfma_f32_16x16x4f32, the same k permutation for A and B.
+// so a stage holds k-step 16 (64 bytes per operand row), 3 stages; workgroup tiles of 128 x 128 (4
+// waves, 16 KB per stage, two or three per CU). A lane's 16-byte fragment holds k = 4g..4g+3 of its
+// row (g = lane / 16) and feeds four v_mfma_f32_16x16x4f32, the same k permutation for A and B.
 //   k-contiguous operand: LDS [row][slot][4], chunk q (k = 4q..4q+3) of row r in slot q ^ swz(r),
 //     a wave instruction fills 16 rows, 64 contiguous bytes of each (as in the FP64 kernel).
 //   row-contiguous operand: LDS [k][row], a 16-byte chunk = 4 consecutive rows at one k; a wave
-//     instruction fills 256 rows at one k, or 128 rows at two k (lanes 0-31 the first, 32-63 the
-//     second). Needs a row count that is a multiple of 4 (the launcher sends other shapes to
-//     gemm_real_kernel).
-// Rows beyond the matrix read a clamped in-bounds row (they feed only unstored outputs). K must be
-// a multiple of 16 (the launcher hands a remainder to gemm_real_kernel).
+//     instruction fills 128 rows at two k (lanes 0-31 the first, 32-63 the second).
+// Rows beyond the matrix read a clamped in-bounds row (they feed only unstored outputs); a ragged
+// last k-step is read separately (ring_steps).
 // ---------------------------------------------------------------------------------------------
 template <bool KC, int ROWS, int NW>
 struct SdldsOperand {
@@ -784,85 +764,10 @@ struct SdldsOperand {
   }
 };
 
-// One BM x BN C tile at (m0, n0): WM x 2 waves of 64 x (BN / 2).
-template <bool A_KC, bool B_KC, int S, int BM, int BN = 128>
-__device__ __forceinline__ void sdlds_tile_at(const GemmParams<float>& prm, int m0, int n0) {
-  constexpr int WM = BM / 64, NW = 2 * WM, TN = BN / 2, TJ = TN / 16;
-  constexpr int A_ELEMS = BM * 16, STAGE = A_ELEMS + BN * 16;
-  constexpr int PER = (BM / 16 + BN / 16) / NW;  // load instructions per wave and stage
-  using OpA = SdldsOperand<A_KC, BM, NW>;
-  using OpB = SdldsOperand<B_KC, BN, NW>;
-  __shared__ __attribute__((aligned(16))) float lds[S * STAGE];
-  const int M = prm.m, N = prm.n, K = prm.k;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wm = wave % WM, wn = wave / WM;
-  const int li = lane & 15, lg = lane >> 4;
-  const int nkt = K / 16;
-
-  flt4 acc[4][TJ];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < TJ; ++j) acc[i][j] = flt4{0, 0, 0, 0};
-
-  auto issue = [&](int kt) {
-    float* st = lds + (kt % S) * STAGE;
-    OpA::issue(prm.a, prm.lda, m0, M, kt * 16, st, wave, lane);
-    OpB::issue(prm.b, prm.ldb, n0, N, kt * 16, st + A_ELEMS, wave, lane);
-  };
-#pragma unroll
-  for (int s = 0; s < S - 1; ++s)
-    if (s < nkt) issue(s);
-  for (int kt = 0; kt < nkt; ++kt) {
-    // this wave's loads of stage kt have landed once at most PER per later stage are pending; its
-    // LDS reads of stage kt-1 are done (lgkmcnt 0); the barrier extends both to the workgroup
-    const int later = min(S - 2, nkt - 1 - kt);
-    if (later >= 2) __builtin_amdgcn_s_waitcnt(0x070 | (2 * PER));
-    else if (later == 1) __builtin_amdgcn_s_waitcnt(0x070 | PER);
-    else __builtin_amdgcn_s_waitcnt(0x070);
-    __builtin_amdgcn_s_barrier();
-    if (kt + S - 1 < nkt) issue(kt + S - 1);  // into the slot of stage kt-1, free after the barrier
-    const float* st = lds + (kt % S) * STAGE;
-    v4f a[4], b[TJ];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) a[i] = OpA::frag(st, lg, wm * 64 + i * 16 + li);
-#pragma unroll
-    for (int j = 0; j < TJ; ++j) b[j] = OpB::frag(st + A_ELEMS, lg, wn * TN + j * 16 + li);
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < TJ; ++j) acc[i][j] = mfma(b[j][t], a[i][t], acc[i][j]);
-  }
-
-  const float alpha = prm.alpha, beta = prm.beta;
-  const bool acc_prev = prm.accumulate != 0, use_cin = beta != 0.0f;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int gi = m0 + wm * 64 + i * 16 + li;
-    if (gi >= M) continue;
-#pragma unroll
-    for (int j = 0; j < TJ; ++j) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int gj = n0 + wn * TN + j * 16 + out_col<float>(lane, r);
-        if (gj >= N) continue;
-        float v = alpha * acc[i][j][r];
-        float* dst = prm.c + (long)gi + (long)gj * prm.ldc;
-        if (acc_prev) v += *dst;
-        if (use_cin) v += beta * prm.cin[(long)gi + (long)gj * prm.ldcin];
-        *dst = v;
-      }
-    }
-  }
-}
-
 // The FP32 tile software-pipelined as dbig_tile_at (FP64): the fragments of stage kt+1 are read
 // into a second register set while the 16 x TJ MFMAs of stage kt run, the loads of stage kt+3 go
 // between its first MFMAs, scheduling-group barriers pin that order, and the loads always run
-// (clamped to the last stage) so that every wait count is a constant. Per output block the MFMA
-// sequence is sdlds_tile_at's: the results are the same bits.
+// (clamped to the last stage) so that every wait count is a constant.
 template <bool A_KC, bool B_KC, int BM, int BN>
 __device__ __forceinline__ void spipe_tile_at(const GemmParams<float>& prm, int m0, int n0) {
   constexpr int S = 3;
@@ -994,17 +899,9 @@ __global__ __launch_bounds__(256, 2) void gemm_s_pipe_kernel(GemmParams<float> p
   spipe_tile_at<A_KC, B_KC, 128, 128>(prm, bm * 128, bn * 128);
 }
 
-template <bool A_KC, bool B_KC, int S, int OCC, int BM, int BN = 128>
-__global__ __launch_bounds__(BM * 2, OCC) void gemm_s_dlds_kernel(GemmParams<float> prm) {
-  const int nbm = (prm.m + BM - 1) / BM, nbn = (prm.n + BN - 1) / BN;
-  int bm, bn;
-  tile_coords(blockIdx.x, nbm, nbn, bm, bn);
-  sdlds_tile_at<A_KC, B_KC, S, BM, BN>(prm, bm * BM, bn * BN);
-}
-
 // Persistent batched FP64 GEMM on the direct-to-LDS tile body: the same item protocol as
-// gemm_real_batched_kernel, operands in the batch's device arena (dlds_tile_at with ARENA: any
-// m, n >= 1 and any k), three workgroups per CU like gemm_d_dlds_kernel.
+// gemm_real_batched_kernel, operands in the batch's device arena (any m, n >= 1 and any k),
+// three workgroups per CU.
 template <bool A_KC, bool B_KC, int S>
 __global__ __launch_bounds__(256, 3) void gemm_d_dlds_batched_kernel(const GemmParams<double>* __restrict__ probs,
                                                                     const int* __restrict__ items, int n_items,
@@ -1017,36 +914,9 @@ __global__ __launch_bounds__(256, 3) void gemm_d_dlds_batched_kernel(const GemmP
     __syncthreads();  // everyone has read `next` before thread 0 overwrites it
     if (it >= n_items) break;
     const GemmParams<double> prm = probs[items[3 * it]];
-    dlds_tile_at<A_KC, B_KC, S, true>(prm, items[3 * it + 1] * 128, items[3 * it + 2] * 128);
+    dlds_tile_at<A_KC, B_KC, S>(prm, items[3 * it + 1] * 128, items[3 * it + 2] * 128);
     __syncthreads();  // every wave is done with the LDS ring before the next item refills it
   }
-}
-
-// Several independent FP64 products of one shape class (same ops, alpha, k) in one launch: the
-// grid is the concatenation of the products' workgroup ranges, each padded to a multiple of 8 so
-// that a workgroup's XCD (blockIdx.x % 8) is the one tile_coords assumes. Padding workgroups exit
-// before any barrier.
-template <bool A_KC, bool B_KC, int S, int OCC = 2>
-__global__ __launch_bounds__(256, OCC) void gemm_d_dlds_group_kernel(DgemmGroup g) {
-  const int w = blockIdx.x;
-  int t = 0;
-  while (t + 1 < g.count && w >= g.wg_start[t + 1]) ++t;
-  GemmParams<double> prm = g.base;
-  prm.m = g.m[t];
-  prm.n = g.n[t];
-  prm.a = g.a[t];
-  prm.lda = g.lda[t];
-  prm.b = g.b[t];
-  prm.ldb = g.ldb[t];
-  prm.c = g.c[t];
-  prm.ldc = g.ldc[t];
-  prm.cin = g.cin[t];
-  prm.ldcin = g.ldcin[t];
-  prm.beta = g.beta[t];
-  prm.accumulate = g.accumulate[t];
-  const int local = w - g.wg_start[t];
-  if (local >= ((prm.m + 127) / 128) * ((prm.n + 127) / 128)) return;
-  dlds_tile<A_KC, B_KC, S>(prm, local);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1058,11 +928,9 @@ __global__ __launch_bounds__(256, OCC) void gemm_d_dlds_group_kernel(DgemmGroup 
 //   k-contiguous operand (A for 'T'/'C', B for 'N'): LDS [row][slot], chunk q (k = 2q, 2q+1) of
 //     row r in slot q ^ swz(r); a wave instruction fills 16 rows, 64 contiguous bytes of each.
 //   row-contiguous operand (A for 'N', B for 'T'/'C'): LDS [k][row], a 16-byte chunk = 2
-//     consecutive rows at one k; a wave instruction fills the 128 rows of one k. Needs an even row
-//     count (the launcher sends other shapes to gemm_cplx_kernel).
+//     consecutive rows at one k; a wave instruction fills the 128 rows of one k.
 // Conjugation ('C') negates the imaginary fragment in registers. Rows beyond the matrix read a
-// clamped in-bounds row. K must be a multiple of 8 (the launcher hands a remainder to
-// gemm_cplx_kernel).
+// clamped in-bounds row; a ragged last k-step is read separately (ring_steps).
 // ---------------------------------------------------------------------------------------------
 template <bool KC>
 struct CdldsOperand {
@@ -1101,122 +969,11 @@ struct CdldsOperand {
   }
 };
 
-template <bool A_KC, bool B_KC, bool A_CONJ, bool B_CONJ, int S>
-__device__ __forceinline__ void cdlds_tile(const GemmParams<float>& prm, int block) {
-  constexpr int TILE = 128 * 16;  // floats per operand and stage (8 KB)
-  constexpr int STAGE = 2 * TILE;
-  __shared__ __attribute__((aligned(16))) float lds[S * STAGE];
-  const int M = prm.m, N = prm.n, K = prm.k;
-  const int nbm = (M + 127) / 128, nbn = (N + 127) / 128;
-  int bm, bn;
-  tile_coords(block, nbm, nbn, bm, bn);
-  const int m0 = bm * 128, n0 = bn * 128;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wm = wave & 1, wn = wave >> 1;
-  const int li = lane & 15, lg = lane >> 4;
-  const int nkt = K / 8;
-
-  flt4 cre[4][4], cim[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      cre[i][j] = flt4{0, 0, 0, 0};
-      cim[i][j] = flt4{0, 0, 0, 0};
-    }
-
-  auto issue = [&](int kt) {
-    float* st = lds + (kt % S) * STAGE;
-    CdldsOperand<A_KC>::issue(prm.a, prm.lda, m0, M, kt * 8, st, wave, lane);
-    CdldsOperand<B_KC>::issue(prm.b, prm.ldb, n0, N, kt * 8, st + TILE, wave, lane);
-  };
-#pragma unroll
-  for (int s = 0; s < S - 1; ++s)
-    if (s < nkt) issue(s);
-  for (int kt = 0; kt < nkt; ++kt) {
-    // this wave's loads of stage kt have landed once at most 4 per later stage are pending, and
-    // its LDS reads of stage kt-1 are done; the barrier extends both to the workgroup
-    const int later = min(S - 2, nkt - 1 - kt);
-    if (later >= 2) __builtin_amdgcn_s_waitcnt(0x070 | 8);
-    else if (later == 1) __builtin_amdgcn_s_waitcnt(0x070 | 4);
-    else __builtin_amdgcn_s_waitcnt(0x070);
-    __builtin_amdgcn_s_barrier();
-    if (kt + S - 1 < nkt) issue(kt + S - 1);
-    const float* st = lds + (kt % S) * STAGE;
-    v4f a[4], b[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      a[i] = CdldsOperand<A_KC>::frag(st, lg, wm * 64 + i * 16 + li);
-      if (A_CONJ) {
-        a[i][1] = -a[i][1];
-        a[i][3] = -a[i][3];
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      b[j] = CdldsOperand<B_KC>::frag(st + TILE, lg, wn * 64 + j * 16 + li);
-      if (B_CONJ) {
-        b[j][1] = -b[j][1];
-        b[j][3] = -b[j][3];
-      }
-    }
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float ar = a[i][2 * t], ai = a[i][2 * t + 1], nai = -ai;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const float br = b[j][2 * t], bi = b[j][2 * t + 1];
-          cre[i][j] = mfma(br, ar, cre[i][j]);
-          cre[i][j] = mfma(bi, nai, cre[i][j]);
-          cim[i][j] = mfma(bi, ar, cim[i][j]);
-          cim[i][j] = mfma(br, ai, cim[i][j]);
-        }
-      }
-  }
-
-  const float alr = prm.alpha, ali = prm.alpha_im;
-  const float ber = prm.beta, bei = prm.beta_im;
-  const bool acc_prev = prm.accumulate != 0;
-  const bool use_cin = ber != 0.0f || bei != 0.0f;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int gi = m0 + wm * 64 + i * 16 + li;
-    if (gi >= M) continue;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int gj = n0 + wn * 64 + j * 16 + out_col<float>(lane, r);
-        if (gj >= N) continue;
-        const float xr = cre[i][j][r], xi = cim[i][j][r];
-        float vr = alr * xr - ali * xi;
-        float vi = alr * xi + ali * xr;
-        float* dst = prm.c + 2 * ((long)gi + (long)gj * prm.ldc);
-        if (acc_prev) {
-          vr += dst[0];
-          vi += dst[1];
-        }
-        if (use_cin) {
-          const float* ci = prm.cin + 2 * ((long)gi + (long)gj * prm.ldcin);
-          const float cr = ci[0], cm = ci[1];
-          vr += ber * cr - bei * cm;
-          vi += ber * cm + bei * cr;
-        }
-        dst[0] = vr;
-        dst[1] = vi;
-      }
-    }
-  }
-}
-
-// The same tile software-pipelined as spipe_tile_at (two workgroups per CU): the fragments of
+// One tile, software-pipelined as spipe_tile_at (two workgroups per CU): the fragments of
 // stage kt+1 are read into a second register set (for a row-contiguous B, into the registers of
 // each B fragment as it is used up) while the 128 MFMAs of stage kt run, the loads of
 // stage kt+3 go between its first MFMAs, scheduling-group barriers pin that order, and the loads
-// always run (clamped to the last stage) so that every wait count is a constant. Per output block
-// the MFMA sequence is cdlds_tile's: the results are the same bits.
+// always run (clamped to the last stage) so that every wait count is a constant.
 template <bool A_KC, bool B_KC, bool A_CONJ, bool B_CONJ>
 __device__ __forceinline__ void cpipe_tile(const GemmParams<float>& prm, int block) {
   constexpr int TILE = 128 * 16, STAGE = 2 * TILE, S = 3;
@@ -1485,44 +1242,12 @@ __global__ __launch_bounds__(256, 2) void gemm_c_pipe_kernel(GemmParams<float> p
   cpipe_tile<A_KC, B_KC, A_CONJ, B_CONJ>(prm, blockIdx.x);
 }
 
-template <bool A_KC, bool B_KC, bool A_CONJ, bool B_CONJ, int S, int OCC>
-__global__ __launch_bounds__(256, OCC) void gemm_c_dlds_kernel(GemmParams<float> prm) {
-  cdlds_tile<A_KC, B_KC, A_CONJ, B_CONJ, S>(prm, blockIdx.x);
-}
-
-// The product of a grouped launch that workgroup w works on, with its parameters; -1 for a padding
-// workgroup. Products start on multiples of 8 workgroups, so that a workgroup's XCD
-// (blockIdx.x % 8) is the one tile_coords assumes.
-template <typename R>
-__device__ __forceinline__ int group_member(const TileGroup<R>& g, int w, int tiles_m, int tiles_n,
-                                            GemmParams<R>& prm, int& local) {
-  int t = 0;
-  while (t + 1 < g.count && w >= g.wg_start[t + 1]) ++t;
-  prm = g.base;
-  prm.m = g.m[t];
-  prm.n = g.n[t];
-  prm.a = g.a[t];
-  prm.lda = g.lda[t];
-  prm.b = g.b[t];
-  prm.ldb = g.ldb[t];
-  prm.c = g.c[t];
-  prm.ldc = g.ldc[t];
-  prm.cin = g.cin[t];
-  prm.ldcin = g.ldcin[t];
-  prm.beta = g.beta[t];
-  prm.beta_im = g.beta_im[t];
-  prm.accumulate = g.accumulate[t];
-  local = w - g.wg_start[t];
-  const int nbm = (prm.m + tiles_m - 1) / tiles_m, nbn = (prm.n + tiles_n - 1) / tiles_n;
-  return local < nbm * nbn ? t : -1;
-}
-
 // ---------------------------------------------------------------------------------------------
 // Software-pipelined FP64 GEMM, two tile widths BN: 128 x 256 workgroup tiles (2 x 2 waves of
 // 64 x 128, one workgroup per CU, so each wave has a SIMD to itself and its 32 accumulator blocks,
 // 256 registers, live in AGPRs) for the largest products, and 128 x 128 tiles (waves of 64 x 64,
 // two workgroups per CU, accumulators in VGPRs) for the others. The stage layouts are those of
-// gemm_d_dlds_kernel (k-step 8, a 3-stage direct-to-LDS ring; (128 + BN) x 64 bytes per stage).
+// dlds_tile_at (k-step 8, a 3-stage direct-to-LDS ring; (128 + BN) x 64 bytes per stage).
 // With one or two waves per SIMD little hides a stall, so the loop is pipelined by hand: the
 // fragments of stage kt+1 are read into a second register set while the 2 x 4 x BN/32 MFMAs of
 // stage kt run, the loads of stage kt+3 go between the first MFMAs, and scheduling-group barriers
@@ -1530,11 +1255,11 @@ __device__ __forceinline__ int group_member(const TileGroup<R>& g, int w, int ti
 // scheduling barriers at both ends of a stage keep the compiler from hoisting MFMAs above the
 // workgroup barrier, which made it rotate accumulators between AGPRs on every iteration. The loads
 // always run, the k index of stages past the end clamped to the last one (its slot is not read
-// again), so every wait count is a constant. Each output block sees the MFMA sequence of
-// gemm_d_dlds_kernel: the results are the same bits.
+// again), so every wait count is a constant. Both widths give every output block the same MFMA
+// sequence: the results are the same bits.
 // TN 8192^3 / 16384^3 on HBM-resident operands: 73.3 / 73.4 TFLOP/s with 128 x 256 tiles and
-// 73.2 / 72.0 with 128 x 128 tiles at two per CU, against 71.1 / 71.1 for gemm_d_dlds_kernel (128 x
-// 128, three per CU, no software pipelining); 128 x 256 without the scheduling groups 69.9 / 70.1,
+// 73.2 / 72.0 with 128 x 128 tiles at two per CU, against 71.1 / 71.1 for 128 x 128 tiles at
+// three per CU without software pipelining; 128 x 256 without the scheduling groups 69.9 / 70.1,
 // with a 4-stage ring 73.0 / 73.1, with one load per 4 MFMAs 72.4 / 72.6. 40000^3: 72.5 with 128 x
 // 256 tiles, 69.0 with 128 x 128 (twice the B re-reads); on the 8064 x 8192 x 8000 blocks of the
 // host-to-host call 128 x 128 tiles win (72.3 against 69.3 with C read in the epilogue): with one
@@ -1807,19 +1532,6 @@ __global__ __launch_bounds__(256, 2) void gemm_s_pipe_group_kernel(SgemmGroup g)
   spipe_tile_at<A_KC, B_KC, 128, 128>(prm, bm * 128, bn * 128);
 }
 
-// Grouped FP32 tile GEMMs (256 x 256 workgroup tiles: every member has m, n > 128). Padding
-// workgroups exit before any barrier.
-template <bool A_KC, bool B_KC, int S, int OCC>
-__global__ __launch_bounds__(512, OCC) void gemm_s_dlds_group_kernel(SgemmGroup g) {
-  GemmParams<float> prm;
-  int local;
-  if (group_member(g, blockIdx.x, 256, 256, prm, local) < 0) return;
-  const int nbm = (prm.m + 255) / 256, nbn = (prm.n + 255) / 256;
-  int bm, bn;
-  tile_coords(local, nbm, nbn, bm, bn);
-  sdlds_tile_at<A_KC, B_KC, S, 256, 256>(prm, bm * 256, bn * 256);
-}
-
 // Grouped complex FP32 tile GEMMs (128 x 128 complex workgroup tiles).
 template <bool A_KC, bool B_KC, bool A_CONJ, bool B_CONJ>
 __global__ __launch_bounds__(256, 2) void gemm_c_pipe_group_kernel(SgemmGroup g) {
@@ -1829,19 +1541,11 @@ __global__ __launch_bounds__(256, 2) void gemm_c_pipe_group_kernel(SgemmGroup g)
   cpipe_tile<A_KC, B_KC, A_CONJ, B_CONJ>(prm, local);
 }
 
-template <bool A_KC, bool B_KC, bool A_CONJ, bool B_CONJ, int S, int OCC>
-__global__ __launch_bounds__(256, OCC) void gemm_c_dlds_group_kernel(SgemmGroup g) {
-  GemmParams<float> prm;
-  int local;
-  if (group_member(g, blockIdx.x, 128, 128, prm, local) < 0) return;
-  cdlds_tile<A_KC, B_KC, A_CONJ, B_CONJ, S>(prm, local);
-}
-
 // ---------------------------------------------------------------------------------------------
 // Complex FP64 GEMM with direct global->LDS loads (ZGEMM), the complex sibling of
-// gemm_d_dlds_kernel. WG tile 64x64 complex, 2x2 waves of 32x32 (2x2 blocks, re and im
-// accumulators, four real MFMAs per block update), k-step 8 complex per stage, S-stage ring of
-// 16 KB stages (S = 3, three workgroups per CU). A 16-byte chunk is one complex element, so one
+// dlds_tile_at. WG tile 64x64 complex, 2x2 waves of 32x32 (2x2 blocks, re and im
+// accumulators, four real MFMAs per block update), k-step 8 complex per stage, a 3-stage ring of
+// 16 KB stages. A 16-byte chunk is one complex element, so one
 // ds_read_b128 yields both MFMA operands (re, im) of a lane.
 //   k-contiguous operand (A for 'T'/'C', B for 'N'): LDS [row][slot], 128 bytes per row; a wave
 //     instruction fills 8 rows, lanes 8j..8j+7 reading the 128 contiguous bytes of row j, lane l
@@ -1850,8 +1554,7 @@ __global__ __launch_bounds__(256, OCC) void gemm_c_dlds_group_kernel(SgemmGroup 
 //   row-contiguous operand (A for 'N', B for 'T'/'C'): LDS [k][row], a wave instruction fills
 //     the 64 rows of one k (1 KB contiguous in global memory).
 // Conjugation ('C') negates the imaginary fragment in registers. Rows beyond the matrix read a
-// clamped in-bounds row. K must be a multiple of 8 (the launcher hands a remainder to
-// gemm_cplx_kernel).
+// clamped in-bounds row; a ragged last k-step is read separately (ring_steps).
 // ---------------------------------------------------------------------------------------------
 template <bool KC>
 struct ZdldsOperand {
@@ -1882,116 +1585,10 @@ struct ZdldsOperand {
   }
 };
 
-template <bool A_KC, bool B_KC, bool A_CONJ, bool B_CONJ, int S>
-__device__ __forceinline__ void zdlds_tile(const GemmParams<double>& prm, int block) {
-  constexpr int TILE = 64 * 8 * 2;  // doubles per operand and stage (8 KB)
-  constexpr int STAGE = 2 * TILE;
-  __shared__ __attribute__((aligned(16))) double lds[S * STAGE];
-  const int M = prm.m, N = prm.n, K = prm.k;
-  const int nbm = (M + 63) / 64, nbn = (N + 63) / 64;
-  int bm, bn;
-  tile_coords(block, nbm, nbn, bm, bn);
-  const int m0 = bm * 64, n0 = bn * 64;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wm = wave & 1, wn = wave >> 1;
-  const int li = lane & 15, lg = lane >> 4;
-  const int nkt = K / 8;
-
-  dbl4 cre[2][2], cim[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      cre[i][j] = dbl4{0, 0, 0, 0};
-      cim[i][j] = dbl4{0, 0, 0, 0};
-    }
-
-  auto issue = [&](int kt) {
-    double* st = lds + (kt % S) * STAGE;
-    ZdldsOperand<A_KC>::issue(prm.a, prm.lda, m0, M, kt * 8, st, wave, lane);
-    ZdldsOperand<B_KC>::issue(prm.b, prm.ldb, n0, N, kt * 8, st + TILE, wave, lane);
-  };
-#pragma unroll
-  for (int s = 0; s < S - 1; ++s)
-    if (s < nkt) issue(s);
-  for (int kt = 0; kt < nkt; ++kt) {
-    // this wave's loads of stage kt have landed once at most 4 per later stage are pending, and
-    // its LDS reads of stage kt-1 are done; the barrier extends both to the workgroup
-    const int later = min(S - 2, nkt - 1 - kt);
-    if (later >= 3) __builtin_amdgcn_s_waitcnt(0x070 | 12);
-    else if (later == 2) __builtin_amdgcn_s_waitcnt(0x070 | 8);
-    else if (later == 1) __builtin_amdgcn_s_waitcnt(0x070 | 4);
-    else __builtin_amdgcn_s_waitcnt(0x070);
-    __builtin_amdgcn_s_barrier();
-    if (kt + S - 1 < nkt) issue(kt + S - 1);
-    const double* st = lds + (kt % S) * STAGE;
-#pragma unroll
-    for (int kk = 0; kk < 2; ++kk) {
-      v2d a[2], b[2];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        a[i] = ZdldsOperand<A_KC>::elem(st, wm * 32 + i * 16 + li, 4 * kk + lg);
-        if (A_CONJ) a[i][1] = -a[i][1];
-      }
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        b[j] = ZdldsOperand<B_KC>::elem(st + TILE, wn * 32 + j * 16 + li, 4 * kk + lg);
-        if (B_CONJ) b[j][1] = -b[j][1];
-      }
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const double nai = -a[i][1];
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          cre[i][j] = mfma(b[j][0], a[i][0], cre[i][j]);
-          cre[i][j] = mfma(b[j][1], nai, cre[i][j]);
-          cim[i][j] = mfma(b[j][1], a[i][0], cim[i][j]);
-          cim[i][j] = mfma(b[j][0], a[i][1], cim[i][j]);
-        }
-      }
-    }
-  }
-
-  const double alr = prm.alpha, ali = prm.alpha_im;
-  const double ber = prm.beta, bei = prm.beta_im;
-  const bool acc_prev = prm.accumulate != 0;
-  const bool use_cin = ber != 0.0 || bei != 0.0;
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int gi = m0 + wm * 32 + i * 16 + li;
-    if (gi >= M) continue;
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int gj = n0 + wn * 32 + j * 16 + out_col<double>(lane, r);
-        if (gj >= N) continue;
-        const double xr = cre[i][j][r], xi = cim[i][j][r];
-        double vr = alr * xr - ali * xi;
-        double vi = alr * xi + ali * xr;
-        double* dst = prm.c + 2 * ((long)gi + (long)gj * prm.ldc);
-        if (acc_prev) {
-          vr += dst[0];
-          vi += dst[1];
-        }
-        if (use_cin) {
-          const double* ci = prm.cin + 2 * ((long)gi + (long)gj * prm.ldcin);
-          const double cr = ci[0], cm = ci[1];
-          vr += ber * cr - bei * cm;
-          vi += ber * cm + bei * cr;
-        }
-        dst[0] = vr;
-        dst[1] = vi;
-      }
-    }
-  }
-}
-
-// The same tile software-pipelined as dbig_tile_at (two workgroups per CU): the fragments of stage
+// One tile, software-pipelined as dbig_tile_at (two workgroups per CU): the fragments of stage
 // kt+1 are read into a second register set while the 32 MFMAs of stage kt run, the 4 loads of
 // stage kt+3 go between its first MFMAs, scheduling-group barriers pin that order, and the loads
-// always run (clamped to the last stage) so that every wait count is a constant. Per output block
-// the MFMA sequence is zdlds_tile's: the results are the same bits.
+// always run (clamped to the last stage) so that every wait count is a constant.
 template <bool A_KC, bool B_KC, bool A_CONJ, bool B_CONJ>
 __device__ __forceinline__ void zpipe_tile(const GemmParams<double>& prm, int block) {
   constexpr int TILE = 64 * 8 * 2, STAGE = 2 * TILE, S = 3;
@@ -2171,36 +1768,6 @@ __global__ __launch_bounds__(256, 2) void gemm_z_pipe_group_kernel(DgemmGroup g)
   zpipe_tile<A_KC, B_KC, A_CONJ, B_CONJ>(prm, local);
 }
 
-template <bool A_KC, bool B_KC, bool A_CONJ, bool B_CONJ, int S, int OCC = 2>
-__global__ __launch_bounds__(256, OCC) void gemm_z_dlds_kernel(GemmParams<double> prm) {
-  zdlds_tile<A_KC, B_KC, A_CONJ, B_CONJ, S>(prm, blockIdx.x);
-}
-
-// The complex sibling of gemm_d_dlds_group_kernel (64x64 complex workgroup tiles).
-template <bool A_KC, bool B_KC, bool A_CONJ, bool B_CONJ, int S, int OCC = 2>
-__global__ __launch_bounds__(256, OCC) void gemm_z_dlds_group_kernel(DgemmGroup g) {
-  const int w = blockIdx.x;
-  int t = 0;
-  while (t + 1 < g.count && w >= g.wg_start[t + 1]) ++t;
-  GemmParams<double> prm = g.base;
-  prm.m = g.m[t];
-  prm.n = g.n[t];
-  prm.a = g.a[t];
-  prm.lda = g.lda[t];
-  prm.b = g.b[t];
-  prm.ldb = g.ldb[t];
-  prm.c = g.c[t];
-  prm.ldc = g.ldc[t];
-  prm.cin = g.cin[t];
-  prm.ldcin = g.ldcin[t];
-  prm.beta = g.beta[t];
-  prm.beta_im = g.beta_im[t];
-  prm.accumulate = g.accumulate[t];
-  const int local = w - g.wg_start[t];
-  if (local >= ((prm.m + 63) / 64) * ((prm.n + 63) / 64)) return;
-  zdlds_tile<A_KC, B_KC, A_CONJ, B_CONJ, S>(prm, local);
-}
-
 inline bool is_kc_a(char op) { return op != 'N'; }
 inline bool is_kc_b(char op) { return op == 'N'; }
 
@@ -2237,12 +1804,6 @@ hipError_t launch_cplx(const GemmParams<R>& p, hipStream_t s) {
   return launch_cplx_conj<R, false, false>(p, s, grid, block);
 }
 
-// Which FP64 kernel a product of m x n runs on (for a group: its members together), by what the
-// measurements favour: the 128 x 256 tiles for products of at least 2^27 elements of C (their
-// halved B re-reads pay; 40000^2: 72.5 against 69.0 TFLOP/s), the pipelined 128 x 128 tiles at
-// two per CU below that (8064 x 8192 blocks: 72.3 against 69.3 with C read in the epilogue), and
-// the 128 x 128 kernel at three per CU when neither grid has two workgroups per CU to fill the
-// device with.
 int device_cus() {
   static const int cus = [] {
     int dev = 0, c = 256;
@@ -2252,67 +1813,213 @@ int device_cus() {
   }();
   return cus;
 }
-long dgemm_tiles(int m, int n, int bn) { return (long)((m + 127) / 128) * ((n + bn - 1) / bn); }
-enum DgemmKind { kDgemmRing3 = 0, kDgemmPipe = 1, kDgemmBig = 2 };
-// largest: the largest member's m x n; big_ok: every member has m, n > 128; tiles128 / tiles256:
-// the workgroups of all members on either grid
-// FP32: the pipelined 128 x 128 tiles when the product (a group: its members together) has two of
-// them per CU
-bool sgemm_pipe(long tiles128) { return tiles128 >= 2L * device_cus(); }
-bool sgemm_pipe(int m, int n) { return sgemm_pipe(dgemm_tiles(m, n, 128)); }
-int dgemm_kind(long largest, bool big_ok, long tiles128, long tiles256) {
-  if (big_ok && largest >= (1L << 27) && tiles256 >= 2L * device_cus()) return kDgemmBig;
-  if (tiles128 >= 2L * device_cus()) return kDgemmPipe;
-  return kDgemmRing3;
+long grid_tiles(int m, int n, int bm, int bn) { return (long)((m + bm - 1) / bm) * ((n + bn - 1) / bn); }
+
+// Which kernels a product runs on: a function of the product alone, so that a grouped launch gives
+// each of its products the bits of a launch of its own.
+//   kReal  register-staged (variant 0, k = 0, an extreme leading dimension);
+//   kKs    the small tiles that split k over a workgroup's waves, of shape `shape`;
+//   kPipe  the pipelined 128 x 128 (complex double: 64 x 64) tiles, for which there must be two per
+//          CU, where the estimated times say so. Their times lie within a few percent of each
+//          other once both have many tiles per CU; what decides is how the last round of tiles
+//          fills the device, and there the small tiles win: DGEMM 3000^3 on 576 tiles of 128 x 128
+//          (2.25 per CU) 1048 us, on 64 x 64 781 us. The pipelined ones re-read the operands half
+//          as often, so they keep near ties (2%) and, but for complex double (whose small tiles of
+//          48 x 48 are as large as its pipelined ones), everything from 12 tiles per CU on.
+struct Route {
+  enum Kind { kReal, kKs, kPipe } kind;
+  int shape;
+};
+template <typename R>
+Route route(KsType t, const GemmParams<R>& p) {
+  if (p.variant != 1 || p.k <= 0) return {Route::kReal, 0};
+  const bool cplx = t == KsType::Z || t == KsType::C;
+  const int edge = t == KsType::Z ? 64 : 128, cus = device_cus();
+  const long tiles = grid_tiles(p.m, p.n, edge, edge);
+  // what the chunked row loads of both kernels need of a short leading dimension
+  const bool chunks_ok = ks_chunks_ok<R>(cplx, p.opa != 'N', p.m, p.lda) && ks_chunks_ok<R>(cplx, p.opb == 'N', p.n, p.ldb);
+  const bool pipe = tiles >= 2L * cus && chunks_ok;
+  if (!ks_takes(p, cplx)) return {pipe ? Route::kPipe : Route::kReal, 0};
+  double us = 0;
+  const int shape = ks_shape(t, p.m, p.n, p.k, cus, &us);
+  const bool many = t != KsType::Z && tiles >= 12L * cus;
+  if (pipe && (many || 0.98 * pipe_time(t, tiles, p.k, cus) <= us)) return {Route::kPipe, 0};
+  return {Route::kKs, shape};
 }
 
-int dgemm_kind(const GemmParams<double>& p) {
-  return dgemm_kind((long)p.m * p.n, p.m > 128 && p.n > 128, dgemm_tiles(p.m, p.n, 128), dgemm_tiles(p.m, p.n, 256));
-}
+// The pipelined FP64 tiles: 128 x 256 for products of at least 2^27 elements of C (their halved B
+// re-reads pay; 40000^2: 72.5 against 69.0 TFLOP/s), 128 x 128 at two per CU below that (8064 x
+// 8192 blocks: 72.3 against 69.3 with C read in the epilogue). The same bits. largest: the largest
+// m x n of the launch; big_ok: every product has m, n > 128.
+bool dgemm_wide(long largest, bool big_ok) { return big_ok && largest >= (1L << 27); }
 
-template <bool AKC, bool BKC>
-void launch_dlds(const GemmParams<double>& p, hipStream_t s) {
-  const int kind = dgemm_kind(p);
-  if (kind == kDgemmBig) {
-    hipLaunchKernelGGL((gemm_d_big_kernel<AKC, BKC>), dim3(dgemm_tiles(p.m, p.n, 256)), dim3(256), 0, s, p);
-    return;
-  }
-  if (kind == kDgemmPipe) {
-    hipLaunchKernelGGL((gemm_d_pipe_kernel<AKC, BKC>), dim3(dgemm_tiles(p.m, p.n, 128)), dim3(256), 0, s, p);
-    return;
-  }
-  const int nbm = (p.m + 127) / 128, nbn = (p.n + 127) / 128;
-  // 3-stage ring, 3 workgroups per CU (48 KB of LDS each): 70.9 TFLOP/s on TN 8192^3 against
-  // 68.8 for 4 stages at 2 per CU, 68.7 for 5 at 2, 43.5 for 6 at 1
-  hipLaunchKernelGGL((gemm_d_dlds_kernel<AKC, BKC, 3, 3>), dim3(nbm * nbn), dim3(256), 0, s, p);
-}
-
-// FP64 through the direct-LDS kernels. The pipelined ones take any m, n and k; the three-per-CU one
-// the largest multiple of 8 in K, a remainder going to gemm_real_kernel, accumulating (beta only on
-// the first part).
-hipError_t launch_gemm_d_direct(const GemmParams<double>& p, hipStream_t s) {
+hipError_t launch_pipe_d(const GemmParams<double>& p, hipStream_t s) {
   const bool akc = is_kc_a(p.opa), bkc = is_kc_b(p.opb);
-  const bool pipe = p.k > 0 && dgemm_kind(p) != kDgemmRing3;
-  const int k8 = pipe ? p.k : p.k / 8 * 8;
-  // for the three-per-CU kernel a row-contiguous operand with an odd row count would need a 2-row
-  // chunk that straddles the last row: such shapes keep the register-staged kernel
-  const bool pairs_ok = (akc || p.m % 2 == 0) && (bkc || p.n % 2 == 0);
-  if (!pipe && (k8 == 0 || p.m < 2 || p.n < 2 || !pairs_ok)) return launch_real<double>(p, s);
-  GemmParams<double> q = p;
-  q.k = k8;
-  if (akc && bkc) launch_dlds<true, true>(q, s);
-  else if (akc) launch_dlds<true, false>(q, s);
-  else if (bkc) launch_dlds<false, true>(q, s);
-  else launch_dlds<false, false>(q, s);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess || k8 == p.k) return e;
-  GemmParams<double> r = p;
-  r.k = p.k - k8;
-  r.a = p.a + (akc ? (long)k8 : (long)k8 * p.lda);
-  r.b = p.b + (bkc ? (long)k8 : (long)k8 * p.ldb);
-  r.accumulate = 1;
-  r.beta = 0.0;
-  return launch_real<double>(r, s);
+  const bool wide = dgemm_wide((long)p.m * p.n, p.m > 128 && p.n > 128);
+  const dim3 grid(grid_tiles(p.m, p.n, 128, wide ? 256 : 128)), block(256);
+  if (wide) {
+    if (akc && bkc) hipLaunchKernelGGL((gemm_d_big_kernel<true, true>), grid, block, 0, s, p);
+    else if (akc) hipLaunchKernelGGL((gemm_d_big_kernel<true, false>), grid, block, 0, s, p);
+    else if (bkc) hipLaunchKernelGGL((gemm_d_big_kernel<false, true>), grid, block, 0, s, p);
+    else hipLaunchKernelGGL((gemm_d_big_kernel<false, false>), grid, block, 0, s, p);
+    return hipGetLastError();
+  }
+  if (akc && bkc) hipLaunchKernelGGL((gemm_d_pipe_kernel<true, true>), grid, block, 0, s, p);
+  else if (akc) hipLaunchKernelGGL((gemm_d_pipe_kernel<true, false>), grid, block, 0, s, p);
+  else if (bkc) hipLaunchKernelGGL((gemm_d_pipe_kernel<false, true>), grid, block, 0, s, p);
+  else hipLaunchKernelGGL((gemm_d_pipe_kernel<false, false>), grid, block, 0, s, p);
+  return hipGetLastError();
+}
+
+hipError_t launch_pipe_d_group(const GemmParams<double>* tiles, int count, hipStream_t s) {
+  bool big_ok = true;
+  long largest = 0;
+  for (int t = 0; t < count; ++t) {
+    big_ok = big_ok && tiles[t].m > 128 && tiles[t].n > 128;
+    largest = std::max(largest, (long)tiles[t].m * tiles[t].n);
+  }
+  const bool wide = dgemm_wide(largest, big_ok);
+  DgemmGroup g;
+  int wg = 0;
+  if (!make_group(tiles, count, 128, wide ? 256 : 128, g, wg)) return hipErrorInvalidValue;
+  const bool akc = is_kc_a(g.base.opa), bkc = is_kc_b(g.base.opb);
+  const dim3 grid(wg), block(256);
+  if (wide) {
+    if (akc && bkc) hipLaunchKernelGGL((gemm_d_big_group_kernel<true, true>), grid, block, 0, s, g);
+    else if (akc) hipLaunchKernelGGL((gemm_d_big_group_kernel<true, false>), grid, block, 0, s, g);
+    else if (bkc) hipLaunchKernelGGL((gemm_d_big_group_kernel<false, true>), grid, block, 0, s, g);
+    else hipLaunchKernelGGL((gemm_d_big_group_kernel<false, false>), grid, block, 0, s, g);
+    return hipGetLastError();
+  }
+  if (akc && bkc) hipLaunchKernelGGL((gemm_d_pipe_group_kernel<true, true>), grid, block, 0, s, g);
+  else if (akc) hipLaunchKernelGGL((gemm_d_pipe_group_kernel<true, false>), grid, block, 0, s, g);
+  else if (bkc) hipLaunchKernelGGL((gemm_d_pipe_group_kernel<false, true>), grid, block, 0, s, g);
+  else hipLaunchKernelGGL((gemm_d_pipe_group_kernel<false, false>), grid, block, 0, s, g);
+  return hipGetLastError();
+}
+
+hipError_t launch_pipe_s(const GemmParams<float>& p, hipStream_t s) {
+  const bool akc = is_kc_a(p.opa), bkc = is_kc_b(p.opb);
+  const dim3 grid(grid_tiles(p.m, p.n, 128, 128)), block(256);
+  if (akc && bkc) hipLaunchKernelGGL((gemm_s_pipe_kernel<true, true>), grid, block, 0, s, p);
+  else if (akc) hipLaunchKernelGGL((gemm_s_pipe_kernel<true, false>), grid, block, 0, s, p);
+  else if (bkc) hipLaunchKernelGGL((gemm_s_pipe_kernel<false, true>), grid, block, 0, s, p);
+  else hipLaunchKernelGGL((gemm_s_pipe_kernel<false, false>), grid, block, 0, s, p);
+  return hipGetLastError();
+}
+
+hipError_t launch_pipe_s_group(const GemmParams<float>* tiles, int count, hipStream_t s) {
+  SgemmGroup g;
+  int wg = 0;
+  if (!make_group(tiles, count, 128, 128, g, wg)) return hipErrorInvalidValue;
+  const bool akc = is_kc_a(g.base.opa), bkc = is_kc_b(g.base.opb);
+  const dim3 grid(wg), block(256);
+  if (akc && bkc) hipLaunchKernelGGL((gemm_s_pipe_group_kernel<true, true>), grid, block, 0, s, g);
+  else if (akc) hipLaunchKernelGGL((gemm_s_pipe_group_kernel<true, false>), grid, block, 0, s, g);
+  else if (bkc) hipLaunchKernelGGL((gemm_s_pipe_group_kernel<false, true>), grid, block, 0, s, g);
+  else hipLaunchKernelGGL((gemm_s_pipe_group_kernel<false, false>), grid, block, 0, s, g);
+  return hipGetLastError();
+}
+
+// The nine layouts of a complex kernel: k-contiguity of A and B and their conjugation.
+#define TMM_CPLX_LAYOUTS(opa, opb, LAUNCH)                         \
+  do {                                                             \
+    const bool ca_ = (opa) == 'C', cb_ = (opb) == 'C';             \
+    if (is_kc_a(opa) && is_kc_b(opb)) {                            \
+      if (ca_) LAUNCH(true, true, true, false);                    \
+      else LAUNCH(true, true, false, false);                       \
+    } else if (is_kc_a(opa)) {                                     \
+      if (ca_ && cb_) LAUNCH(true, false, true, true);             \
+      else if (ca_) LAUNCH(true, false, true, false);              \
+      else if (cb_) LAUNCH(true, false, false, true);              \
+      else LAUNCH(true, false, false, false);                      \
+    } else if (is_kc_b(opb)) {                                     \
+      LAUNCH(false, true, false, false);                           \
+    } else if (cb_) {                                              \
+      LAUNCH(false, false, false, true);                           \
+    } else {                                                       \
+      LAUNCH(false, false, false, false);                          \
+    }                                                              \
+  } while (0)
+
+hipError_t launch_pipe_z(const GemmParams<double>& p, hipStream_t s) {
+  const dim3 grid(grid_tiles(p.m, p.n, 64, 64)), block(256);
+#define TMM_Z(AK, BK, CA, CB) hipLaunchKernelGGL((gemm_z_pipe_kernel<AK, BK, CA, CB>), grid, block, 0, s, p)
+  TMM_CPLX_LAYOUTS(p.opa, p.opb, TMM_Z);
+#undef TMM_Z
+  return hipGetLastError();
+}
+
+hipError_t launch_pipe_z_group(const GemmParams<double>* tiles, int count, hipStream_t s) {
+  DgemmGroup g;
+  int wg = 0;
+  if (!make_group(tiles, count, 64, 64, g, wg)) return hipErrorInvalidValue;
+  const dim3 grid(wg), block(256);
+#define TMM_Z(AK, BK, CA, CB) hipLaunchKernelGGL((gemm_z_pipe_group_kernel<AK, BK, CA, CB>), grid, block, 0, s, g)
+  TMM_CPLX_LAYOUTS(g.base.opa, g.base.opb, TMM_Z);
+#undef TMM_Z
+  return hipGetLastError();
+}
+
+hipError_t launch_pipe_c(const GemmParams<float>& p, hipStream_t s) {
+  const dim3 grid(grid_tiles(p.m, p.n, 128, 128)), block(256);
+#define TMM_C(AK, BK, CA, CB) hipLaunchKernelGGL((gemm_c_pipe_kernel<AK, BK, CA, CB>), grid, block, 0, s, p)
+  TMM_CPLX_LAYOUTS(p.opa, p.opb, TMM_C);
+#undef TMM_C
+  return hipGetLastError();
+}
+
+hipError_t launch_pipe_c_group(const GemmParams<float>* tiles, int count, hipStream_t s) {
+  SgemmGroup g;
+  int wg = 0;
+  if (!make_group(tiles, count, 128, 128, g, wg)) return hipErrorInvalidValue;
+  const dim3 grid(wg), block(256);
+#define TMM_C(AK, BK, CA, CB) hipLaunchKernelGGL((gemm_c_pipe_group_kernel<AK, BK, CA, CB>), grid, block, 0, s, g)
+  TMM_CPLX_LAYOUTS(g.base.opa, g.base.opb, TMM_C);
+#undef TMM_C
+  return hipGetLastError();
+}
+
+// The kernels of one element type.
+template <typename R>
+struct Kernels {
+  KsType type;
+  hipError_t (*real)(const GemmParams<R>&, hipStream_t);
+  hipError_t (*ks)(const GemmParams<R>&, int, hipStream_t);
+  hipError_t (*ks_group)(const GemmParams<R>*, int, hipStream_t);
+  hipError_t (*pipe)(const GemmParams<R>&, hipStream_t);
+  hipError_t (*pipe_group)(const GemmParams<R>*, int, hipStream_t);
+};
+const Kernels<double> kD = {KsType::D, launch_real<double>, launch_ks_d, launch_ks_d_group, launch_pipe_d, launch_pipe_d_group};
+const Kernels<float> kS = {KsType::S, launch_real<float>, launch_ks_s, launch_ks_s_group, launch_pipe_s, launch_pipe_s_group};
+const Kernels<double> kZ = {KsType::Z, launch_cplx<double>, launch_ks_z, launch_ks_z_group, launch_pipe_z, launch_pipe_z_group};
+const Kernels<float> kC = {KsType::C, launch_cplx<float>, launch_ks_c, launch_ks_c_group, launch_pipe_c, launch_pipe_c_group};
+
+template <typename R>
+hipError_t launch_one(const Kernels<R>& k, const GemmParams<R>& p, hipStream_t s) {
+  if (p.m <= 0 || p.n <= 0) return hipSuccess;
+  const Route r = route(k.type, p);
+  if (r.kind == Route::kKs) return k.ks(p, r.shape, s);
+  return r.kind == Route::kPipe ? k.pipe(p, s) : k.real(p, s);
+}
+
+// The products of a group by the kernel each would run on alone, one launch per kernel.
+template <typename R>
+hipError_t launch_many(const Kernels<R>& k, const GemmParams<R>* tiles, int count, hipStream_t s) {
+  if (count <= 0) return hipSuccess;
+  if (count > kDgemmGroupMax) return hipErrorInvalidValue;
+  GemmParams<R> pipe[kDgemmGroupMax], ks[kDgemmGroupMax];
+  int npipe = 0, nks = 0;
+  hipError_t e = hipSuccess;
+  for (int t = 0; t < count && e == hipSuccess; ++t) {
+    const Route::Kind kind = route(k.type, tiles[t]).kind;
+    if (kind == Route::kKs) ks[nks++] = tiles[t];
+    else if (kind == Route::kPipe) pipe[npipe++] = tiles[t];
+    else e = launch_one(k, tiles[t], s);
+  }
+  if (e == hipSuccess && npipe > 0) e = k.pipe_group(pipe, npipe, s);
+  if (e == hipSuccess && nks > 0) e = nks == 1 ? launch_one(k, ks[0], s) : k.ks_group(ks, nks, s);
+  return e;
 }
 
 }  // namespace
@@ -2322,10 +2029,7 @@ bool dgemm_groupable(const GemmParams<double>& p) {
   return p.variant == 1 && p.k >= 8 && p.k % 8 == 0 && p.m >= 2 && p.n >= 2 && (akc || p.m % 2 == 0) &&
          (bkc || p.n % 2 == 0);
 }
-
 bool zgemm_groupable(const GemmParams<double>& p) { return p.variant == 1 && p.k >= 8 && p.k % 8 == 0 && p.m >= 1 && p.n >= 1; }
-// FP32 groups run the 256 x 256 tiles: m, n > 128, K a multiple of 16, row-contiguous operands in
-// whole 4-row chunks (what launch_gemm_s_direct sends to that kernel without a remainder launch)
 bool sgemm_groupable(const GemmParams<float>& p) {
   const bool akc = is_kc_a(p.opa), bkc = is_kc_b(p.opb);
   return p.variant == 1 && p.k >= 16 && p.k % 16 == 0 && p.m > 128 && p.n > 128 && (akc || p.m % 4 == 0) &&
@@ -2337,174 +2041,14 @@ bool cgemm_groupable(const GemmParams<float>& p) {
          (bkc || p.n % 2 == 0);
 }
 
-namespace {
-// The group descriptor of `count` products of one shape class; false if they do not form one.
-// edge_m, edge_n: rows and columns of C per workgroup of the group's kernel.
-template <typename R, typename Pred>
-bool make_group(const GemmParams<R>* tiles, int count, int edge_m, int edge_n, Pred groupable, TileGroup<R>& g,
-                int& wg) {
-  if (count <= 0 || count > kDgemmGroupMax) return false;
-  g = TileGroup<R>{};
-  g.base = tiles[0];
-  g.count = count;
-  wg = 0;
-  for (int t = 0; t < count; ++t) {
-    const GemmParams<R>& p = tiles[t];
-    if (!groupable(p) || p.k != g.base.k || p.opa != g.base.opa || p.opb != g.base.opb ||
-        p.alpha != g.base.alpha || p.alpha_im != g.base.alpha_im)
-      return false;
-    g.wg_start[t] = wg;
-    wg += (((p.m + edge_m - 1) / edge_m) * ((p.n + edge_n - 1) / edge_n) + 7) / 8 * 8;
-    g.m[t] = p.m;
-    g.n[t] = p.n;
-    g.a[t] = p.a;
-    g.lda[t] = p.lda;
-    g.b[t] = p.b;
-    g.ldb[t] = p.ldb;
-    g.c[t] = p.c;
-    g.ldc[t] = p.ldc;
-    g.cin[t] = p.cin;
-    g.ldcin[t] = p.ldcin;
-    g.beta[t] = p.beta;
-    g.beta_im[t] = p.beta_im;
-    g.accumulate[t] = p.accumulate;
-  }
-  g.wg_start[count] = wg;
-  return true;
-}
-}  // namespace
-
-hipError_t launch_gemm_z_group(const GemmParams<double>* tiles, int count, hipStream_t s) {
-  DgemmGroup g;
-  int wg = 0;
-  if (count <= 0) return hipSuccess;
-  if (!make_group(tiles, count, 64, 64, zgemm_groupable, g, wg)) return hipErrorInvalidValue;
-  const bool akc = is_kc_a(g.base.opa), bkc = is_kc_b(g.base.opb);
-  const bool ca = g.base.opa == 'C', cb = g.base.opb == 'C';
-  // the pipelined tile at two workgroups per CU when the group has two tiles per CU to fill it
-  const bool pipe = wg >= 2L * device_cus();
-#define TMM_ZG(AK, BK, CA, CB)                                                                        \
-  do {                                                                                               \
-    if (pipe) hipLaunchKernelGGL((gemm_z_pipe_group_kernel<AK, BK, CA, CB>), dim3(wg), dim3(256), 0, s, g); \
-    else hipLaunchKernelGGL((gemm_z_dlds_group_kernel<AK, BK, CA, CB, 3, 3>), dim3(wg), dim3(256), 0, s, g); \
-  } while (0)
-  if (akc && bkc) {
-    if (ca) TMM_ZG(true, true, true, false);
-    else TMM_ZG(true, true, false, false);
-  } else if (akc) {
-    if (ca && cb) TMM_ZG(true, false, true, true);
-    else if (ca) TMM_ZG(true, false, true, false);
-    else if (cb) TMM_ZG(true, false, false, true);
-    else TMM_ZG(true, false, false, false);
-  } else if (bkc) {
-    TMM_ZG(false, true, false, false);
-  } else {
-    if (cb) TMM_ZG(false, false, false, true);
-    else TMM_ZG(false, false, false, false);
-  }
-#undef TMM_ZG
-  return hipGetLastError();
-}
-
-hipError_t launch_gemm_d_group(const GemmParams<double>* tiles, int count, hipStream_t s) {
-  DgemmGroup g;
-  int wg = 0;
-  if (count <= 0) return hipSuccess;
-  bool big_ok = true;
-  long largest = 0, t128 = 0, t256 = 0;
-  for (int t = 0; t < count; ++t) {
-    big_ok = big_ok && tiles[t].m > 128 && tiles[t].n > 128;
-    largest = std::max(largest, (long)tiles[t].m * tiles[t].n);
-    t128 += dgemm_tiles(tiles[t].m, tiles[t].n, 128);
-    t256 += dgemm_tiles(tiles[t].m, tiles[t].n, 256);
-  }
-  const int kind = dgemm_kind(largest, big_ok, t128, t256);
-  if (!make_group(tiles, count, 128, kind == kDgemmBig ? 256 : 128, dgemm_groupable, g, wg))
-    return hipErrorInvalidValue;
-  const bool akc = is_kc_a(g.base.opa), bkc = is_kc_b(g.base.opb);
-  if (kind == kDgemmBig) {
-    if (akc && bkc) hipLaunchKernelGGL((gemm_d_big_group_kernel<true, true>), dim3(wg), dim3(256), 0, s, g);
-    else if (akc) hipLaunchKernelGGL((gemm_d_big_group_kernel<true, false>), dim3(wg), dim3(256), 0, s, g);
-    else if (bkc) hipLaunchKernelGGL((gemm_d_big_group_kernel<false, true>), dim3(wg), dim3(256), 0, s, g);
-    else hipLaunchKernelGGL((gemm_d_big_group_kernel<false, false>), dim3(wg), dim3(256), 0, s, g);
-    return hipGetLastError();
-  }
-  if (kind == kDgemmPipe) {
-    if (akc && bkc) hipLaunchKernelGGL((gemm_d_pipe_group_kernel<true, true>), dim3(wg), dim3(256), 0, s, g);
-    else if (akc) hipLaunchKernelGGL((gemm_d_pipe_group_kernel<true, false>), dim3(wg), dim3(256), 0, s, g);
-    else if (bkc) hipLaunchKernelGGL((gemm_d_pipe_group_kernel<false, true>), dim3(wg), dim3(256), 0, s, g);
-    else hipLaunchKernelGGL((gemm_d_pipe_group_kernel<false, false>), dim3(wg), dim3(256), 0, s, g);
-    return hipGetLastError();
-  }
-  if (akc && bkc) hipLaunchKernelGGL((gemm_d_dlds_group_kernel<true, true, 3, 3>), dim3(wg), dim3(256), 0, s, g);
-  else if (akc) hipLaunchKernelGGL((gemm_d_dlds_group_kernel<true, false, 3, 3>), dim3(wg), dim3(256), 0, s, g);
-  else if (bkc) hipLaunchKernelGGL((gemm_d_dlds_group_kernel<false, true, 3, 3>), dim3(wg), dim3(256), 0, s, g);
-  else hipLaunchKernelGGL((gemm_d_dlds_group_kernel<false, false, 3, 3>), dim3(wg), dim3(256), 0, s, g);
-  return hipGetLastError();
-}
-
-hipError_t launch_gemm_s_group(const GemmParams<float>* tiles, int count, hipStream_t s) {
-  SgemmGroup g;
-  int wg = 0;
-  if (count <= 0) return hipSuccess;
-  long t128 = 0;
-  for (int t = 0; t < count; ++t) t128 += dgemm_tiles(tiles[t].m, tiles[t].n, 128);
-  const bool pipe = sgemm_pipe(t128);
-  if (!make_group(tiles, count, pipe ? 128 : 256, pipe ? 128 : 256, sgemm_groupable, g, wg))
-    return hipErrorInvalidValue;
-  const bool akc = is_kc_a(g.base.opa), bkc = is_kc_b(g.base.opb);
-  if (pipe) {
-    if (akc && bkc) hipLaunchKernelGGL((gemm_s_pipe_group_kernel<true, true>), dim3(wg), dim3(256), 0, s, g);
-    else if (akc) hipLaunchKernelGGL((gemm_s_pipe_group_kernel<true, false>), dim3(wg), dim3(256), 0, s, g);
-    else if (bkc) hipLaunchKernelGGL((gemm_s_pipe_group_kernel<false, true>), dim3(wg), dim3(256), 0, s, g);
-    else hipLaunchKernelGGL((gemm_s_pipe_group_kernel<false, false>), dim3(wg), dim3(256), 0, s, g);
-    return hipGetLastError();
-  }
-  if (akc && bkc) hipLaunchKernelGGL((gemm_s_dlds_group_kernel<true, true, 3, 1>), dim3(wg), dim3(512), 0, s, g);
-  else if (akc) hipLaunchKernelGGL((gemm_s_dlds_group_kernel<true, false, 3, 1>), dim3(wg), dim3(512), 0, s, g);
-  else if (bkc) hipLaunchKernelGGL((gemm_s_dlds_group_kernel<false, true, 3, 1>), dim3(wg), dim3(512), 0, s, g);
-  else hipLaunchKernelGGL((gemm_s_dlds_group_kernel<false, false, 3, 1>), dim3(wg), dim3(512), 0, s, g);
-  return hipGetLastError();
-}
-
-template <bool AK, bool BK, bool CA, bool CB>
-void launch_cg(bool pipe, int wg, hipStream_t s, const SgemmGroup& g) {
-  if (pipe) hipLaunchKernelGGL((gemm_c_pipe_group_kernel<AK, BK, CA, CB>), dim3(wg), dim3(256), 0, s, g);
-  else hipLaunchKernelGGL((gemm_c_dlds_group_kernel<AK, BK, CA, CB, 3, 2>), dim3(wg), dim3(256), 0, s, g);
-}
-template <bool AK, bool BK, bool CA, bool CB>
-void launch_c1(bool pipe, dim3 grid, hipStream_t s, const GemmParams<float>& q) {
-  if (pipe) hipLaunchKernelGGL((gemm_c_pipe_kernel<AK, BK, CA, CB>), grid, dim3(256), 0, s, q);
-  else hipLaunchKernelGGL((gemm_c_dlds_kernel<AK, BK, CA, CB, 3, 2>), grid, dim3(256), 0, s, q);
-}
-
-hipError_t launch_gemm_c_group(const GemmParams<float>* tiles, int count, hipStream_t s) {
-  SgemmGroup g;
-  int wg = 0;
-  if (count <= 0) return hipSuccess;
-  if (!make_group(tiles, count, 128, 128, cgemm_groupable, g, wg)) return hipErrorInvalidValue;
-  const bool akc = is_kc_a(g.base.opa), bkc = is_kc_b(g.base.opb);
-  const bool ca = g.base.opa == 'C', cb = g.base.opb == 'C';
-  // the pipelined tile when the group has two tiles per CU to fill it
-  const bool pipe = sgemm_pipe(wg);
-#define TMM_CG(AK, BK, CA, CB) launch_cg<AK, BK, CA, CB>(pipe, wg, s, g)
-  if (akc && bkc) {
-    if (ca) TMM_CG(true, true, true, false);
-    else TMM_CG(true, true, false, false);
-  } else if (akc) {
-    if (ca && cb) TMM_CG(true, false, true, true);
-    else if (ca) TMM_CG(true, false, true, false);
-    else if (cb) TMM_CG(true, false, false, true);
-    else TMM_CG(true, false, false, false);
-  } else if (bkc) {
-    TMM_CG(false, true, false, false);
-  } else {
-    if (cb) TMM_CG(false, false, false, true);
-    else TMM_CG(false, false, false, false);
-  }
-#undef TMM_CG
-  return hipGetLastError();
-}
+hipError_t launch_gemm_d(const GemmParams<double>& p, hipStream_t s) { return launch_one(kD, p, s); }
+hipError_t launch_gemm_s(const GemmParams<float>& p, hipStream_t s) { return launch_one(kS, p, s); }
+hipError_t launch_gemm_z(const GemmParams<double>& p, hipStream_t s) { return launch_one(kZ, p, s); }
+hipError_t launch_gemm_c(const GemmParams<float>& p, hipStream_t s) { return launch_one(kC, p, s); }
+hipError_t launch_gemm_d_group(const GemmParams<double>* tiles, int count, hipStream_t s) { return launch_many(kD, tiles, count, s); }
+hipError_t launch_gemm_s_group(const GemmParams<float>* tiles, int count, hipStream_t s) { return launch_many(kS, tiles, count, s); }
+hipError_t launch_gemm_z_group(const GemmParams<double>* tiles, int count, hipStream_t s) { return launch_many(kZ, tiles, count, s); }
+hipError_t launch_gemm_c_group(const GemmParams<float>* tiles, int count, hipStream_t s) { return launch_many(kC, tiles, count, s); }
 
 hipError_t launch_gemm_d_batched(char opa, char opb, const GemmParams<double>* probs, const int* items, int n_items,
                                  int* counter, int n_workgroups, hipStream_t s, int body) {
@@ -2524,158 +2068,6 @@ hipError_t launch_gemm_d_batched(char opa, char opb, const GemmParams<double>* p
   else if (bkc) hipLaunchKernelGGL((gemm_real_batched_kernel<double, false, true>), grid, block, 0, s, probs, items, n_items, counter);
   else hipLaunchKernelGGL((gemm_real_batched_kernel<double, false, false>), grid, block, 0, s, probs, items, n_items, counter);
   return hipGetLastError();
-}
-
-hipError_t launch_gemm_d(const GemmParams<double>& p, hipStream_t s) {
-  if (p.m <= 0 || p.n <= 0) return hipSuccess;
-  if (p.variant == 1) return launch_gemm_d_direct(p, s);
-  return launch_real<double>(p, s);
-}
-// FP32 through the direct-LDS kernels. The pipelined one takes any k and any row count (but not a
-// row-contiguous operand whose 4-row chunks could reach over more than one column end); the others
-// the largest multiple of 16 in K, a remainder going to gemm_real_kernel, accumulating (beta only
-// on the first part).
-hipError_t launch_gemm_s_direct(const GemmParams<float>& p, hipStream_t s) {
-  const bool akc = is_kc_a(p.opa), bkc = is_kc_b(p.opb);
-  const bool chunks_ok = (akc || p.m % 4 == 0 || p.lda >= 3) && (bkc || p.n % 4 == 0 || p.ldb >= 3);
-  const bool pipe = p.k > 0 && sgemm_pipe(p.m, p.n) && chunks_ok;
-  const int k16 = pipe ? p.k : p.k / 16 * 16;
-  // the other kernels need whole 4-row chunks of a row-contiguous operand
-  const bool rows_ok = (akc || p.m % 4 == 0) && (bkc || p.n % 4 == 0);
-  if (!pipe && (k16 == 0 || !rows_ok)) return launch_real<float>(p, s);
-  GemmParams<float> q = p;
-  q.k = k16;
-  // 256 x 256 workgroup tiles (8 waves of 64 x 128, one workgroup per CU) once m and n allow:
-  // SGEMM TN 16384^3 142.3, 40000^3 140.0, 8064^2 x 8000 134.0 TFLOP/s against 135.8, 134.5, 127.8
-  // for 256 x 128 tiles (8 waves of 64 x 64, two per CU; 32 against 48 bytes of LDS writes per
-  // MFMA); 256 x 128 in turn ran NN 138.2 and TN 135.1 against 134.8 and 134.3 for 128 x 128 tiles
-  // at three per CU
-  if (pipe) {
-    const dim3 grid(dgemm_tiles(p.m, p.n, 128)), block(256);
-    if (akc && bkc) hipLaunchKernelGGL((gemm_s_pipe_kernel<true, true>), grid, block, 0, s, q);
-    else if (akc) hipLaunchKernelGGL((gemm_s_pipe_kernel<true, false>), grid, block, 0, s, q);
-    else if (bkc) hipLaunchKernelGGL((gemm_s_pipe_kernel<false, true>), grid, block, 0, s, q);
-    else hipLaunchKernelGGL((gemm_s_pipe_kernel<false, false>), grid, block, 0, s, q);
-  } else if (p.m > 128 && p.n > 128) {
-    const dim3 grid(((p.m + 255) / 256) * ((p.n + 255) / 256)), block(512);
-    if (akc && bkc) hipLaunchKernelGGL((gemm_s_dlds_kernel<true, true, 3, 1, 256, 256>), grid, block, 0, s, q);
-    else if (akc) hipLaunchKernelGGL((gemm_s_dlds_kernel<true, false, 3, 1, 256, 256>), grid, block, 0, s, q);
-    else if (bkc) hipLaunchKernelGGL((gemm_s_dlds_kernel<false, true, 3, 1, 256, 256>), grid, block, 0, s, q);
-    else hipLaunchKernelGGL((gemm_s_dlds_kernel<false, false, 3, 1, 256, 256>), grid, block, 0, s, q);
-  } else if (p.m > 128) {
-    const dim3 grid(((p.m + 255) / 256) * ((p.n + 127) / 128)), block(512);
-    if (akc && bkc) hipLaunchKernelGGL((gemm_s_dlds_kernel<true, true, 3, 2, 256>), grid, block, 0, s, q);
-    else if (akc) hipLaunchKernelGGL((gemm_s_dlds_kernel<true, false, 3, 2, 256>), grid, block, 0, s, q);
-    else if (bkc) hipLaunchKernelGGL((gemm_s_dlds_kernel<false, true, 3, 2, 256>), grid, block, 0, s, q);
-    else hipLaunchKernelGGL((gemm_s_dlds_kernel<false, false, 3, 2, 256>), grid, block, 0, s, q);
-  } else {
-    const dim3 grid((p.n + 127) / 128), block(256);
-    if (akc && bkc) hipLaunchKernelGGL((gemm_s_dlds_kernel<true, true, 3, 3, 128>), grid, block, 0, s, q);
-    else if (akc) hipLaunchKernelGGL((gemm_s_dlds_kernel<true, false, 3, 3, 128>), grid, block, 0, s, q);
-    else if (bkc) hipLaunchKernelGGL((gemm_s_dlds_kernel<false, true, 3, 3, 128>), grid, block, 0, s, q);
-    else hipLaunchKernelGGL((gemm_s_dlds_kernel<false, false, 3, 3, 128>), grid, block, 0, s, q);
-  }
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess || k16 == p.k) return e;
-  GemmParams<float> r = p;
-  r.k = p.k - k16;
-  r.a = p.a + (akc ? (long)k16 : (long)k16 * p.lda);
-  r.b = p.b + (bkc ? (long)k16 : (long)k16 * p.ldb);
-  r.accumulate = 1;
-  r.beta = 0.0f;
-  return launch_real<float>(r, s);
-}
-
-hipError_t launch_gemm_s(const GemmParams<float>& p, hipStream_t s) {
-  if (p.m <= 0 || p.n <= 0) return hipSuccess;
-  if (p.variant == 1) return launch_gemm_s_direct(p, s);
-  return launch_real<float>(p, s);
-}
-hipError_t launch_gemm_z(const GemmParams<double>& p, hipStream_t s) {
-  if (p.m <= 0 || p.n <= 0) return hipSuccess;
-  if (p.variant == 0) return launch_cplx<double>(p, s);
-  const dim3 grid(((p.m + 63) / 64) * ((p.n + 63) / 64)), block(256);
-  const bool pipe = p.k > 0 && (long)grid.x >= 2L * device_cus();  // as for the groups
-  // the pipelined kernel takes any k; the other one the largest multiple of 8 in K, the remainder
-  // going through gemm_cplx_kernel, accumulating (beta only on the first part)
-  const int k8 = pipe ? p.k : p.k / 8 * 8;
-  if (k8 == 0) return launch_cplx<double>(p, s);
-  const bool akc = is_kc_a(p.opa), bkc = is_kc_b(p.opb);
-  GemmParams<double> q = p;
-  q.k = k8;
-  const bool ca = p.opa == 'C', cb = p.opb == 'C';
-  // 3-stage ring, 3 workgroups per CU: 69.7 TFLOP/s on CN 8192^3 against 67.9 for 4 stages at 2
-#define TMM_ZDLDS(AK, BK, CA, CB)                                                              \
-  do {                                                                                         \
-    if (pipe) hipLaunchKernelGGL((gemm_z_pipe_kernel<AK, BK, CA, CB>), grid, block, 0, s, q);  \
-    else hipLaunchKernelGGL((gemm_z_dlds_kernel<AK, BK, CA, CB, 3, 3>), grid, block, 0, s, q); \
-  } while (0)
-  if (akc && bkc) {
-    if (ca) TMM_ZDLDS(true, true, true, false);
-    else TMM_ZDLDS(true, true, false, false);
-  } else if (akc) {
-    if (ca && cb) TMM_ZDLDS(true, false, true, true);
-    else if (ca) TMM_ZDLDS(true, false, true, false);
-    else if (cb) TMM_ZDLDS(true, false, false, true);
-    else TMM_ZDLDS(true, false, false, false);
-  } else if (bkc) {
-    TMM_ZDLDS(false, true, false, false);
-  } else {
-    if (cb) TMM_ZDLDS(false, false, false, true);
-    else TMM_ZDLDS(false, false, false, false);
-  }
-#undef TMM_ZDLDS
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess || k8 == p.k) return e;
-  GemmParams<double> r = p;
-  r.k = p.k - k8;
-  r.a = p.a + 2 * (akc ? (long)k8 : (long)k8 * p.lda);
-  r.b = p.b + 2 * (bkc ? (long)k8 : (long)k8 * p.ldb);
-  r.accumulate = 1;
-  r.beta = 0.0;
-  r.beta_im = 0.0;
-  return launch_cplx<double>(r, s);
-}
-hipError_t launch_gemm_c(const GemmParams<float>& p, hipStream_t s) {
-  if (p.m <= 0 || p.n <= 0) return hipSuccess;
-  const bool akc = is_kc_a(p.opa), bkc = is_kc_b(p.opb);
-  const dim3 grid(((p.m + 127) / 128) * ((p.n + 127) / 128));
-  const bool pipe = p.k > 0 && sgemm_pipe((long)grid.x);  // as for the groups
-  // the pipelined kernel takes any k and any row count; the other one the largest multiple of 8 in
-  // K, the remainder going through gemm_cplx_kernel, accumulating (beta only on the first part),
-  // and whole 2-row chunks of a row-contiguous operand
-  const int k8 = pipe ? p.k : p.k / 8 * 8;
-  const bool rows_ok = pipe || ((akc || p.m % 2 == 0) && (bkc || p.n % 2 == 0));
-  if (p.variant != 1 || k8 == 0 || !rows_ok) return launch_cplx<float>(p, s);
-  GemmParams<float> q = p;
-  q.k = k8;
-  const bool ca = p.opa == 'C', cb = p.opb == 'C';
-#define TMM_CDLDS(AK, BK, CA, CB) launch_c1<AK, BK, CA, CB>(pipe, grid, s, q)
-  if (akc && bkc) {
-    if (ca) TMM_CDLDS(true, true, true, false);
-    else TMM_CDLDS(true, true, false, false);
-  } else if (akc) {
-    if (ca && cb) TMM_CDLDS(true, false, true, true);
-    else if (ca) TMM_CDLDS(true, false, true, false);
-    else if (cb) TMM_CDLDS(true, false, false, true);
-    else TMM_CDLDS(true, false, false, false);
-  } else if (bkc) {
-    TMM_CDLDS(false, true, false, false);
-  } else {
-    if (cb) TMM_CDLDS(false, false, false, true);
-    else TMM_CDLDS(false, false, false, false);
-  }
-#undef TMM_CDLDS
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess || k8 == p.k) return e;
-  GemmParams<float> r = p;
-  r.k = p.k - k8;
-  r.a = p.a + 2 * (akc ? (long)k8 : (long)k8 * p.lda);
-  r.b = p.b + 2 * (bkc ? (long)k8 : (long)k8 * p.ldb);
-  r.accumulate = 1;
-  r.beta = 0.0f;
-  r.beta_im = 0.0f;
-  return launch_cplx<float>(r, s);
 }
 
 }  // namespace tmm

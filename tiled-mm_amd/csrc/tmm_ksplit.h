@@ -1,1 +1,119 @@
+// Tile kernels with the inner dimension split over a workgroup's waves: launch interface, and the
+// choice between their tile shapes and the 128 x 128 (complex double: 64 x 64) pipelined kernels.
 #pragma once
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+
+#include "tmm_kernels.h"
+
+namespace tmm {
+
+// Element types as the tables below order them.
+enum class KsType { D = 0, S = 1, Z = 2, C = 3 };
+
+// Tile shapes in blocks of 16 rows and columns, and the ring stages of each. Two stages where that
+// lets more workgroups share a CU (a third one ran 2-4% slower at 2048^3); the smallest shapes have
+// so little work per stage that they take four. Complex double stops at 3 x 3 and complex float
+// at 3 x 4: larger tiles exceed the 256 registers of two waves per SIMD.
+#define TMM_KS_SHAPES_SMALL(X, S23) \
+  X(1, 1, 4) X(1, 2, 4) X(2, 1, 4) X(2, 2, 2) X(2, 3, S23) X(3, 2, S23) X(3, 3, 2)
+#define TMM_KS_SHAPES_MIDDLE(X) X(2, 4, 2) X(4, 2, 2) X(3, 4, 2) X(4, 3, 2)
+#define TMM_KS_SHAPES_LARGE(X) X(4, 4, 2)
+
+struct KsShape {
+  int m, n;
+};
+#define TMM_KS_ENTRY(a, b, s) {a, b},
+constexpr KsShape kKsShapes[] = {TMM_KS_SHAPES_SMALL(TMM_KS_ENTRY, 3) TMM_KS_SHAPES_MIDDLE(TMM_KS_ENTRY)
+                                     TMM_KS_SHAPES_LARGE(TMM_KS_ENTRY)};
+#undef TMM_KS_ENTRY
+constexpr int kKsShapeCount[4] = {12, 12, 7, 11};  // shapes of each element type, a prefix of kKsShapes
+
+struct KsCost {  // a type's costs; cycles of a 2.4 GHz clock
+  int bk;        // inner dimension of a stage
+  int block;     // a wave's MFMA cycles per stage and 16 x 16 block
+  int stage;     // what a stage costs beside its MFMAs
+  int pipe;      // the same of a k-step of the pipelined kernel
+  int pipe_bk;   // inner dimension of that k-step (16 blocks per wave; complex double: 8 of half the size)
+  double tile;   // us per block of a tile's prologue and epilogue
+};
+// Fitted to the times of every shape at about 20 sizes from 17 x 33 x 5 to 6222 x 6255 x 3501 (the
+// choice they lead to is within 3% of the fastest shape at each of them).
+constexpr KsCost kKsCost[4] = {{8, 128, 170, 150, 8, 0.28},
+                               {16, 128, 280, 290, 16, 0.26},
+                               {4, 256, 170, 250, 8, 0.78},
+                               {8, 256, 300, 385, 8, 0.33}};
+
+// Time in us of a product of (together) `tiles` tiles of shape s and inner dimension k on `cus`
+// compute units: whole tiles per CU, four waves sharing a tile's stages.
+inline double ks_time(KsType t, KsShape s, long tiles, long k, int cus) {
+  const KsCost& c = kKsCost[(int)t];
+  const int blocks = s.m * s.n;
+  // a stage cannot run faster than the L2 delivers it (about 24 bytes per cycle and CU), which
+  // binds for the smallest tiles; 12 complex float blocks leave fewer registers to overlap with
+  const double extra = t == KsType::C && blocks == 12 ? 240 : 0;
+  double per = std::max(blocks * c.block + c.stage + extra, (s.m + s.n) * 4096 / 24.0);
+  // With many tiles per CU and a long inner dimension the workgroups of an XCD drift apart in k and
+  // share less in its L2: at four or more tiles per CU the real types lose up to 8% from 24 KB to
+  // 64 KB of inner dimension (FP64 TN 5000^3 3.74 ms against 3.61 without the loss, 6000 x 6000 x
+  // 8000 8.73 against 8.09).
+  if (t <= KsType::S && tiles > 4L * cus) {
+    const double kb = k * (t == KsType::D ? 8.0 : 4.0);
+    per *= 1 + 0.08 * std::min(1.0, std::max(0.0, (kb - 24000) / 40000));
+  }
+  return 2.3 + c.tile * blocks + (double)((tiles + cus - 1) / cus) * ((double)k / c.bk / 4) * per / 2400;
+}
+// The same for `tiles` workgroup tiles of the pipelined kernel.
+inline double pipe_time(KsType t, long tiles, long k, int cus) {
+  const KsCost& c = kKsCost[(int)t];
+  const int step = t == KsType::Z ? 8 * c.block : 16 * c.block;  // a wave's MFMA cycles per k-step
+  return 2.3 + 4 * c.tile + (double)((tiles + cus - 1) / cus) * ((double)k / c.pipe_bk) * (step + c.pipe) / 2400;
+}
+
+inline long ks_tiles(KsShape s, long m, long n) { return ((m + 16 * s.m - 1) / (16 * s.m)) * ((n + 16 * s.n - 1) / (16 * s.n)); }
+
+// Fastest shape for an m x n x k product, and its time in us.
+inline int ks_shape(KsType t, long m, long n, long k, int cus, double* us) {
+  int best = 0;
+  double least = 0;
+  for (int i = 0; i < kKsShapeCount[(int)t]; ++i) {
+    const double x = ks_time(t, kKsShapes[i], ks_tiles(kKsShapes[i], m, n), k, cus);
+    if (i == 0 || x < least) {
+      least = x;
+      best = i;
+    }
+  }
+  *us = least;
+  return best;
+}
+
+// Whether an operand's 16-byte row chunks reach over the end of at most one column (a chunk of 4
+// floats over the end of a column, or of two complex floats, of a leading dimension below its size).
+template <typename R>
+bool ks_chunks_ok(bool cplx, bool kc, long rows, long ld) {
+  const long chunk = 16 / ((long)sizeof(R) * (cplx ? 2 : 1));
+  return kc || rows % chunk == 0 || ld >= chunk - 1;
+}
+// Whether the kernels take the product: a lane's byte offsets inside a load (up to 15 rows or
+// columns) are 32 bits wide.
+template <typename R>
+bool ks_takes(const GemmParams<R>& p, bool cplx) {
+  const long es = (long)sizeof(R) * (cplx ? 2 : 1);
+  return p.variant == 1 && p.k > 0 && p.lda * es <= (1L << 28) && p.ldb * es <= (1L << 28) &&
+         ks_chunks_ok<R>(cplx, p.opa != 'N', p.m, p.lda) && ks_chunks_ok<R>(cplx, p.opb == 'N', p.n, p.ldb);
+}
+
+// One product on the given shape (an index of kKsShapes), or a group of products with one op pair,
+// alpha and k in one launch; every product must satisfy ks_takes. The result does not depend on
+// the shape, nor on the grouping.
+#define TMM_KS_DECLARE(t, R)                                                   \
+  hipError_t launch_ks_##t(const GemmParams<R>& p, int shape, hipStream_t s); \
+  hipError_t launch_ks_##t##_group(const GemmParams<R>* tiles, int count, hipStream_t s);
+TMM_KS_DECLARE(d, double)
+TMM_KS_DECLARE(s, float)
+TMM_KS_DECLARE(z, double)
+TMM_KS_DECLARE(c, float)
+#undef TMM_KS_DECLARE
+
+}  // namespace tmm

@@ -1,0 +1,20 @@
+// Complex float instances of the kernels that split the inner dimension over a workgroup's waves.
+#include "tmm_ksplit_kernel.h"
+
+namespace tmm {
+
+hipError_t launch_ks_c(const GemmParams<float>& p, int shape, hipStream_t s) {
+  int i = 0;
+#define TMM_KS_CASE(a, b, st) \
+  if (shape == i++) return ks::launch_shape<ks::TypeC, a, b, st>(p, s);
+  TMM_KS_SHAPES_SMALL(TMM_KS_CASE, 2)
+  TMM_KS_SHAPES_MIDDLE(TMM_KS_CASE)
+#undef TMM_KS_CASE
+  return hipErrorInvalidValue;
+}
+
+hipError_t launch_ks_c_group(const GemmParams<float>* tiles, int count, hipStream_t s) {
+  return ks::launch_group<ks::TypeC, 3, 3, 2>(tiles, count, s);
+}
+
+}  // namespace tmm

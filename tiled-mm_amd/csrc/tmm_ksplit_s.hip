@@ -1,0 +1,21 @@
+// Float instances of the kernels that split the inner dimension over a workgroup's waves.
+#include "tmm_ksplit_kernel.h"
+
+namespace tmm {
+
+hipError_t launch_ks_s(const GemmParams<float>& p, int shape, hipStream_t s) {
+  int i = 0;
+#define TMM_KS_CASE(a, b, st) \
+  if (shape == i++) return ks::launch_shape<ks::TypeS, a, b, st>(p, s);
+  TMM_KS_SHAPES_SMALL(TMM_KS_CASE, 3)
+  TMM_KS_SHAPES_MIDDLE(TMM_KS_CASE)
+  TMM_KS_SHAPES_LARGE(TMM_KS_CASE)
+#undef TMM_KS_CASE
+  return hipErrorInvalidValue;
+}
+
+hipError_t launch_ks_s_group(const GemmParams<float>* tiles, int count, hipStream_t s) {
+  return ks::launch_group<ks::TypeS, 4, 4, 2>(tiles, count, s);
+}
+
+}  // namespace tmm
