@@ -29,7 +29,7 @@ struct OzakiGemmParams {
   double* c;
   long ldc;
   // when fa is set, the launch does nothing if *fa | *fb is non-zero (the operands' fallback
-  // flags, see ozaki_exponents)
+  // flags: an entry is non-finite or at least 2^kFallbackExp in magnitude)
   const int* fa;
   const int* fb;
 };
@@ -40,9 +40,6 @@ struct OzakiGemmParams {
 // every product and sum of the emulation stays far from the FP64 range (2^(2*480+17) < 2^1023).
 constexpr int kFallbackExp = 480;
 
-// e[r] (r < rows): exponent with max_k |x(r, k)| < 2^e[r]; *flag (when not null) becomes 1 if an
-// entry is non-finite or at least 2^kFallbackExp in magnitude, else 0.
-hipError_t ozaki_exponents(const double* p, long ld, bool kc, int rows, int k, int* e, int* flag, hipStream_t s);
 hipError_t ozaki_split(const double* p, long ld, bool kc, int rows, int k, const int* e, int nslices, int rows_pad,
                        int kpad, int8_t* out, hipStream_t s);
 hipError_t ozaki_gemm(const OzakiGemmParams& p, hipStream_t s);

@@ -40,50 +40,77 @@ __device__ __forceinline__ int frexp_exp_of(double v) {
   return be == 0 ? -1022 : be - 1022;
 }
 
-// p mod m for p < 2^32 and 2 <= m <= 256, magic = ceil(2^32 / m): the estimate q = p*magic/2^32
-// is floor(p/m) or one more, so a single correction gives the remainder.
-__device__ __forceinline__ unsigned mod_small(unsigned p, unsigned m, unsigned magic) {
-  const unsigned q = __umulhi(p, magic);
-  const int r = (int)(p - q * m);
-  return (unsigned)(r < 0 ? r + (int)m : r);
-}
-
 // ---------------------------------------------------------------------------------------------
 // Exponents: e[r] = max over k of frexp-exponent(|x(r, k)|). x(r, k) at p[k + r*ld] (KC) or
-// p[r + k*ld] (RC). Grid: (row blocks, k splits); partial maxima meet in atomicMax. Inf and NaN
-// have frexp-exponent 1025 here, so a partial maximum above kFallbackExp marks the operand for
-// the native fallback (*flag = 1; every writer stores the same value).
+// p[r + k*ld] (RC). A workgroup of 1024 threads takes a few rows over the whole inner dimension, so
+// every e[r] has one writer: no initialising launch and no atomics. Many loads of a thread are in
+// flight together (8 per batch). Bound by memory: two operands of 4096 x 4096 65 us (4.1 TB/s), of
+// 2048 x 2048 14 us; with atomics, one load at a time and 64 workgroups, one row-contiguous operand
+// of 2048 x 2048 took 108 us.
 // ---------------------------------------------------------------------------------------------
-__global__ void exp_init_kernel(int* e, int rows, int* flag) {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r < rows) e[r] = kExpNone;
-  if (flag && r == 0) *flag = 0;
-}
+struct OperandSrc {
+  const double* p;
+  long ld;
+  int kc, rows, k;
+  int* e;     // rows exponents
+  int* flag;  // behind them: non-zero if an entry is non-finite or at least 2^kFallbackExp
+};
 
-__global__ __launch_bounds__(256) void exp_rows_rc_kernel(const double* __restrict__ p, long ld, int rows, int k,
-                                                          int kper, int* __restrict__ e, int* __restrict__ flag) {
-  const int r = blockIdx.x * 256 + threadIdx.x;
-  if (r >= rows) return;
-  const int k0 = blockIdx.y * kper, k1 = min(k, k0 + kper);
-  int m = kExpNone;
-  for (int kk = k0; kk < k1; ++kk) m = max(m, frexp_exp_of(p[(long)r + (long)kk * ld]));
-  if (m != kExpNone) atomicMax(&e[r], m);
-  if (m > kFallbackExp && flag) *flag = 1;
-}
+// 16 rows per workgroup, 128 contiguous bytes of a row-contiguous operand (4, to spread few rows over
+// more CUs, ran slower: 500 x 40000 twice, 171 us against 140).
+constexpr int kExpRows = 16;
 
-__global__ __launch_bounds__(256) void exp_rows_kc_kernel(const double* __restrict__ p, long ld, int rows, int k,
-                                                          int kper, int* __restrict__ e, int* __restrict__ flag) {
-  // one wave per (row, k range)
-  const int wave = (blockIdx.x * 256 + threadIdx.x) >> 6, lane = threadIdx.x & 63;
-  if (wave >= rows) return;
-  const int k0 = blockIdx.y * kper, k1 = min(k, k0 + kper);
+__device__ __forceinline__ void exponents16(const OperandSrc& o, int block, int* lds) {
+  const int r0 = block * kExpRows, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   int m = kExpNone;
-  const double* row = p + (long)wave * ld;
-  for (int kk = k0 + lane; kk < k1; kk += 64) m = max(m, frexp_exp_of(row[kk]));
+  if (o.kc) {  // a wave per row
+    const int r = r0 + wave;
+    if (r < o.rows) {
+      const double* row = o.p + (long)r * o.ld;
+#pragma unroll 8
+      for (int kk = lane; kk < o.k; kk += 64) m = max(m, frexp_exp_of(row[kk]));
+    }
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) m = max(m, __shfl_xor(m, off));
-  if (lane == 0 && m != kExpNone) atomicMax(&e[wave], m);
-  if (lane == 0 && m > kFallbackExp && flag) *flag = 1;
+    for (int off = 32; off > 0; off >>= 1) m = max(m, __shfl_xor(m, off));
+    if (lane == 0 && r < o.rows) o.e[r] = m;
+    return;
+  }
+  const int r = r0 + (lane & 15);  // 16 rows of 4 k per wave and load
+  if (r < o.rows) {
+    const double* q = o.p + r;
+#pragma unroll 8
+    for (int kk = threadIdx.x >> 4; kk < o.k; kk += 64) m = max(m, frexp_exp_of(q[(long)kk * o.ld]));
+  }
+  m = max(m, __shfl_xor(m, 16));
+  m = max(m, __shfl_xor(m, 32));
+  if (lane < 16) lds[wave * 16 + lane] = m;
+  __syncthreads();
+  if (threadIdx.x < 16 && r < o.rows) {
+    for (int w = 1; w < 16; ++w) m = max(m, lds[w * 16 + lane]);
+    o.e[r] = m;
+  }
+}
+
+// Exponents of two operands, the second's workgroups behind the first's.
+__global__ __launch_bounds__(1024) void exponents_kernel(OperandSrc a, OperandSrc b) {
+  __shared__ int lds[256];
+  const int na = (a.rows + kExpRows - 1) / kExpRows;
+  if ((int)blockIdx.x < na) exponents16(a, blockIdx.x, lds);
+  else exponents16(b, blockIdx.x - na, lds);
+}
+
+// *flag from the operand's exponents, by one workgroup. Inf and NaN have frexp-exponent 1025, so an
+// exponent above kFallbackExp marks the operand for the native fallback.
+__device__ __forceinline__ void operand_flag(const OperandSrc& o) {
+  int big = 0;
+  for (int r = threadIdx.x; r < o.rows; r += blockDim.x) big |= o.e[r] > kFallbackExp;
+  big = __syncthreads_or(big);
+  if (threadIdx.x == 0) *o.flag = big ? 1 : 0;
+}
+
+__global__ __launch_bounds__(1024) void operand_flag_kernel(OperandSrc a, OperandSrc b) {
+  if (blockIdx.x == 0) operand_flag(a);
+  else operand_flag(b);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -153,7 +180,7 @@ __global__ __launch_bounds__(256) void split_kernel(const double* __restrict__ p
 // layout: one contiguous 16 KB block per 256 rows and 64 k, blocks of a row block in k order, 64-byte
 // rows inside) into res + q*plane (uint8 in [0, modulus) at i + j*ldres; ldres a multiple of 16,
 // rows m..ldres-1 receive padding). The launch does nothing if *fa | *fb is non-zero (the operands'
-// fallback flags, see ozaki_exponents).
+// fallback flags, an entry is non-finite or at least 2^kFallbackExp in magnitude).
 struct CrtProductParams {
   int m, n, kpad, nmod;
   const int8_t* a;
@@ -474,21 +501,16 @@ void* ozaki_scratch(int device) {
   return g_scratch_ptr[device];
 }
 
-hipError_t ozaki_exponents(const double* p, long ld, bool kc, int rows, int k, int* e, int* flag, hipStream_t s) {
-  if (rows <= 0) return hipSuccess;
-  hipLaunchKernelGGL(exp_init_kernel, dim3((rows + 255) / 256), dim3(256), 0, s, e, rows, flag);
-  if (k <= 0) return hipGetLastError();
-  if (kc) {
-    const int ksplit = k >= 8192 ? 8 : 1, kper = (k + ksplit - 1) / ksplit;
-    hipLaunchKernelGGL(exp_rows_kc_kernel, dim3((rows + 3) / 4, ksplit), dim3(256), 0, s, p, ld, rows, k, kper, e,
-                       flag);
-  } else {
-    const int ksplit = std::min(64, std::max(1, k / 256)), kper = (k + ksplit - 1) / ksplit;
-    hipLaunchKernelGGL(exp_rows_rc_kernel, dim3((rows + 255) / 256, ksplit), dim3(256), 0, s, p, ld, rows, k, kper, e,
-                       flag);
-  }
+namespace {
+// Exponents of `count` (1 or 2) operands, in one launch.
+hipError_t launch_exponents(const OperandSrc* o, int count, hipStream_t s) {
+  OperandSrc none{};
+  const OperandSrc& b = count > 1 ? o[1] : none;
+  const int blocks = (o[0].rows + kExpRows - 1) / kExpRows + (b.rows + kExpRows - 1) / kExpRows;
+  if (blocks > 0) hipLaunchKernelGGL(exponents_kernel, dim3(blocks), dim3(1024), 0, s, o[0], b);
   return hipGetLastError();
 }
+}  // namespace
 
 hipError_t ozaki_split(const double* p, long ld, bool kc, int rows, int k, const int* e, int nslices, int rows_pad,
                        int kpad, int8_t* out, hipStream_t s) {
@@ -572,8 +594,9 @@ hipError_t ozaki_dgemm(char opa, char opb, int m, int n, int k, double alpha, co
   // op(A) rows: k-contiguous when A is transposed; op(B) columns: k-contiguous when B is not.
   const bool a_kc = opa != 'N', b_kc = opb == 'N';
   hipError_t e;
-  if ((e = ozaki_exponents(a, lda, a_kc, m, k, ea, fa, s)) != hipSuccess) return e;
-  if ((e = ozaki_exponents(b, ldb, b_kc, n, k, eb, fb, s)) != hipSuccess) return e;
+  const OperandSrc src[2] = {{a, lda, a_kc, m, k, ea, fa}, {b, ldb, b_kc, n, k, eb, fb}};
+  if ((e = launch_exponents(src, 2, s)) != hipSuccess) return e;
+  hipLaunchKernelGGL(operand_flag_kernel, dim3(2), dim3(1024), 0, s, src[0], src[1]);
   if ((e = ozaki_split(a, lda, a_kc, m, k, ea, nslices, (int)mpad, (int)kpad, sa, s)) != hipSuccess) return e;
   if ((e = ozaki_split(b, ldb, b_kc, n, k, eb, nslices, (int)npad, (int)kpad, sb, s)) != hipSuccess) return e;
 
@@ -657,25 +680,6 @@ namespace {
 constexpr int kCrtModuli[kCrtMaxModuli] = {256, 255, 253, 251, 247, 241, 239, 233, 229, 227,
                                            223, 211, 199, 197, 193, 191, 181, 179, 173, 167};
 
-struct CrtParams {
-  int n;
-  unsigned m[kCrtMaxModuli];
-  unsigned magic[kCrtMaxModuli];  // ceil(2^32 / m)
-  unsigned c21[kCrtMaxModuli];    // 2^21 mod m
-  unsigned c42[kCrtMaxModuli];    // 2^42 mod m
-};
-
-constexpr long pow_mod(long b, long e, long m) {
-  long r = 1 % m;
-  b %= m;
-  while (e > 0) {
-    if (e & 1) r = r * b % m;
-    b = b * b % m;
-    e >>= 1;
-  }
-  return r;
-}
-
 constexpr long inv_mod(long a, long m) {  // extended Euclid; a and m coprime
   long g = m, x = 0, x1 = 1, a1 = a % m;
   while (a1 != 0) {
@@ -741,46 +745,22 @@ struct CrtSumTable {
   static constexpr CrtSum<N> v = make_crt_sum<N>();
 };
 
-CrtParams make_crt(int n) {
-  CrtParams c{};
+// Constants of the operands' residues, per modulus: 2^30 mod m (balanced), 1 / m, m.
+struct ResidueConsts {
+  int n;
+  double c30[kCrtMaxModuli], inv[kCrtMaxModuli], m[kCrtMaxModuli];
+};
+
+ResidueConsts residue_consts(int n) {
+  ResidueConsts c{};
   c.n = n;
   for (int t = 0; t < n; ++t) {
-    const unsigned m = (unsigned)kCrtModuli[t];
+    const int m = kCrtModuli[t], r = (1 << 30) % m;
+    c.c30[t] = r > m / 2 ? r - m : r;
+    c.inv[t] = 1.0 / m;
     c.m[t] = m;
-    c.magic[t] = (unsigned)((((unsigned long long)1 << 32) + m - 1) / m);
-    c.c21[t] = (unsigned)pow_mod(2, 21, m);
-    c.c42[t] = (unsigned)pow_mod(2, 42, m);
   }
   return c;
-}
-
-// Scaled, rounded entry x = round(|v| 2^(bits - er)) <= 2^62, split exactly into 21-bit digits
-// x = x2 2^42 + x1 2^21 + x0, so that x mod m = (x2 c42 + x1 c21 + x0) mod m with one reduction
-// of a value below 2^30.
-struct Split21 {
-  unsigned x0, x1, x2;
-  bool neg;
-};
-__device__ __forceinline__ Split21 split21(double v, int er, int bits) {
-  Split21 s;
-  s.neg = v < 0.0;
-  const double x = er == kExpNone ? 0.0 : rint(ldexp(fabs(v), bits - er));
-  const double h2 = floor(x * 0x1p-42);
-  const double rem = x - h2 * 0x1p42;
-  const double h1 = floor(rem * 0x1p-21);
-  s.x2 = (unsigned)h2;
-  s.x1 = (unsigned)h1;
-  s.x0 = (unsigned)(rem - h1 * 0x1p21);
-  return s;
-}
-
-// Balanced residue (int8) of a split entry modulo cp.m[q].
-__device__ __forceinline__ uint32_t residue8(const Split21& s, const CrtParams& cp, int q) {
-  const unsigned m = cp.m[q];
-  unsigned r = mod_small(s.x2 * cp.c42[q] + s.x1 * cp.c21[q] + s.x0, m, cp.magic[q]);
-  if (s.neg && r != 0) r = m - r;
-  const int bal = 2 * r >= m ? (int)r - (int)m : (int)r;
-  return (uint32_t)(uint8_t)(int8_t)bal;
 }
 
 // Byte offset of entry (r, k) in a residue plane of rows_pad x kpad in k-step tiled layout: one
@@ -790,62 +770,84 @@ __device__ __forceinline__ long crt_tiled_offset(int r, int k, int kpad) {
   return ((long)(r >> 8) * (kpad >> 6) + (k >> 6)) * 16384 + (r & 255) * 64 + (k & 63);
 }
 
-// Balanced residues of the scaled, rounded entries: one int8 plane per modulus, rows_pad x kpad
-// in k-step tiled layout (zero outside the matrix); k-contiguous source: each thread handles 4
-// consecutive k of one row and writes one 4-byte word (consecutive threads, consecutive words).
-__global__ __launch_bounds__(256) void crt_residue_kc_kernel(const double* __restrict__ p, long ld, int rows, int k,
-                                                             const int* __restrict__ e, int bits, CrtParams cp,
-                                                             int rows_pad, int kpad, int8_t* __restrict__ out) {
-  // thread tid writes bytes 4*tid .. 4*tid+3 of each plane (k-step tiled layout, crt_tiled_offset)
-  const long tid = (long)blockIdx.x * 256 + threadIdx.x;
-  if (tid >= (long)rows_pad * (kpad / 4)) return;
-  const long blk = tid >> 12;  // 16 KB block = (256-row block, 64-k step)
-  const int nks = kpad / 64;
-  const int r = (int)(blk / nks) * 256 + (int)((tid >> 4) & 255);
-  const int kq = (int)(blk % nks) * 16 + (int)(tid & 15);
-  const int er = r < rows ? e[r] : kExpNone;
-  Split21 s[4];
+// Balanced residues of an operand's scaled, rounded entries x = rint(v 2^(bits - e)), |x| <= 2^62: one
+// int8 plane per modulus, rows_pad x kpad in k-step tiled layout (zero outside the matrix). A
+// workgroup takes 64 rows x 64 k through LDS (global reads of 512 contiguous bytes either way; its
+// 64 rows fill 4 KB of one 16 KB block per plane), then each thread 16 consecutive k of one row.
+//   x = xh 2^30 + xl exactly (|xh| <= 2^32, |xl| <= 2^29); y = xh c30 + xl is congruent to x, an exact
+//   integer below 2^40; q = rint(y / m) by adding and taking off 1.5 2^52: y times the rounded 1 / m
+//   is off by less than 2^-20, and y / m lies at least 1 / (2m) from a half for odd m and is exact
+//   for 256, so y - q m is the balanced residue (128 and -128 are the same byte); adding 1.5 2^52
+//   once more leaves it in the low byte. Five FP64 instructions and 3/4 of a byte permutation, all
+//   full-rate; the integer form's multiply-highs are quarter-rate ones. Bound by memory: 16 moduli of
+// two operands of 2048 x 2048 46 us (4.4 TB/s), of 4096 x 4096 209 us; a launch per operand with the
+// integer form took 87 us at 2048 x 2048.
+struct ResidueDst {
+  int bits, kpad;
+  long plane;
+  int8_t* out;
+};
+constexpr int kResStride = 65;  // doubles per LDS row (odd: 64 rows of one k fall into distinct banks)
+
+__device__ __forceinline__ void residues64(const OperandSrc& o, const ResidueDst& d, const ResidueConsts& cc, int block,
+                                           double* tile) {
+  const int t = threadIdx.x, nks = d.kpad / 64;
+  const int r0 = (((block >> 2) / nks) * 4 + (block & 3)) * 64, k0 = (block >> 2) % nks * 64;
 #pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    const int kk = kq * 4 + t;
-    s[t] = split21(r < rows && kk < k ? p[(long)kk + (long)r * ld] : 0.0, er, bits);
+  for (int j = 0; j < 16; ++j) {
+    const int hi = (t >> 6) + 4 * j, lo = t & 63;
+    const int rl = o.kc ? hi : lo, kl = o.kc ? lo : hi, r = r0 + rl, kk = k0 + kl;
+    double v = 0.0;
+    if (r < o.rows && kk < o.k) v = o.p[o.kc ? (long)kk + (long)r * o.ld : (long)r + (long)kk * o.ld];
+    tile[rl * kResStride + kl] = v;
   }
-  const long plane = (long)rows_pad * kpad;
-  int8_t* o = out + tid * 4;
-  for (int q = 0; q < cp.n; ++q) {
-    uint32_t word = 0;
+  __syncthreads();
+  // 4 lanes take a row: a wave's 64 stores of 16 bytes fill 1 KB
+  const int rl = t >> 2, g = t & 3, r = r0 + rl;
+  const int er = r < o.rows ? o.e[r] : kExpNone;
+  double xh[16], xl[16];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) word |= residue8(s[t], cp, q) << (8 * t);
-    *(uint32_t*)(o + q * plane) = word;
+  for (int i = 0; i < 16; ++i) {
+    const double v = tile[rl * kResStride + 16 * g + i];
+    const double x = er == kExpNone ? 0.0 : rint(ldexp(v, d.bits - er));
+    xh[i] = rint(x * 0x1p-30);
+    xl[i] = fma(-xh[i], 0x1p30, x);
+  }
+  const double magic = 0x1.8p52;
+  int8_t* out = d.out + crt_tiled_offset(r, k0 + 16 * g, d.kpad);
+  for (int q = 0; q < cc.n; ++q) {
+    const double c30 = cc.c30[q], inv = cc.inv[q], m = cc.m[q];
+    unsigned b[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const double y = fma(xh[i], c30, xl[i]);
+      const double n = fma(y, inv, magic) - magic;
+      b[i] = (unsigned)__double2loint(fma(-n, m, y) + magic);
+    }
+    unsigned w[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      // bytes 0 of two words into the low and, shifted, the high half
+      const unsigned lo = __builtin_amdgcn_perm(b[4 * i + 1], b[4 * i], 0x0c0c0400);
+      const unsigned hi = __builtin_amdgcn_perm(b[4 * i + 3], b[4 * i + 2], 0x04000c0c);
+      w[i] = lo | hi;
+    }
+    *(uint4*)(out + q * d.plane) = uint4{w[0], w[1], w[2], w[3]};
   }
 }
 
-// Same for a row-contiguous source: a block transposes a 64-row x 64-k tile through LDS (reads
-// of 64 consecutive rows per k), then each thread takes 16 consecutive k of one row and writes
-// 16 bytes per plane (the block's 64 rows fill 4 KB of one 16 KB k-step block). Grid
-// (rows_pad / 64, kpad / 64).
-__global__ __launch_bounds__(256) void crt_residue_rc_kernel(const double* __restrict__ p, long ld, int rows, int k,
-                                                             const int* __restrict__ e, int bits, CrtParams cp,
-                                                             int kpad, long plane, int8_t* __restrict__ out) {
-  __shared__ double tile[64][64];  // [k][row]
-  const int r0 = blockIdx.x * 64, k0 = blockIdx.y * 64, t = threadIdx.x;
-#pragma unroll
-  for (int j = 0; j < 16; ++j) {
-    const int kl = (t >> 6) + 4 * j, rl = t & 63, r = r0 + rl, kk = k0 + kl;
-    tile[kl][rl] = r < rows && kk < k ? p[(long)r + (long)kk * ld] : 0.0;
-  }
-  __syncthreads();
-  const int rl = t & 63, g = t >> 6, r = r0 + rl;
-  const int er = r < rows ? e[r] : kExpNone;
-  Split21 s[16];
-#pragma unroll
-  for (int i = 0; i < 16; ++i) s[i] = split21(tile[16 * g + i][rl], er, bits);
-  int8_t* o = out + crt_tiled_offset(r, k0 + 16 * g, kpad);
-  for (int q = 0; q < cp.n; ++q) {
-    uint32_t w[4] = {0, 0, 0, 0};
-#pragma unroll
-    for (int i = 0; i < 16; ++i) w[i >> 2] |= residue8(s[i], cp, q) << (8 * (i & 3));
-    *(uint4*)(o + q * plane) = uint4{w[0], w[1], w[2], w[3]};
+// Residues of two operands, the second's workgroups (nb) behind the first's (na), and their
+// fallback flags.
+__global__ __launch_bounds__(256) void residues_kernel(OperandSrc a, ResidueDst da, int na, OperandSrc b, ResidueDst db,
+                                                       ResidueConsts cc) {
+  __shared__ double tile[64 * kResStride];
+  const int w = blockIdx.x;
+  if (w < na) {
+    if (w == 0) operand_flag(a);
+    residues64(a, da, cc, w, tile);
+  } else {
+    if (w == na) operand_flag(b);
+    residues64(b, db, cc, w - na, tile);
   }
 }
 
@@ -987,24 +989,42 @@ size_t ozaki2_workspace_bytes(int m, int n, int k, int nmod) {
   return ozaki2_operand_bytes(m, kr, nmod) + ozaki2_operand_bytes(n, kr, nmod) + ozaki2_product_bytes(m, n, nmod);
 }
 
+namespace {
+struct PrepareJob {
+  const double* p;
+  long ld;
+  bool kc;
+  int rows;
+  void* out;
+};
+// Prepare `count` (1 or 2) operands of inner dimension k: their exponents in one launch, their
+// residues and flags in another.
+hipError_t prepare(const PrepareJob* jobs, int count, int k, int nmod, hipStream_t s) {
+  const int kp = (int)pad_to(std::max(k, 1), OZ_BK), bits = ozaki2_bits(nmod, k);
+  OperandSrc src[2] = {};
+  ResidueDst dst[2] = {};
+  int blocks[2] = {0, 0};
+  for (int i = 0; i < count; ++i) {
+    const PrepareJob& j = jobs[i];
+    const long rows_pad = pad_to(j.rows, OZ_BM);
+    int* e = (int*)j.out;
+    src[i] = OperandSrc{j.p, j.ld, j.kc, j.rows, k, e, e + j.rows};
+    dst[i] = ResidueDst{bits, kp, rows_pad * kp, (int8_t*)j.out + exp_flag_bytes(j.rows)};
+    blocks[i] = (int)(rows_pad / 64 * (kp / 64));
+  }
+  const hipError_t e = launch_exponents(src, count, s);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(residues_kernel, dim3(blocks[0] + blocks[1]), dim3(256), 0, s, src[0], dst[0], blocks[0], src[1],
+                     dst[1], residue_consts(nmod));
+  return hipGetLastError();
+}
+}  // namespace
+
 hipError_t ozaki2_prepare(const double* p, long ld, bool kc, int rows, int k, int nmod, void* out, hipStream_t s) {
   if (rows <= 0) return hipSuccess;
   if (nmod < kCrtMinModuli || nmod > kCrtMaxModuli || k > kCrtMaxK) return hipErrorInvalidValue;
-  const int kp = (int)pad_to(std::max(k, 1), OZ_BK);
-  const long rows_pad = pad_to(rows, OZ_BM);
-  int* ex = (int*)out;
-  int8_t* res = (int8_t*)out + exp_flag_bytes(rows);
-  const CrtParams cp = make_crt(nmod);
-  const int bits = ozaki2_bits(nmod, k);
-  hipError_t e;
-  if ((e = ozaki_exponents(p, ld, kc, rows, k, ex, ex + rows, s)) != hipSuccess) return e;
-  if (kc)
-    hipLaunchKernelGGL(crt_residue_kc_kernel, dim3((unsigned)((rows_pad * (kp / 4) + 255) / 256)), dim3(256), 0, s, p,
-                       ld, rows, k, ex, bits, cp, (int)rows_pad, kp, res);
-  else
-    hipLaunchKernelGGL(crt_residue_rc_kernel, dim3((unsigned)(rows_pad / 64), (unsigned)(kp / 64)), dim3(256), 0, s, p,
-                       ld, rows, k, ex, bits, cp, kp, rows_pad * kp, res);
-  return hipGetLastError();
+  const PrepareJob job{p, ld, kc, rows, out};
+  return prepare(&job, 1, k, nmod, s);
 }
 
 hipError_t ozaki2_products(int m, int n, int k, const void* pa, const void* pb, int nmod, void* work, hipStream_t s) {
@@ -1121,8 +1141,8 @@ hipError_t ozaki2_dgemm(char opa, char opb, int m, int n, int k, double alpha, c
     const int k0 = q * kCrtMaxK, kk = std::min(k, k0 + kCrtMaxK) - k0;
     const double* ap = a + (a_kc ? (long)k0 : (long)k0 * lda);
     const double* bp = b + (b_kc ? (long)k0 : (long)k0 * ldb);
-    if ((e = ozaki2_prepare(ap, lda, a_kc, m, kk, nmod, pa, s)) != hipSuccess) return e;
-    if ((e = ozaki2_prepare(bp, ldb, b_kc, n, kk, nmod, pb, s)) != hipSuccess) return e;
+    const PrepareJob jobs[2] = {{ap, lda, a_kc, m, pa}, {bp, ldb, b_kc, n, pb}};
+    if ((e = prepare(jobs, 2, kk, nmod, s)) != hipSuccess) return e;
     if ((e = ozaki2_product(m, n, kk, alpha, pa, pb, q == 0 ? beta : 0.0, cin, ldcin, q == 0 ? accumulate : true, c,
                             ldc, nmod, rc, s)) != hipSuccess)
       return e;
