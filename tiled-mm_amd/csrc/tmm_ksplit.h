@@ -88,6 +88,14 @@ inline int ks_shape(KsType t, long m, long n, long k, int cus, double* us) {
   return best;
 }
 
+// Time in us of a product on the faster of the two kernels.
+inline double product_time(KsType t, long m, long n, long k, int cus) {
+  double us = 0;
+  ks_shape(t, m, n, k, cus, &us);
+  const long edge = t == KsType::Z ? 64 : 128, tiles = ((m + edge - 1) / edge) * ((n + edge - 1) / edge);
+  return tiles >= 2L * cus ? std::min(us, pipe_time(t, tiles, k, cus)) : us;
+}
+
 // Whether an operand's 16-byte row chunks reach over the end of at most one column (a chunk of 4
 // floats over the end of a column, or of two complex floats, of a leading dimension below its size).
 template <typename R>

@@ -1,6 +1,8 @@
 // Out-of-core GEMM planner (see tmm_plan.hpp).
 #include "tmm_plan.hpp"
 
+#include <cmath>
+
 #include <algorithm>
 #include <map>
 #include <stdexcept>
@@ -289,6 +291,84 @@ Plan make_plan(const PlanRequest& rq) {
     }
   }
   return P;
+}
+
+namespace {
+// Estimated seconds of a call with rq's blocks: make_plan's order of copies and products (one group,
+// one compute queue), each queue working through its own in order.
+double call_seconds(const PlanRequest& rq, int es, const std::function<double(long, long, long)>& gemm_s) {
+  const double kByte = es / 56e9, kCopy = 10e-6, kLaunch = 8e-6, kWake = 15e-6, kThreads = 60e-6;
+  const int tm = std::min(rq.tile_m, rq.m), tn = std::min(rq.tile_n, rq.n);
+  const int nm = (rq.m + tm - 1) / tm, nn = (rq.n + tn - 1) / tn;
+  std::vector<int> kb(1, 0);
+  if (rq.first_chunk_k > 0 && rq.first_chunk_k < rq.tile_k && rq.k > rq.tile_k) kb.push_back(rq.first_chunk_k);
+  while (kb.back() < rq.k) kb.push_back((int)std::min<long>((long)kb.back() + rq.tile_k, rq.k));
+  const int chunks = (int)kb.size() - 1;
+  const auto order = shell_order(nm, nn);
+  std::vector<double> a(nm), b(nn), cin(order.size(), 0.0);
+  double in = 0, mul = 0, out = 0;
+  for (int c = 0; c < chunks; ++c) {
+    const int kc = kb[c + 1] - kb[c];
+    const double tile_s = gemm_s(tm, tn, kc);
+    std::fill(a.begin(), a.end(), -1.0);
+    std::fill(b.begin(), b.end(), -1.0);
+    for (size_t p = 0; p < order.size(); ++p) {
+      const int i = order[p].first, j = order[p].second;
+      const double rows = std::min(tm, rq.m - i * tm), cols = std::min(tn, rq.n - j * tn);
+      if (a[i] < 0) a[i] = in += rows * kc * kByte + kCopy;
+      if (b[j] < 0) b[j] = in += cols * kc * kByte + kCopy;
+      if (rq.beta_nonzero && c == (chunks == 1 ? 0 : 1 + (int)((long)p * (chunks - 1) / (long)order.size())))
+        cin[p] = in += rows * cols * kByte + kCopy;
+      mul = std::max({mul, a[i], b[j], c == chunks - 1 ? cin[p] : 0.0});
+      mul += tile_s * (rows / tm) * (cols / tn) + kLaunch;
+      if (c == chunks - 1) out = std::max(out, mul + kWake) + rows * cols * kByte + kCopy;
+    }
+  }
+  return out + (order.size() * chunks > 1 ? kThreads : 0.0);
+}
+}  // namespace
+
+void pipeline_panels(PlanRequest& rq, int elem_bytes, int align, int k_align,
+                     const std::function<double(long, long, long)>& gemm_s) {
+  const double m = rq.m, n = rq.n, k = rq.k, es = elem_bytes;
+  const double bytes_in = es * (m * k + k * n + (rq.beta_nonzero ? m * n : 0)), bytes_out = es * m * n;
+  if (rq.k <= 0 || bytes_in + bytes_out < 8e6) return;
+  const double whole = gemm_s(rq.tile_m, rq.tile_n, rq.k) * (m / rq.tile_m) * (n / rq.tile_n);
+  if (whole > 2 * std::max(bytes_in, bytes_out) / 56e9) return;
+  const PlanRequest base = rq;
+  double least = 0.97 * call_seconds(base, elem_bytes, gemm_s);
+  auto edge = [align](int ext, int tile, int cut) {  // cut 1: the present blocks
+    if (cut == 1) return tile;
+    const long parts = (long)((ext + tile - 1) / tile) * cut;
+    return (int)(((ext + parts - 1) / parts + align - 1) / align * align);
+  };
+  for (int halves = 0; halves < 2; ++halves) {  // the present chunks, or two equal ones if no longer
+    PlanRequest r = base;
+    if (halves) {
+      r.first_chunk_k = 0;
+      r.tile_k = (int)(((rq.k + 1L) / 2 + k_align - 1) / k_align * k_align);
+      if (rq.k < 2048 || r.tile_k > base.tile_k) continue;
+    }
+    for (int cm = 1; cm <= 12; cm += cm < 4 ? 1 : 2) {
+      r.tile_m = edge(rq.m, base.tile_m, cm);
+      if (cm > 1 && (r.tile_m >= base.tile_m || r.tile_m < 2 * align)) continue;
+      for (int cn = 1; cn <= 12; cn += cn < 4 ? 1 : 2) {
+        r.tile_n = edge(rq.n, base.tile_n, cn);
+        if (cn > 1 && (r.tile_n >= base.tile_n || r.tile_n < 2 * align)) continue;
+        const double nm = std::ceil(m / r.tile_m), nn = std::ceil(n / r.tile_n);
+        if (nm * nn > 128) break;
+        // one group: the work pool of make_plan
+        const double tk = std::min<double>(r.tile_k, k);
+        const double pool = 2 * tk * (nm * r.tile_m + nn * r.tile_n) + (rq.beta_nonzero ? 2 : 1) * nm * nn * (double)r.tile_m * r.tile_n;
+        if (pool > (double)rq.pool_budget_elems) continue;
+        const double t = call_seconds(r, elem_bytes, gemm_s);
+        if (t < least) {
+          least = t;
+          rq = r;
+        }
+      }
+    }
+  }
 }
 
 int operand_producer(const Plan& P, size_t gemm, Mat mat) {

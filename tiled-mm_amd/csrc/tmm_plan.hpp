@@ -17,6 +17,7 @@
 #include <cstdint>
 #include <functional>
 #include <string>
+#include <utility>
 #include <vector>
 
 namespace tmm {
@@ -95,6 +96,20 @@ std::vector<std::pair<int, int>> shell_order(int nTm, int nTn);
 
 // Build the plan. Throws std::invalid_argument on inconsistent input.
 Plan make_plan(const PlanRequest& rq);
+
+// Block sizes that shorten a call to which the host link matters. With one block, or a few large
+// ones, the copies in, the products and the copies back follow each other at both ends of the call:
+// nothing runs before the first blocks are in, and the last block's product and copy back run alone
+// (DGEMM TN 1976 x 2631 x 2728 in one block: 1.76 ms in, 0.43 ms of product, 0.73 ms out, 3.06 ms in
+// all). The blocks are cut in either dimension, and k perhaps into two equal chunks, by the estimated time
+// of the call: the plan's copies and products in their order on three queues, the host link at 56
+// GB/s per direction and 10 us per copy (measured), gemm_s(rows, columns, k) seconds per product.
+// rq: the request with its present blocks (tile_*, first_chunk_k), which stay where no cut gains 3%,
+// where the products take more than twice the link's time (both ends are then a small part), and in
+// calls of less than 8 MB, whose copies cost more apart than together. align: granularity of the cuts;
+// k_align: of the chunks.
+void pipeline_panels(PlanRequest& rq, int elem_bytes, int align, int k_align,
+                     const std::function<double(long, long, long)>& gemm_s);
 
 // Index of the H2D op that filled the A (mat == Mat::A) or B operand block a GEMM op reads, or
 // -1 when none of its dependencies did (the operand then has no identity to share).

@@ -21,6 +21,7 @@
 #include <sstream>
 
 #include "tmm_kernels.h"
+#include "tmm_ksplit.h"
 #include "tmm_ozaki.h"
 
 namespace tmm {
@@ -175,6 +176,7 @@ Handle::Handle(int dt, int streams, int tm, int tn, int tk)
     : dtype(dt), n_streams(streams), max_tm(tm), max_tn(tn), max_tk(tk) {
   elem_bytes = dt == 0 ? 4 : dt == 1 ? 8 : dt == 2 ? 8 : 16;
   hip_check(hipGetDevice(&device), "hipGetDevice");
+  hip_check(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device), "hipDeviceGetAttribute");
   // The copy streams first, then one compute stream; further compute streams only when a plan
   // runs tile GEMMs on several queues (compute_stream). HIP streams share the device's few
   // hardware queues once they outnumber them, and a copy stream sharing one with the busy
@@ -409,7 +411,7 @@ void strided_copy_parallel(ThreadPool& tp, char* dst, size_t dpitch, const char*
                            size_t height) {
   const size_t total = width * height;
   if (total == 0) return;
-  const size_t min_task = 1 << 20;
+  const size_t min_task = 1 << 19;
   int ntask = (int)std::min<size_t>(std::max<size_t>(1, total / min_task), (size_t)(tp.size() + 1) * 2);
   tp.parallel_for(ntask, [&](int t) {
     size_t b0 = total * (size_t)t / ntask, b1 = total * (size_t)(t + 1) / ntask;
@@ -495,8 +497,13 @@ struct Scatterer {
 // scheme II DGEMM TN 40000^3 (host-link bound): 0.90-0.99 s per call with 6 x 64 MiB, 0.834 s with
 // 6 x 128 MiB, 0.838 with 4 x 256, 0.841 with 12 x 64, 0.825 with 12 x 128; the native call
 // (kernel bound) ran 1.856-1.862 s with every ring.
+// A piece is at most a slot, and 1/64 of the call's bytes (at least 8 MiB) in a smaller call, so that
+// packing, the DMA and the scatter of its pieces overlap (63 MB in and 45 MB out as three pieces:
+// 3.3 ms, most of it one after the other).
 constexpr size_t kStageBytes = 128u << 20;
+constexpr size_t kStageMinPiece = 8u << 20;
 constexpr int kStageSlots = 8;
+size_t stage_piece(size_t call_bytes) { return std::min(kStageBytes, std::max(kStageMinPiece, call_bytes / 64)); }
 
 // Cross-thread state of one plan execution (one thread per copy queue, the caller's thread for
 // the GEMMs). Every op is "marked" once it has been enqueued and, when another queue depends on
@@ -560,6 +567,7 @@ void execute_plan(Handle& h, const Plan& P, const GemmCall& call, const bool pin
 
   const bool any_pageable_in = !pinned[0] || !pinned[1] || (use_beta && !pinned[2]);
   const bool pageable_out = call.copy_back && !pinned[2];
+  const size_t piece_in = stage_piece(P.h2d_elems * es), piece_out = stage_piece(P.d2h_elems * es);
   if (any_pageable_in) h.stage_in.ensure(kStageSlots, kStageBytes);
   if (pageable_out) h.stage_out.ensure(kStageSlots, kStageBytes);
   ThreadPool* tp = (any_pageable_in || pageable_out) ? &h.pool_threads() : nullptr;
@@ -662,9 +670,16 @@ void execute_plan(Handle& h, const Plan& P, const GemmCall& call, const bool pin
   // their first DMA is enqueued, instead of with hipStreamWaitEvent: no barrier packet then
   // sits in a copy stream, where, should that stream share a hardware queue with a compute
   // stream, it would hold back the GEMMs submitted after it.
+  // A plan of one product runs on the caller's thread alone, its copy back ordered on the device:
+  // starting two threads and waking one of them took longer than a small call's work.
+  const bool one_product = n_gemm == 1;
   auto wait_deps_host = [&](const Op& op) {
     for (int d : op.deps) {
       if (d < 0 || P.ops[d].queue == op.queue) continue;
+      if (one_product) {
+        hip_check(hipStreamWaitEvent(stream_of(op.queue), h.events[d], 0), "hipStreamWaitEvent");
+        continue;
+      }
       if (!sync.wait(d)) throw Error(2, "aborted after a failure in another queue");
       hip_check(hipEventSynchronize(h.events[d]), "hipEventSynchronize (copy dependency)");
     }
@@ -684,7 +699,7 @@ void execute_plan(Handle& h, const Plan& P, const GemmCall& call, const bool pin
       } else {
         StagingRing& R = h.stage_in;
         if (width > R.slot_bytes) R.ensure(kStageSlots, width);
-        const int cpp = (int)std::max<size_t>(1, R.slot_bytes / width);
+        const int cpp = (int)std::max<size_t>(1, std::min(R.slot_bytes, piece_in) / width);
         for (int c0 = 0; c0 < op.cols; c0 += cpp) {
           const int nc = std::min(cpp, op.cols - c0);
           const int sl = R.next;
@@ -768,7 +783,7 @@ void execute_plan(Handle& h, const Plan& P, const GemmCall& call, const bool pin
       } else {
         StagingRing& R = h.stage_out;
         if (width > R.slot_bytes) throw Error(5, "C tile column larger than a staging slot");
-        const int cpp = (int)std::max<size_t>(1, R.slot_bytes / width);
+        const int cpp = (int)std::max<size_t>(1, std::min(R.slot_bytes, piece_out) / width);
         for (int c0 = 0; c0 < op.cols; c0 += cpp) {
           const int nc = std::min(cpp, op.cols - c0);
           const int sl = R.next;
@@ -788,14 +803,14 @@ void execute_plan(Handle& h, const Plan& P, const GemmCall& call, const bool pin
   };
 
   // Run the ops of one thread in plan order: sel = -2 the compute queues, 0 / 1 the H2D / D2H
-  // queue. GEMMs wait for other queues on the device (hipStreamWaitEvent), copies on the host
+  // queue, -1 all of them. GEMMs wait for other queues on the device (hipStreamWaitEvent), copies on the host
   // (inside enqueue). Returns early once any thread has failed.
   auto run_ops = [&](bool worker, int sel) {
     try {
       if (worker) hip_check(hipSetDevice(h.device), "hipSetDevice");
       for (size_t oi = 0; oi < nops; ++oi) {
         const Op& op = P.ops[oi];
-        if (!(sel == -2 ? op.queue >= 2 : op.queue == sel)) continue;
+        if (sel != -1 && !(sel == -2 ? op.queue >= 2 : op.queue == sel)) continue;
         if (op.queue >= 2 && group_of[oi] >= 0) {
           const std::vector<size_t>& g = groups[group_of[oi]];
           if (oi != g[0]) continue;  // enqueued and marked with its group
@@ -869,7 +884,9 @@ void execute_plan(Handle& h, const Plan& P, const GemmCall& call, const bool pin
       sync.fail(2, e.what());
     }
   };
-  {
+  if (one_product) {
+    run_ops(false, -1);
+  } else {
     std::thread th_in([&] { run_ops(true, 0); });
     std::thread th_out([&] { run_ops(true, 1); });
     run_ops(false, -2);
@@ -988,6 +1005,7 @@ void gemm_host(Handle& h, const GemmCall& in) {
     tn = align_edge(call.n, tn, align_n);
   }
 
+  const int block_m = tm, block_n = tn;
   PlanRequest rq;
   rq.opa = call.opa;
   rq.opb = call.opb;
@@ -1043,6 +1061,16 @@ void gemm_host(Handle& h, const GemmCall& in) {
     }
     rq.pool_budget_elems = budget / es;
   }
+  // calls to which the host link matters: smaller blocks (native products; the emulation shares
+  // prepared operands between whole blocks)
+  if (h.coarsen && call.copy_back && !ozaki_active(h) && h.first_chunk < 0) {
+    const KsType type = h.dtype == 0 ? KsType::S : h.dtype == 1 ? KsType::D : h.dtype == 2 ? KsType::C : KsType::Z;
+    const int cus = h.cus;
+    pipeline_panels(rq, es, 64, kstep, [type, cus](long m, long n, long k) {
+      return product_time(type, m, n, k, cus) * 1e-6;
+    });
+    if (rq.tile_m != tm || rq.tile_n != tn) rq.n_compute_queues = 1;  // a block fills the device
+  }
   Plan P;
   try {
     P = make_plan(rq);
@@ -1079,8 +1107,8 @@ void gemm_host(Handle& h, const GemmCall& in) {
   h.stats[0] = (double)P.h2d_elems * es;
   h.stats[1] = (double)P.d2h_elems * es;
   h.stats[2] = ngemm;
-  h.stats[3] = P.tile_m;
-  h.stats[4] = P.tile_n;
+  h.stats[3] = std::min(block_m, call.m);
+  h.stats[4] = std::min(block_n, call.n);
   h.stats[5] = P.tile_k;
   h.stats[6] = P.nTk;
   h.stats[7] = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();

@@ -121,6 +121,7 @@ struct Handle {
   int dtype = 1;
   int elem_bytes = 8;
   int device = 0;
+  int cus = 256;  // compute units of the device
   int n_streams = 2;
   int max_tm = 5000, max_tn = 5000, max_tk = 5000;
   int cur_tm = 0, cur_tn = 0, cur_tk = 0;  // current tile sizes (set_tile_sizes)
