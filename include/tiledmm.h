@@ -178,7 +178,8 @@ int tmm_synchronize(tmm_handle* h);
  *                        after the other) and enqueueing them on the three queues (H2D and D2H
  *                        overlap); 1 always the graph; 0 never.
  *   TMM_OPT_BATCH_BODY   tmm_dgemm_batched tile body: -1 (default) the autotuner's choice (the faster
- *                        one measured), 0 register-staged LDS double buffer, 1 direct-to-LDS ring.
+ *                        one measured), 0 register-staged LDS double buffer, 1 direct-to-LDS rings with the inner
+ *                        dimension split over the waves. A batch with a dimension above 2^25 runs on 0.
  *   TMM_OPT_BATCH_QUEUES tmm_dgemm_batched compute queues: 0 (default) the autotuner's choice, 1 or 2.
  *   TMM_OPT_BATCH_EMULATION tmm_dgemm_batched on a handle with TMM_OPT_OZAKI_MODULI set: -1 (default)
  *                        each problem runs as Ozaki scheme II products when the autotuner's model

@@ -16,12 +16,12 @@
 //     its modelled emulated time, 2mnk / (R_emu * min(1, tiles / CUs)) + o_emu with tiles its
 //     256x256 product tiles, beats 2mnk / R_native;
 //   * the compute queue count (1 or 2): with 2, consecutive groups' kernels may overlap, which
-//     hides the last partial wave of each group (modelled as one 128x128 tile of the group's
-//     largest k per group);
+//     hides the last partial wave of each group (modelled as one tile of the group's largest k per
+//     group);
 //   * G in {1, 2, 4, ..., 64}, and one captured hipGraph vs the queues (pinned memory only): this
 //     ROCm's graph executor runs copy nodes one after the other, so with the graph H2D and D2H
 //     add up: T = max(H + D + c/G, C + h + d) without per-group host cost.
-// The persistent grid fills the CUs at the chosen body's occupancy (2 or 3 workgroups per CU).
+// The persistent grid fills the CUs at the bodies' occupancy (2 workgroups per CU).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -98,7 +98,7 @@ void calibrate_rates(Handle& h) {
   dev.release();
 
   // persistent kernel rates on problems of 1024^3 (contents irrelevant: zero-filled); 64 tiles
-  // each, 6 * CUs tiles in all, so that both grids (2 and 3 workgroups per CU) run whole rounds
+  // of 128 x 128 each, 6 * CUs in all, so that the grid (2 workgroups per CU) runs whole rounds
   int dev_id = 0, cus = 256;
   hip_check(hipGetDevice(&dev_id), "hipGetDevice");
   hip_check(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev_id), "hipDeviceGetAttribute");
@@ -106,39 +106,51 @@ void calibrate_rates(Handle& h) {
   DeviceBuffer mats, meta;
   mats.reserve((size_t)3 * np * sz * sz * 8);
   hip_check(hipMemsetAsync(mats.ptr, 0, (size_t)3 * np * sz * sz * 8, s), "hipMemsetAsync");
-  std::vector<GemmParams<double>> desc(np);
-  std::vector<int> items;
+  std::vector<GemmParams<double>> desc(np + 1);
+  std::vector<int> items[2];  // of each tile body
   for (int i = 0; i < np; ++i) {
     double* base = (double*)mats.ptr + (size_t)3 * i * sz * sz;
     desc[i] = GemmParams<double>{'N', 'N', sz, sz, sz, 1.0, 0.0, base, sz, base + (size_t)sz * sz, sz, 0.0, 0.0,
                                  nullptr, sz, 0, base + (size_t)2 * sz * sz, sz};
-    for (int bm = 0; bm < sz / 128; ++bm)
-      for (int bn = 0; bn < sz / 128; ++bn) {
-        items.push_back(i);
-        items.push_back(bm);
-        items.push_back(bn);
-      }
+    for (int body = 0; body < 2; ++body)
+      for (int bm = 0; bm < sz / batched_tile(body); ++bm)
+        for (int bn = 0; bn < sz / batched_tile(body); ++bn) items[body].insert(items[body].end(), {i, bm, bn});
   }
-  meta.reserve(sizeof(GemmParams<double>) * np + items.size() * sizeof(int) + 1024);
-  GemmParams<double>* d_desc = (GemmParams<double>*)meta.ptr;
-  int* d_items = (int*)((char*)meta.ptr + ((sizeof(GemmParams<double>) * np + 255) & ~(size_t)255));
-  int* d_counter = d_items + ((items.size() + 63) & ~(size_t)63);
-  hip_check(hipMemcpy(d_desc, desc.data(), sizeof(GemmParams<double>) * np, hipMemcpyHostToDevice), "hipMemcpy");
-  hip_check(hipMemcpy(d_items, items.data(), items.size() * sizeof(int), hipMemcpyHostToDevice), "hipMemcpy");
-  const int n_items = (int)(items.size() / 3);
+  desc[np] = desc[0];  // and one 8 x 8 x 8 product, as a single item
+  desc[np].m = desc[np].n = desc[np].k = 8;
+  items[1].insert(items[1].end(), {np, 0, 0});
+  const size_t at_items0 = (sizeof(GemmParams<double>) * desc.size() + 255) & ~(size_t)255;
+  const size_t at_items1 = at_items0 + ((items[0].size() * sizeof(int) + 255) & ~(size_t)255);
+  const size_t at_counters = at_items1 + ((items[1].size() * sizeof(int) + 255) & ~(size_t)255);
+  meta.reserve(at_counters + 16 * sizeof(int));
+  char* m = (char*)meta.ptr;
+  GemmParams<double>* d_desc = (GemmParams<double>*)m;
+  int* d_items[2] = {(int*)(m + at_items0), (int*)(m + at_items1)};
+  int* d_counters = (int*)(m + at_counters);  // one per launch
+  hip_check(hipMemcpy(d_desc, desc.data(), sizeof(GemmParams<double>) * desc.size(), hipMemcpyHostToDevice), "hipMemcpy");
+  for (int body = 0; body < 2; ++body)
+    hip_check(hipMemcpy(d_items[body], items[body].data(), items[body].size() * sizeof(int), hipMemcpyHostToDevice),
+              "hipMemcpy");
+  hip_check(hipMemsetAsync(d_counters, 0, 16 * sizeof(int), s), "hipMemsetAsync");
   for (int body = 0; body < 2; ++body) {
-    const int grid = (body ? 3 : 2) * cus;  // the body's workgroups per CU
-    hip_check(launch_gemm_d_batched('N', 'N', d_desc, d_items, n_items, d_counter, grid, s, body), "batched launch");
+    const int n_items = np * (sz / batched_tile(body)) * (sz / batched_tile(body));
+    auto run = [&](int launch) {
+      hip_check(launch_gemm_d_batched('N', 'N', d_desc, d_items[body], n_items, d_counters + 2 * body + launch, 2 * cus, s,
+                                      body),
+                "batched launch");
+    };
+    run(0);
     hip_check(hipEventRecord(e0, s), "hipEventRecord");
-    hip_check(launch_gemm_d_batched('N', 'N', d_desc, d_items, n_items, d_counter, grid, s, body), "batched launch");
+    run(1);
     hip_check(hipEventRecord(e1, s), "hipEventRecord");
     const double t = elapsed();
     (body == 0 ? h.rates.kernel_flops : h.rates.kernel_flops_dlds) = 2.0 * np * (double)sz * sz * sz / t;
   }
-  // per-group fixed cost: an empty item list still runs the counter kernel and the grid
+  // per-group fixed cost: the launch of a single small tile
   hip_check(hipEventRecord(e0, s), "hipEventRecord");
   for (int r = 0; r < 8; ++r)
-    hip_check(launch_gemm_d_batched('N', 'N', d_desc, d_items, 0, d_counter, 3 * cus, s, 1), "batched launch");
+    hip_check(launch_gemm_d_batched('N', 'N', d_desc, d_items[1] + items[1].size() - 3, 1, d_counters + 4 + r, 2 * cus, s, 1),
+              "batched launch");
   hip_check(hipEventRecord(e1, s), "hipEventRecord");
   h.rates.group_overhead_s = std::max(10e-6, elapsed() / 8 + 10e-6);  // + events and copy-queue switches
   hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");
@@ -208,7 +220,11 @@ BatchConfig choose_batch_config(Handle& h, const BatchShape& shape) {
   best.predicted_s = 1e300;
   // tile body: the faster persistent kernel, with as many workgroups as fit the CUs
   best.body = h.batch_body >= 0 ? h.batch_body : (r.kernel_flops_dlds >= r.kernel_flops ? 1 : 0);
-  best.workgroups = (best.body ? 3 : 2) * cus;
+  // the k-split body's lane offsets are 32 bits wide: leading dimensions (= rows) of up to 256 MB
+  if (std::max({*std::max_element(shape.m.begin(), shape.m.end()), *std::max_element(shape.n.begin(), shape.n.end()),
+                *std::max_element(shape.k.begin(), shape.k.end())}) > (1 << 25))
+    best.body = 0;
+  best.workgroups = 2 * cus;
   const double rate = best.body ? r.kernel_flops_dlds : r.kernel_flops;
   // native or emulated per problem; the compute total and the largest k of the native items
   const int cnt = (int)shape.m.size();
@@ -233,8 +249,8 @@ BatchConfig choose_batch_config(Handle& h, const BatchShape& shape) {
     csum += tn;
     kmax = std::max(kmax, shape.k[i]);
   }
-  // a group's last partial wave: about one 128x128 tile of the largest k on one CU's share
-  const double tail = 2.0 * 128 * 128 * (double)kmax / (rate / (3.0 * cus));
+  // a group's last partial wave: about one tile of the largest k on one workgroup's share
+  const double edge = batched_tile(best.body), tail = 2.0 * edge * edge * (double)kmax / (rate / (2.0 * cus));
   const double hsum = shape.h2d_bytes / r.h2d_Bps, dsum = shape.d2h_bytes / r.d2h_Bps;
   const bool graph_ok = shape.pinned && h.batch_graph != 0, graph_only = graph_ok && h.batch_graph == 1;
   for (int G = 1; G <= 64; G *= 2) {

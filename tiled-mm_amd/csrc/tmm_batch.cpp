@@ -5,9 +5,9 @@
 // device-wide synchronisation). Here the whole batch is one pipeline:
 //   * the problems are packed into one device arena and cut into G groups of about equal
 //     host-link bytes; group g's H2D copies (spread over two copy queues), one persistent
-//     batched-kernel launch over all 128x128 C tiles of the group (largest k first), and its D2H
-//     copies run on their own queues, so H2D of group g+1 overlaps the kernel of group g and the
-//     D2H of group g-1;
+//     batched-kernel launch over all C tiles of the group (largest k first), and its D2H copies run
+//     on their own queues, so H2D of group g+1 overlaps the kernel of group g and the D2H of group
+//     g-1;
 //   * with pinned host matrices the whole sequence is captured once into a hipGraph and
 //     launched as one graph (no per-problem launch overhead);
 //   * G, the persistent grid, the tile body (register-staged or direct-to-LDS), the compute
@@ -141,14 +141,15 @@ void gemm_batched_host(Handle& h, char opa, char opb, int count, const int* m, c
   double* dev = (double*)h.pool.ptr;
   std::vector<GemmParams<double>> desc(count);
   std::vector<std::vector<int>> items(G);
+  const int edge = batched_tile(cfg.body);
   for (int g = 0; g < G; ++g) {
     std::vector<int> order;
     for (int i = gstart[g]; i < gstart[g + 1]; ++i) order.push_back(i);
     std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return P[x].k > P[y].k; });
     for (int i : order)
       if (!cfg.emulate[i])
-      for (int bm = 0; bm < (P[i].m + 127) / 128; ++bm)
-        for (int bn = 0; bn < (P[i].n + 127) / 128; ++bn) {
+      for (int bm = 0; bm < (P[i].m + edge - 1) / edge; ++bm)
+        for (int bn = 0; bn < (P[i].n + edge - 1) / edge; ++bn) {
           items[g].push_back(i);
           items[g].push_back(bm);
           items[g].push_back(bn);
@@ -176,21 +177,24 @@ void gemm_batched_host(Handle& h, char opa, char opb, int count, const int* m, c
     d.c = dev + p.offC;
     d.ldc = std::max(1, p.m);
   }
-  size_t meta_bytes = sizeof(GemmParams<double>) * count + 256;
+  // descriptors, work items and the groups' zeroed item counters in one upload
   std::vector<size_t> item_off(G + 1, 0);
   for (int g = 0; g < G; ++g) item_off[g + 1] = item_off[g] + items[g].size();
-  meta_bytes += item_off[G] * sizeof(int) + 256 + 64 * G;
+  auto align256 = [](size_t b) { return (b + 255) & ~(size_t)255; };
+  const size_t at_items = align256(sizeof(GemmParams<double>) * count);
+  const size_t at_counters = align256(at_items + item_off[G] * sizeof(int)), meta_bytes = at_counters + 64 * (size_t)G;
   h.batch_meta.reserve(meta_bytes);
   char* meta = (char*)h.batch_meta.ptr;
   GemmParams<double>* d_desc = (GemmParams<double>*)meta;
-  int* d_items = (int*)(meta + ((sizeof(GemmParams<double>) * count + 255) & ~(size_t)255));
-  int* d_counters = d_items + ((item_off[G] + 63) & ~(size_t)63);
-  hip_check(hipMemcpy(d_desc, desc.data(), sizeof(GemmParams<double>) * count, hipMemcpyHostToDevice), "hipMemcpy");
+  int* d_items = (int*)(meta + at_items);
+  int* d_counters = (int*)(meta + at_counters);
   {
-    std::vector<int> flat(item_off[G]);
-    for (int g = 0; g < G; ++g) std::copy(items[g].begin(), items[g].end(), flat.begin() + item_off[g]);
-    if (!flat.empty())
-      hip_check(hipMemcpy(d_items, flat.data(), flat.size() * sizeof(int), hipMemcpyHostToDevice), "hipMemcpy");
+    std::vector<char> flat(meta_bytes);
+    std::memcpy(flat.data(), desc.data(), sizeof(GemmParams<double>) * count);
+    for (int g = 0; g < G; ++g)
+      if (!items[g].empty())
+        std::memcpy(flat.data() + at_items + item_off[g] * sizeof(int), items[g].data(), items[g].size() * sizeof(int));
+    hip_check(hipMemcpy(meta, flat.data(), meta_bytes, hipMemcpyHostToDevice), "hipMemcpy");
   }
 
   hipStream_t sh = h.h2d, sd = h.d2h;

@@ -410,10 +410,6 @@ __global__ __launch_bounds__(256, 2) void gemm_real_batched_kernel(const GemmPar
   }
 }
 
-__global__ void zero_counter_kernel(int* c) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) c[0] = 0;
-}
-
 // ---------------------------------------------------------------------------------------------
 // Complex GEMM: 256 threads, 2x2 waves, wave tile 32x32 complex (2x2 blocks, re and im
 // accumulators), WG tile 64x64 complex. Each block update is four real MFMAs.
@@ -569,152 +565,8 @@ __device__ __forceinline__ V last_frag(const R* __restrict__ p, long ld, int row
 }
 
 // ---------------------------------------------------------------------------------------------
-// FP64 tile with direct global->LDS loads (global_load_lds_dwordx4) into an S-stage LDS ring, the
-// body of the batched path. WG tile 128x128, 2x2 waves of 64x64, k-step 8 per stage, S stages of
-// 16 KB (S = 3, three workgroups per CU).
-// The loads of stage kt+S-1 are issued right after the barrier of stage kt, so S-1 stages are in
-// flight while the MFMAs run; no registers or ds_write instructions carry the operands.
-//   k-contiguous operand (A for 'T', B for 'N'): LDS [row][slot][2], a 16-byte chunk = 2
-//     consecutive k of one row, the 4 chunks of a row XOR-permuted over its 4 slots; a wave
-//     instruction fills 16 consecutive rows, reading 64 contiguous bytes of each.
-//   row-contiguous operand (A for 'N', B for 'T'): LDS [k][row], a 16-byte chunk = 2 consecutive
-//     rows at one k; a wave instruction fills all 128 rows of one k (coalesced in global memory).
-// Rows beyond the matrix load a clamped row: they only feed outputs that are not stored.
-// ---------------------------------------------------------------------------------------------
-template <bool KC>
-struct DldsOperand {
-  // k-contiguous stage layout: [row][slot][2], 64 bytes per row, slot s of row r holding the k
-  // pair (2q, 2q+1) with q = s ^ kc_swz(r). The fragment read of one k pair by 16 consecutive rows
-  // then touches 8 distinct 16-byte bank groups per 8 lanes (rows r, r+1 share a swizzle and sit
-  // 64 bytes apart), i.e. it is free of bank conflicts.
-  __device__ __forceinline__ static int kc_swz(int r) { return (r >> 1) & 3; }
-  // issue this wave's 2 loads of one stage (8 instructions per workgroup). The operand lies in a
-  // device arena with at least 16 more bytes after its last column, so a row-contiguous operand of
-  // odd row count may read its last 2-row chunk one row past the end (that row only feeds unstored
-  // outputs).
-  __device__ __forceinline__ static void issue(const double* __restrict__ p, long ld, int r0, int nrows, int k0,
-                                               double* stage, int wave, int lane) {
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const int inst = wave * 2 + t;  // 0..7
-      const double* src;
-      double* dst;
-      if (KC) {
-        // 16 rows x 64 bytes per instruction: lanes 4j..4j+3 read the 4 chunks of row j, so the
-        // global access is contiguous per row; lane l lands in slot l % 4 of its row, which holds
-        // chunk (l % 4) ^ swz(row) (see kc_slot)
-        const int local = inst * 16 + (lane >> 2);
-        const int q = (lane & 3) ^ kc_swz(local);
-        const int row = min(r0 + local, nrows - 1);
-        src = p + (long)(2 * q + k0) + (long)row * ld;
-        dst = stage + inst * 128;
-      } else {
-        const int kk = inst;
-        const int row = min(r0 + 2 * lane, (nrows - 1) & ~1);
-        src = p + (long)row + (long)(k0 + kk) * ld;
-        dst = stage + kk * 128;
-      }
-      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
-                                       (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
-    }
-  }
-  // values at k = 2g, 2g+1 of row `row` of the stage
-  __device__ __forceinline__ static void frag(const double* stage, int g, int row, double& v0, double& v1) {
-    if (KC) {
-      const v2d c = *(const v2d*)(stage + row * 8 + (g ^ kc_swz(row)) * 2);
-      v0 = c[0];
-      v1 = c[1];
-    } else {
-      v0 = stage[(2 * g) * 128 + row];
-      v1 = stage[(2 * g + 1) * 128 + row];
-    }
-  }
-};
-
-// One 128x128 C tile at (m0, n0) of a problem in the batch's device arena (see
-// DldsOperand::issue): any m, n >= 1, any K (the last K % 8 values are added in the epilogue from
-// global memory).
-template <bool A_KC, bool B_KC, int S>
-__device__ __forceinline__ void dlds_tile_at(const GemmParams<double>& prm, int m0, int n0) {
-  constexpr int STAGE = 2 * 1024;  // A and B, 1024 doubles each
-  __shared__ __attribute__((aligned(16))) double lds[S * STAGE];
-  const int M = prm.m, N = prm.n, K = prm.k;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wm = wave & 1, wn = wave >> 1;
-  const int li = lane & 15, lg = lane >> 4;
-  const int nkt = K / 8;
-
-  dbl4 acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = dbl4{0, 0, 0, 0};
-
-  auto issue = [&](int kt) {
-    double* st = lds + (kt % S) * STAGE;
-    DldsOperand<A_KC>::issue(prm.a, prm.lda, m0, M, kt * 8, st, wave, lane);
-    DldsOperand<B_KC>::issue(prm.b, prm.ldb, n0, N, kt * 8, st + 1024, wave, lane);
-  };
-#pragma unroll
-  for (int s = 0; s < S - 1; ++s)
-    if (s < nkt) issue(s);
-  for (int kt = 0; kt < nkt; ++kt) {
-    // this wave's loads of stage kt have landed once at most 4 per later stage are pending; its
-    // LDS reads of stage kt-1 are done (lgkmcnt 0); the barrier extends both to the workgroup
-    const int later = min(S - 2, nkt - 1 - kt);
-    if (later >= 3) __builtin_amdgcn_s_waitcnt(0x070 | 12);
-    else if (later == 2) __builtin_amdgcn_s_waitcnt(0x070 | 8);
-    else if (later == 1) __builtin_amdgcn_s_waitcnt(0x070 | 4);
-    else __builtin_amdgcn_s_waitcnt(0x070);
-    __builtin_amdgcn_s_barrier();
-    if (kt + S - 1 < nkt) issue(kt + S - 1);  // into the slot of stage kt-1, free after the barrier
-    const double* st = lds + (kt % S) * STAGE;
-    double a0[4], a1[4], b0[4], b1[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) DldsOperand<A_KC>::frag(st, lg, wm * 64 + i * 16 + li, a0[i], a1[i]);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) DldsOperand<B_KC>::frag(st + 1024, lg, wn * 64 + j * 16 + li, b0[j], b1[j]);
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) acc[i][j] = mfma(b0[j], a0[i], acc[i][j]);
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) acc[i][j] = mfma(b1[j], a1[i], acc[i][j]);
-  }
-
-  const double alpha = prm.alpha, beta = prm.beta;
-  const bool acc_prev = prm.accumulate != 0, use_cin = beta != 0.0;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int gi = m0 + wm * 64 + i * 16 + li;
-    if (gi >= M) continue;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int gj = n0 + wn * 64 + j * 16 + out_col<double>(lane, r);
-        if (gj >= N) continue;
-        double sum = acc[i][j][r];
-        for (int kk = nkt * 8; kk < K; ++kk) {
-          const double av = A_KC ? prm.a[(long)kk + (long)gi * prm.lda] : prm.a[(long)gi + (long)kk * prm.lda];
-          const double bv = B_KC ? prm.b[(long)kk + (long)gj * prm.ldb] : prm.b[(long)gj + (long)kk * prm.ldb];
-          sum = fma(av, bv, sum);
-        }
-        double v = alpha * sum;
-        double* dst = prm.c + (long)gi + (long)gj * prm.ldc;
-        if (acc_prev) v += *dst;
-        if (use_cin) v += beta * prm.cin[(long)gi + (long)gj * prm.ldcin];
-        *dst = v;
-      }
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------------------------
-// FP32 GEMM with direct global->LDS loads: the FP64 kernel's ring with 16-byte chunks of 4 floats,
-// so a stage holds k-step 16 (64 bytes per operand row), 3 stages; workgroup tiles of 128 x 128 (4
+// FP32 GEMM with direct global->LDS loads: the FP64 kernel's ring (BigOperand) with 16-byte chunks
+// of 4 floats, so a stage holds k-step 16 (64 bytes per operand row), 3 stages; workgroup tiles of 128 x 128 (4
 // waves, 16 KB per stage, two or three per CU). A lane's 16-byte fragment holds k = 4g..4g+3 of its
 // row (g = lane / 16) and feeds four v_mfma_f32_16x16x4f32, the same k permutation for A and B.
 //   k-contiguous operand: LDS [row][slot][4], chunk q (k = 4q..4q+3) of row r in slot q ^ swz(r),
@@ -897,26 +749,6 @@ __global__ __launch_bounds__(256, 2) void gemm_s_pipe_kernel(GemmParams<float> p
   int bm, bn;
   tile_coords(blockIdx.x, nbm, nbn, bm, bn);
   spipe_tile_at<A_KC, B_KC, 128, 128>(prm, bm * 128, bn * 128);
-}
-
-// Persistent batched FP64 GEMM on the direct-to-LDS tile body: the same item protocol as
-// gemm_real_batched_kernel, operands in the batch's device arena (any m, n >= 1 and any k),
-// three workgroups per CU.
-template <bool A_KC, bool B_KC, int S>
-__global__ __launch_bounds__(256, 3) void gemm_d_dlds_batched_kernel(const GemmParams<double>* __restrict__ probs,
-                                                                    const int* __restrict__ items, int n_items,
-                                                                    int* __restrict__ counter) {
-  __shared__ int next;
-  for (;;) {
-    if (threadIdx.x == 0) next = atomicAdd(counter, 1);
-    __syncthreads();
-    const int it = next;
-    __syncthreads();  // everyone has read `next` before thread 0 overwrites it
-    if (it >= n_items) break;
-    const GemmParams<double> prm = probs[items[3 * it]];
-    dlds_tile_at<A_KC, B_KC, S>(prm, items[3 * it + 1] * 128, items[3 * it + 2] * 128);
-    __syncthreads();  // every wave is done with the LDS ring before the next item refills it
-  }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1246,8 +1078,9 @@ __global__ __launch_bounds__(256, 2) void gemm_c_pipe_kernel(GemmParams<float> p
 // Software-pipelined FP64 GEMM, two tile widths BN: 128 x 256 workgroup tiles (2 x 2 waves of
 // 64 x 128, one workgroup per CU, so each wave has a SIMD to itself and its 32 accumulator blocks,
 // 256 registers, live in AGPRs) for the largest products, and 128 x 128 tiles (waves of 64 x 64,
-// two workgroups per CU, accumulators in VGPRs) for the others. The stage layouts are those of
-// dlds_tile_at (k-step 8, a 3-stage direct-to-LDS ring; (128 + BN) x 64 bytes per stage).
+// two workgroups per CU, accumulators in VGPRs) for the others. Operands come by direct
+// global->LDS loads of 16 bytes into a 3-stage ring, k-step 8, (128 + BN) x 64 bytes per stage: no
+// registers or ds_write instructions carry them.
 // With one or two waves per SIMD little hides a stall, so the loop is pipelined by hand: the
 // fragments of stage kt+1 are read into a second register set while the 2 x 4 x BN/32 MFMAs of
 // stage kt run, the loads of stage kt+3 go between the first MFMAs, and scheduling-group barriers
@@ -1271,8 +1104,11 @@ struct BigOperand {
   const double* base[PER_WAVE];
   int dst[PER_WAVE];
   long kstride;  // elements per step of k: 1 (k-contiguous) or ld (row-contiguous)
-  // k-contiguous: instruction i fills rows 16i..16i+15 (64 bytes each, slots XOR-permuted as in
-  // DldsOperand); row-contiguous: instruction i fills the 128 rows (i % P) * 128.. at k = i / P,
+  __device__ __forceinline__ static int kc_swz(int r) { return (r >> 1) & 3; }
+  // k-contiguous: LDS [row][slot], a 16-byte chunk = 2 consecutive k of one row, chunk q of row r in
+  // slot q ^ kc_swz(r): the fragment read of one k pair by 16 consecutive rows then touches 8
+  // distinct 16-byte bank groups per 8 lanes (rows r, r+1 share a swizzle and sit 64 bytes apart).
+  // Instruction i fills rows 16i..16i+15, 64 contiguous bytes of each. Row-contiguous: instruction i fills the 128 rows (i % P) * 128.. at k = i / P,
   // P = ROWS / 128, 2 rows per lane (of an odd row count the last lane's second row is the next
   // column's first, or padding: see ring_steps).
   __device__ __forceinline__ BigOperand(const double* p, long ld, int r0, int nrows, int wave, int lane) {
@@ -1282,7 +1118,7 @@ struct BigOperand {
       const int inst = wave * PER_WAVE + t;
       if (KC) {
         const int local = inst * 16 + (lane >> 2);
-        const int q = (lane & 3) ^ DldsOperand<true>::kc_swz(local);
+        const int q = (lane & 3) ^ kc_swz(local);
         base[t] = p + 2 * q + (long)min(r0 + local, nrows - 1) * ld;
         dst[t] = inst * 128;
       } else {
@@ -1302,7 +1138,7 @@ struct BigOperand {
   // stage offset (doubles) of row `row`'s values at k = 2g, 2g+1 (row-contiguous: the second one
   // ROWS further)
   __device__ __forceinline__ static int frag_off(int row, int g) {
-    return KC ? row * 8 + (g ^ DldsOperand<true>::kc_swz(row)) * 2 : 2 * g * ROWS + row;
+    return KC ? row * 8 + (g ^ kc_swz(row)) * 2 : 2 * g * ROWS + row;
   }
   __device__ __forceinline__ static v2d frag(const double* stage, int off) {
     if (KC) return *(const v2d*)(stage + off);
@@ -1543,7 +1379,7 @@ __global__ __launch_bounds__(256, 2) void gemm_c_pipe_group_kernel(SgemmGroup g)
 
 // ---------------------------------------------------------------------------------------------
 // Complex FP64 GEMM with direct global->LDS loads (ZGEMM), the complex sibling of
-// dlds_tile_at. WG tile 64x64 complex, 2x2 waves of 32x32 (2x2 blocks, re and im
+// BigOperand. WG tile 64x64 complex, 2x2 waves of 32x32 (2x2 blocks, re and im
 // accumulators, four real MFMAs per block update), k-step 8 complex per stage, a 3-stage ring of
 // 16 KB stages. A 16-byte chunk is one complex element, so one
 // ds_read_b128 yields both MFMA operands (re, im) of a lane.
@@ -2052,17 +1888,10 @@ hipError_t launch_gemm_c_group(const GemmParams<float>* tiles, int count, hipStr
 
 hipError_t launch_gemm_d_batched(char opa, char opb, const GemmParams<double>* probs, const int* items, int n_items,
                                  int* counter, int n_workgroups, hipStream_t s, int body) {
-  hipLaunchKernelGGL(zero_counter_kernel, dim3(1), dim3(64), 0, s, counter);
-  if (n_items <= 0) return hipGetLastError();
+  if (n_items <= 0) return hipSuccess;
+  if (body == 1) return launch_ks_d_batched(opa, opb, probs, items, n_items, counter, n_workgroups, s);
   dim3 grid(n_workgroups), block(256);
   const bool akc = is_kc_a(opa), bkc = is_kc_b(opb);
-  if (body == 1) {
-    if (akc && bkc) hipLaunchKernelGGL((gemm_d_dlds_batched_kernel<true, true, 3>), grid, block, 0, s, probs, items, n_items, counter);
-    else if (akc) hipLaunchKernelGGL((gemm_d_dlds_batched_kernel<true, false, 3>), grid, block, 0, s, probs, items, n_items, counter);
-    else if (bkc) hipLaunchKernelGGL((gemm_d_dlds_batched_kernel<false, true, 3>), grid, block, 0, s, probs, items, n_items, counter);
-    else hipLaunchKernelGGL((gemm_d_dlds_batched_kernel<false, false, 3>), grid, block, 0, s, probs, items, n_items, counter);
-    return hipGetLastError();
-  }
   if (akc && bkc) hipLaunchKernelGGL((gemm_real_batched_kernel<double, true, true>), grid, block, 0, s, probs, items, n_items, counter);
   else if (akc) hipLaunchKernelGGL((gemm_real_batched_kernel<double, true, false>), grid, block, 0, s, probs, items, n_items, counter);
   else if (bkc) hipLaunchKernelGGL((gemm_real_batched_kernel<double, false, true>), grid, block, 0, s, probs, items, n_items, counter);

@@ -67,10 +67,11 @@ bool cgemm_groupable(const GemmParams<float>& p);
 hipError_t launch_gemm_c_group(const GemmParams<float>* tiles, int count, hipStream_t s);
 
 // Persistent batched FP64 GEMM over device-resident problems (all with the same op flags):
-// items = n_items triples (problem index, tile row, tile column) of 128x128 C tiles; counter is
-// one device int, zeroed by a kernel at the start of the launch sequence (graph-capturable).
-// body 0: register-staged LDS double buffer; 1: direct-to-LDS ring, which needs every operand in
-// a device arena with at least 16 readable bytes after its last column.
+// items = n_items triples (problem index, tile row, tile column) of C tiles of batched_tile(body)
+// rows and columns; counter is one device int that holds 0 at launch. body 0: register-staged LDS
+// double buffer; 1: direct-to-LDS rings with the inner dimension split over the waves, for leading
+// dimensions of up to 256 MB.
+inline int batched_tile(int body) { return body == 1 ? 64 : 128; }
 hipError_t launch_gemm_d_batched(char opa, char opb, const GemmParams<double>* probs, const int* items, int n_items,
                                  int* counter, int n_workgroups, hipStream_t s, int body);
 

@@ -123,5 +123,8 @@ TMM_KS_DECLARE(s, float)
 TMM_KS_DECLARE(z, double)
 TMM_KS_DECLARE(c, float)
 #undef TMM_KS_DECLARE
+// A batch of products as launch_gemm_d_batched describes it, in 64 x 64 tiles.
+hipError_t launch_ks_d_batched(char opa, char opb, const GemmParams<double>* probs, const int* items, int n_items,
+                               int* counter, int n_workgroups, hipStream_t s);
 
 }  // namespace tmm

@@ -18,4 +18,15 @@ hipError_t launch_ks_d_group(const GemmParams<double>* tiles, int count, hipStre
   return ks::launch_group<ks::TypeD, 4, 4, 2>(tiles, count, s);
 }
 
+hipError_t launch_ks_d_batched(char opa, char opb, const GemmParams<double>* probs, const int* items, int n_items,
+                               int* counter, int n_workgroups, hipStream_t s) {
+  const dim3 grid(std::min(n_items, n_workgroups)), block(256);
+  const bool akc = opa != 'N', bkc = opb == 'N';
+  if (akc && bkc) hipLaunchKernelGGL((ks::gemm_ks_batched_kernel<ks::TypeD, true, true, 4, 4, 2>), grid, block, 0, s, probs, items, n_items, counter);
+  else if (akc) hipLaunchKernelGGL((ks::gemm_ks_batched_kernel<ks::TypeD, true, false, 4, 4, 2>), grid, block, 0, s, probs, items, n_items, counter);
+  else if (bkc) hipLaunchKernelGGL((ks::gemm_ks_batched_kernel<ks::TypeD, false, true, 4, 4, 2>), grid, block, 0, s, probs, items, n_items, counter);
+  else hipLaunchKernelGGL((ks::gemm_ks_batched_kernel<ks::TypeD, false, false, 4, 4, 2>), grid, block, 0, s, probs, items, n_items, counter);
+  return hipGetLastError();
+}
+
 }  // namespace tmm
