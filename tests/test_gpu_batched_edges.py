@@ -50,6 +50,39 @@ def test_batched_tile_edges_exact(torch_gpu, flags):
         assert np.isnan(out[m:]).all()
 
 
+@pytest.mark.parametrize("graph", [0, 1])
+@pytest.mark.parametrize("pad,shift", [(0, 0), (0, 1), (1, 0), (2, 1)])
+def test_batched_copies_exact(torch_gpu, pad, shift, graph):
+    """Matrices on both sides of the size that one kernel copies, of the 4096 elements of its pieces,
+    and of 16-byte alignment; contiguous and padded; nothing beyond the matrices is written."""
+    rng = np.random.default_rng(22)
+    sizes = [(362, 362, 362), (363, 362, 361), (1, 1, 1), (64, 64, 64), (4095, 3, 5), (4096, 2, 3), (4097, 3, 2),
+             (3, 4099, 2), (17, 9, 4101)]
+
+    def stored(x):
+        flat = tiledmm.pinned_empty((shift + (x.shape[0] + pad) * x.shape[1] + 1,), np.float64)
+        flat[...] = np.nan
+        out = flat[shift:-1].reshape((x.shape[0] + pad, x.shape[1]), order="F")
+        out[:x.shape[0]] = x
+        return flat, out
+
+    mats = [[rng.integers(-9, 10, s).astype(float) for s in ((m, k), (k, n), (m, n))] for m, n, k in sizes]
+    held = [[stored(x) for x in group] for group in mats]
+    A, B, C = ([group[j][1] for group in held] for j in range(3))
+    ms, ns, ks = zip(*sizes)
+    count = len(sizes)
+    with tiledmm.Handle(tiledmm.F64, 2) as h:
+        h.set_option(tiledmm.OPT_BATCH_GRAPH, graph)
+        for _ in range(2):  # the second call reads the C that the first one left
+            h.gemm_batched("N", "N", ms, ns, ks, [1.0] * count, A, [x.shape[0] for x in A], B,
+                           [x.shape[0] for x in B], [1.0] * count, C, [x.shape[0] for x in C])
+        assert h.stats()["batch_graph"] == graph
+    for (a, b, c), group, size in zip(mats, held, sizes):
+        flat, out = group[2]
+        np.testing.assert_array_equal(out[:size[0]], 2 * (a @ b) + c, err_msg=str(size))
+        assert np.isnan(out[size[0]:]).all() and np.isnan(flat[:shift]).all() and np.isnan(flat[-1])
+
+
 def test_batched_long_columns_take_the_other_body(torch_gpu):
     """Columns of more than 256 MB are beyond the direct-to-LDS body's 32-bit lane offsets: the batch
     runs on the register-staged one. Ones and twos: the sum is exact."""

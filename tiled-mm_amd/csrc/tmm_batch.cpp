@@ -4,10 +4,10 @@
 // Tiled-MM src/Tiled-MM/tiled_mm.cpp:492-624, each with its own tiling, copies and a
 // device-wide synchronisation). Here the whole batch is one pipeline:
 //   * the problems are packed into one device arena and cut into G groups of about equal
-//     host-link bytes; group g's H2D copies (spread over two copy queues), one persistent
-//     batched-kernel launch over all C tiles of the group (largest k first), and its D2H copies run
-//     on their own queues, so H2D of group g+1 overlaps the kernel of group g and the D2H of group
-//     g-1;
+//     host-link bytes; group g's H2D copies (small matrices by one kernel, large ones spread over
+//     two copy queues), one persistent batched-kernel launch over all C tiles of the group (largest
+//     k first), and its D2H copies run on their own queues, so H2D of group g+1 overlaps the kernel
+//     of group g and the D2H of group g-1;
 //   * with pinned host matrices the whole sequence is captured once into a hipGraph and
 //     launched as one graph (no per-problem launch overhead);
 //   * G, the persistent grid, the tile body (register-staged or direct-to-LDS), the compute
@@ -33,9 +33,20 @@ struct Prob {
   const double* b;
   double* c;
   double alpha, beta;
+  void *map_a = nullptr, *map_b = nullptr, *map_c = nullptr;  // a, b, c on the device if a kernel copies them
   size_t offA, offB, offC;  // arena offsets (elements)
   long rowsA, colsA, rowsB, colsB;
 };
+
+// Page-locked matrices of up to this size are copied by one kernel per group and direction
+// (tmm_copy.hip; its workgroups), larger ones by a DMA command each: below it the command's 10 us
+// outweigh the transfer, above it a kernel's reads over the link slow the tile kernels beside it
+// (their loads wait behind them in the L2; 0.27 ms for a group became 0.5). Calls in us with no
+// kernel copies / up to 256 KB / 1 MB / 4 MB: 48 problems of 64 to 1024 rows and columns 2350 / 2377 /
+// 2284 / 2756, 90 of 64 to 700 with padded columns 4707 / 3870 / 3048 / 3154, 300 of 16 to 128 6620 /
+// 1547 / 1518 / 1519, 200 of 64 to 3000 37770 / 37862 / 37385 / 37880.
+constexpr size_t kKernelCopyBytes = 1u << 20;
+constexpr int kCopyInWorkgroups = 64, kCopyOutWorkgroups = 32;
 
 }  // namespace
 
@@ -98,15 +109,22 @@ void gemm_batched_host(Handle& h, char opa, char opb, int count, const int* m, c
 
   // pinned detection for every matrix: the graph path needs all of them pinned
   bool all_pinned = true;
-  for (const Prob& p : P) {
+  for (Prob& p : P) {
     auto span = [](long rows, long cols, long ld) -> size_t {
       return rows == 0 || cols == 0 ? 0 : (size_t)((cols - 1) * ld + rows) * 8;
     };
-    all_pinned = all_pinned && is_pinned_range(p.a, span(p.rowsA, p.colsA, p.lda)) &&
-                 is_pinned_range(p.b, span(p.rowsB, p.colsB, p.ldb)) && is_pinned_range(p.c, span(p.m, p.n, p.ldc));
+    all_pinned = all_pinned && is_pinned_range(p.a, span(p.rowsA, p.colsA, p.lda), &p.map_a) &&
+                 is_pinned_range(p.b, span(p.rowsB, p.colsB, p.ldb), &p.map_b) &&
+                 is_pinned_range(p.c, span(p.m, p.n, p.ldc), &p.map_c);
     if (!all_pinned) break;
   }
   shape.pinned = all_pinned;
+  for (Prob& p : P) {  // only the matrices that a kernel copies keep their device address
+    auto small = [&](long rows, long cols) { return rows > 0 && cols > 0 && (size_t)rows * cols * 8 <= kKernelCopyBytes; };
+    if (!all_pinned || !small(p.rowsA, p.colsA)) p.map_a = nullptr;
+    if (!all_pinned || !small(p.rowsB, p.colsB)) p.map_b = nullptr;
+    if (!all_pinned || !small(p.m, p.n)) p.map_c = nullptr;
+  }
   BatchConfig cfg = choose_batch_config(h, shape);
   cfg.queues = std::max(1, std::min(cfg.queues, (int)h.compute.size()));
   // emulated problems: one workspace per compute queue (groups alternate over the queues),
@@ -177,24 +195,61 @@ void gemm_batched_host(Handle& h, char opa, char opb, int count, const int* m, c
     d.c = dev + p.offC;
     d.ldc = std::max(1, p.m);
   }
-  // descriptors, work items and the groups' zeroed item counters in one upload
+  // the groups' kernel copies: H2D items from in_start[g] on, D2H items from out_start[g] on
+  std::vector<CopyItem> copies;
+  std::vector<int> in_start(G + 1, 0), out_start(G + 1, 0);
+  auto add_copies = [&](const double* src, long ld_src, double* dst, long ld_dst, long rows, long cols) {
+    if (ld_src == rows && ld_dst == rows) {  // contiguous: one long column
+      const long n = rows * cols;
+      for (long e = 0; e < n; e += kCopyItemElems) {
+        const int len = (int)std::min(kCopyItemElems, n - e);
+        copies.push_back(CopyItem{src + e, dst + e, len, len, len, 1});
+      }
+      return;
+    }
+    const long nr = std::min(rows, kCopyItemElems), nc = std::max(1L, kCopyItemElems / nr);
+    for (long c = 0; c < cols; c += nc)
+      for (long r = 0; r < rows; r += nr)
+        copies.push_back(CopyItem{src + r + c * ld_src, dst + r + c * ld_dst, ld_src, ld_dst,
+                                  (int)std::min(nr, rows - r), (int)std::min(nc, cols - c)});
+  };
+  for (int g = 0; g < G; ++g) {
+    in_start[g] = (int)copies.size();
+    for (int i = gstart[g]; i < gstart[g + 1]; ++i) {
+      const Prob& p = P[i];
+      if (p.map_a) add_copies((const double*)p.map_a, p.lda, dev + p.offA, p.rowsA, p.rowsA, p.colsA);
+      if (p.map_b) add_copies((const double*)p.map_b, p.ldb, dev + p.offB, p.rowsB, p.rowsB, p.colsB);
+      if (p.map_c && p.beta != 0.0) add_copies((const double*)p.map_c, p.ldc, dev + p.offC, p.m, p.m, p.n);
+    }
+    out_start[g] = (int)copies.size();
+    for (int i = gstart[g]; i < gstart[g + 1]; ++i) {
+      const Prob& p = P[i];
+      if (p.map_c) add_copies(dev + p.offC, p.m, (double*)p.map_c, p.ldc, p.m, p.n);
+    }
+  }
+  in_start[G] = (int)copies.size();
+
+  // descriptors, work items, copy items and the groups' zeroed item counters in one upload
   std::vector<size_t> item_off(G + 1, 0);
   for (int g = 0; g < G; ++g) item_off[g + 1] = item_off[g] + items[g].size();
   auto align256 = [](size_t b) { return (b + 255) & ~(size_t)255; };
   const size_t at_items = align256(sizeof(GemmParams<double>) * count);
-  const size_t at_counters = align256(at_items + item_off[G] * sizeof(int)), meta_bytes = at_counters + 64 * (size_t)G;
-  h.batch_meta.reserve(meta_bytes);
+  const size_t at_copies = align256(at_items + item_off[G] * sizeof(int));
+  const size_t at_counters = align256(at_copies + copies.size() * sizeof(CopyItem));
+  h.batch_meta.reserve(at_counters + 64 * (size_t)G);
   char* meta = (char*)h.batch_meta.ptr;
   GemmParams<double>* d_desc = (GemmParams<double>*)meta;
   int* d_items = (int*)(meta + at_items);
+  const CopyItem* d_copies = (const CopyItem*)(meta + at_copies);
   int* d_counters = (int*)(meta + at_counters);
   {
-    std::vector<char> flat(meta_bytes);
+    std::vector<char> flat(at_counters + 64 * (size_t)G);
     std::memcpy(flat.data(), desc.data(), sizeof(GemmParams<double>) * count);
     for (int g = 0; g < G; ++g)
       if (!items[g].empty())
         std::memcpy(flat.data() + at_items + item_off[g] * sizeof(int), items[g].data(), items[g].size() * sizeof(int));
-    hip_check(hipMemcpy(meta, flat.data(), meta_bytes, hipMemcpyHostToDevice), "hipMemcpy");
+    if (!copies.empty()) std::memcpy(flat.data() + at_copies, copies.data(), copies.size() * sizeof(CopyItem));
+    hip_check(hipMemcpy(meta, flat.data(), flat.size(), hipMemcpyHostToDevice), "hipMemcpy");
   }
 
   hipStream_t sh = h.h2d, sd = h.d2h;
@@ -215,12 +270,14 @@ void gemm_batched_host(Handle& h, char opa, char opb, int count, const int* m, c
                 "batched Ozaki (CRT) product");
     }
   };
-  // H2D copies go to two copy queues, each copy to the one with fewer bytes issued so far in this
-  // call: a DMA command carries a fixed cost of several microseconds, and with two queues one
+  // DMA H2D copies go to two copy queues, each copy to the one with fewer bytes issued so far in this
+  // call: a DMA command carries a fixed cost of some 10 us, and with two queues one
   // queue's transfer covers the other's. The 512-problem batch (m, n, k log-uniform in [64, 4096],
   // 1536 H2D copies of 4 KB - 130 MB, 64 groups) ran 232-234 ms per call with one H2D queue, 213 ms
   // with two balanced by bytes; a third queue, or a second D2H queue, ran slower.
-  hipStream_t sh2 = h.h2d_aux_stream();
+  bool dma_in = false;
+  for (const Prob& p : P) dma_in = dma_in || !p.map_a || !p.map_b || (p.beta != 0.0 && !p.map_c);
+  hipStream_t sh2 = dma_in ? h.h2d_aux_stream() : sh;
   std::vector<hipEvent_t> ev_in(G), ev_in2(G), ev_k(G);
   for (int g = 0; g < G; ++g) {
     ev_in[g] = h.event(3 * g);
@@ -248,12 +305,12 @@ void gemm_batched_host(Handle& h, char opa, char opb, int count, const int* m, c
          q ? sh2 : sh);
   };
   auto h2d = [&](const Prob& p) {
-    h2d_copy(dev + p.offA, p.a, p.rowsA, p.colsA, p.lda);
-    h2d_copy(dev + p.offB, p.b, p.rowsB, p.colsB, p.ldb);
-    if (p.beta != 0.0) h2d_copy(dev + p.offC, p.c, p.m, p.n, p.ldc);
+    if (!p.map_a) h2d_copy(dev + p.offA, p.a, p.rowsA, p.colsA, p.lda);
+    if (!p.map_b) h2d_copy(dev + p.offB, p.b, p.rowsB, p.colsB, p.ldb);
+    if (p.beta != 0.0 && !p.map_c) h2d_copy(dev + p.offC, p.c, p.m, p.n, p.ldc);
   };
   auto d2h = [&](const Prob& p, hipStream_t s) {
-    if (p.m && p.n)
+    if (p.m && p.n && !p.map_c)
       copy(p.c, (size_t)p.ldc * 8, dev + p.offC, (size_t)p.m * 8, (size_t)p.m * 8, (size_t)p.n, hipMemcpyDeviceToHost,
            s);
   };
@@ -262,18 +319,25 @@ void gemm_batched_host(Handle& h, char opa, char opb, int count, const int* m, c
     hip_check(hipEventRecord(ev_fork, sh), "hipEventRecord");
     for (hipStream_t q : scs) hip_check(hipStreamWaitEvent(q, ev_fork, 0), "hipStreamWaitEvent");
     hip_check(hipStreamWaitEvent(sd, ev_fork, 0), "hipStreamWaitEvent");
-    hip_check(hipStreamWaitEvent(sh2, ev_fork, 0), "hipStreamWaitEvent");
+    if (dma_in) hip_check(hipStreamWaitEvent(sh2, ev_fork, 0), "hipStreamWaitEvent");
     issued[0] = issued[1] = 0;
     for (int g = 0; g < G; ++g) {
       hipStream_t sg = scs[g % cfg.queues];
+      hip_check(launch_copy_items(d_copies + in_start[g], out_start[g] - in_start[g], kCopyInWorkgroups, sh),
+                "batched H2D copy launch");
       for (int i = gstart[g]; i < gstart[g + 1]; ++i) h2d(P[i]);
       hip_check(hipEventRecord(ev_in[g], sh), "hipEventRecord");
-      hip_check(hipEventRecord(ev_in2[g], sh2), "hipEventRecord");
       hip_check(hipStreamWaitEvent(sg, ev_in[g], 0), "hipStreamWaitEvent");
-      hip_check(hipStreamWaitEvent(sg, ev_in2[g], 0), "hipStreamWaitEvent");
+      if (dma_in) {
+        hip_check(hipEventRecord(ev_in2[g], sh2), "hipEventRecord");
+        hip_check(hipStreamWaitEvent(sg, ev_in2[g], 0), "hipStreamWaitEvent");
+      }
       compute_group(g, sg);
       hip_check(hipEventRecord(ev_k[g], sg), "hipEventRecord");
       hip_check(hipStreamWaitEvent(sd, ev_k[g], 0), "hipStreamWaitEvent");
+      hip_check(launch_copy_items(d_copies + out_start[g], in_start[g + 1] - out_start[g], kCopyOutWorkgroups,
+                                  sd),
+                "batched D2H copy launch");
       for (int i = gstart[g]; i < gstart[g + 1]; ++i) d2h(P[i], sd);
     }
     // join back into the H2D queue
@@ -283,8 +347,10 @@ void gemm_batched_host(Handle& h, char opa, char opb, int count, const int* m, c
     }
     hip_check(hipEventRecord(ev_join_d, sd), "hipEventRecord");
     hip_check(hipStreamWaitEvent(sh, ev_join_d, 0), "hipStreamWaitEvent");
-    hip_check(hipEventRecord(ev_join_h2, sh2), "hipEventRecord");
-    hip_check(hipStreamWaitEvent(sh, ev_join_h2, 0), "hipStreamWaitEvent");
+    if (dma_in) {
+      hip_check(hipEventRecord(ev_join_h2, sh2), "hipEventRecord");
+      hip_check(hipStreamWaitEvent(sh, ev_join_h2, 0), "hipStreamWaitEvent");
+    }
   };
 
   if (all_pinned && cfg.use_graph) {

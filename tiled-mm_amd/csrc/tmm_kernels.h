@@ -75,4 +75,16 @@ inline int batched_tile(int body) { return body == 1 ? 64 : 128; }
 hipError_t launch_gemm_d_batched(char opa, char opb, const GemmParams<double>* probs, const int* items, int n_items,
                                  int* counter, int n_workgroups, hipStream_t s, int body);
 
+// Part of a column-major matrix to copy (doubles): rows x cols, at most kCopyItemElems elements.
+struct CopyItem {
+  const double* src;
+  double* dst;
+  long ld_src, ld_dst;
+  int rows, cols;
+};
+constexpr long kCopyItemElems = 4096;
+// Copy n items (a device array) with at most `workgroups` workgroups; source and destination may be
+// page-locked host memory, by its device pointer.
+hipError_t launch_copy_items(const CopyItem* items, int n, int workgroups, hipStream_t s);
+
 }  // namespace tmm

@@ -149,9 +149,11 @@ void StagingRing::release() {
   next = 0;
 }
 
-bool is_pinned_range(const void* p, size_t bytes) {
+bool is_pinned_range(const void* p, size_t bytes, void** device_ptr) {
+  if (device_ptr) *device_ptr = nullptr;
   if (!p || bytes == 0) return true;
-  auto pinned_at = [](const void* q, void** devp) {
+  int owner = -1;
+  auto pinned_at = [&](const void* q, void** devp) {
     hipPointerAttribute_t at;
     hipError_t e = hipPointerGetAttributes(&at, q);
     if (e != hipSuccess) {
@@ -160,13 +162,20 @@ bool is_pinned_range(const void* p, size_t bytes) {
     }
     if (at.type != hipMemoryTypeHost) return false;
     *devp = at.devicePointer;
+    owner = at.device;
     return true;
   };
   void *d0 = nullptr, *d1 = nullptr;
   const char* last = (const char*)p + bytes - 1;
   if (!pinned_at(p, &d0) || !pinned_at(last, &d1)) return false;
   // both ends must map into one allocation with the same offset
-  return (const char*)d1 - (const char*)d0 == (ptrdiff_t)(bytes - 1);
+  if ((const char*)d1 - (const char*)d0 != (ptrdiff_t)(bytes - 1)) return false;
+  if (device_ptr) {
+    int current = 0;
+    hip_check(hipGetDevice(&current), "hipGetDevice");
+    if (owner == current) *device_ptr = d0;
+  }
+  return true;
 }
 
 // ------------------------------------------------------------------------------------------

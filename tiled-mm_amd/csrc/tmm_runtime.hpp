@@ -213,6 +213,7 @@ BatchConfig choose_batch_config(Handle& h, const BatchShape& shape);
 void calibrate_rates(Handle& h);
 
 // True when the whole byte range [p, p+bytes) lies in one pinned (page-locked) allocation.
-bool is_pinned_range(const void* p, size_t bytes);
+// *device_ptr (when not null): p's address on the current device, null if the memory belongs to another.
+bool is_pinned_range(const void* p, size_t bytes, void** device_ptr = nullptr);
 
 }  // namespace tmm
