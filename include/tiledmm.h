@@ -124,13 +124,17 @@ const char* tmm_last_error(tmm_handle* h);
 
 /* Device-resident tile GEMM, the per-tile kernel on its own: replaces the vendor BLAS call
  * cublas_gemm_wrapper -> {s,d,c,z}gemm (tiled_mm.cpp:181-268). All pointers are device
- * pointers; stream = NULL runs on the handle's first compute stream. Asynchronous. */
+ * pointers; stream = NULL runs on the handle's first compute stream. Asynchronous. A product with
+ * a small C and a long inner dimension adds up partial sums in a buffer of up to 20 MB that the handle
+ * allocates at the first one: such calls of one handle run one after the other, whatever their
+ * streams (under stream capture they take neither the buffer nor the faster kernels). */
 int tmm_device_gemm(tmm_handle* h, char trans_a, char trans_b, int m, int n, int k, const void* alpha,
                     const void* a, int ld_a, const void* b, int ld_b, const void* beta, void* c, int ld_c,
                     void* stream);
 /* tmm_device_gemm without any device allocation. No counterpart in the reference: for callers
  * that cannot allocate (code under HIP graph capture, tight serving loops, harnesses that forbid
- * hipMalloc). Same arguments, semantics and kernels as tmm_device_gemm; with an Ozaki option the
+ * hipMalloc). Same arguments and semantics as tmm_device_gemm, and its kernels but for those that
+ * add up partial sums in a buffer; with an Ozaki option the
  * emulation works in a fixed scratch array of TMM_NOALLOC_SCRATCH_BYTES (256 MiB) that the
  * library holds on every device it runs on until the process ends (its address is looked up by
  * tmm_create) instead of the handle's workspace. A product whose workspace would exceed it is

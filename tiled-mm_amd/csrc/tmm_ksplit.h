@@ -112,12 +112,61 @@ bool ks_takes(const GemmParams<R>& p, bool cplx) {
          ks_chunks_ok<R>(cplx, p.opa != 'N', p.m, p.lda) && ks_chunks_ok<R>(cplx, p.opb == 'N', p.n, p.ldb);
 }
 
+// A product whose tiles are shared by several workgroups ("parts"), for a C of fewer tiles than the
+// CUs take and a long inner dimension: without the split most CUs idle (500 x 600 in 32 x 48 tiles: 208
+// for 256 CUs, and a fifth of each stage beside its MFMAs) or a few run alone. Each part's m x n sums
+// go through device memory, and a second kernel adds them: about 5.5 us for the two launches and the
+// events that order the buffer, and 2.5 MB of sums per us. (Adding them up in the last workgroup of a
+// tile to arrive, in one launch, took 20 to 150 us more: one workgroup reads a tile's sums.)
+// Unsplit -> split in us: DGEMM TN 500 x 600 x 40000 478 -> 397, NN 32 x 32 x 20000 64 -> 10, TN 100 x
+// 100 x 10000 33 -> 14, NT 300 x 700 x 15000 135 -> 111; SGEMM TN 500 x 600 x 40000 247 -> 212; ZGEMM NN
+// 500 x 300 x 10000 312 -> 237 (210 in 32 x 32 tiles), CN 200 x 200 x 5000 55 -> 41.
+constexpr int kSplitShapes[4] = {0, 3, 6, 11};  // 16 x 16, 32 x 32, 48 x 48, 64 x 64 (the real types)
+constexpr long kSplitMaxWorkgroups = 512;
+// Bytes that the sums of every split product of the type fit in.
+inline size_t split_bytes(KsType t) {
+  const size_t es[4] = {8, 4, 16, 8};
+  const size_t edge = t <= KsType::S ? 64 : 48;
+  return kSplitMaxWorkgroups * edge * edge * es[(int)t];
+}
+struct SplitPlan {
+  int shape, parts;  // parts < 2: not split
+};
+// The fastest split of an m x n x k product where the model gives it a lead of 4.5 us (it is that far
+// out for an unsplit product of a few small tiles: SGEMM TN 64 x 64 x 4000 runs in 8.4 us unsplit, not
+// 13.2, and 9.6 split); one or two workgroups per CU (one leaves its waits uncovered: 3%), and 8 stages
+// at least for every wave.
+inline SplitPlan split_plan(KsType t, long m, long n, long k, int cus) {
+  SplitPlan best = {0, 1};
+  const KsCost& c = kKsCost[(int)t];
+  const double es[4] = {8, 4, 16, 8};
+  if (k < 64 * c.bk) return best;
+  double least = product_time(t, m, n, k, cus) - 4.5;
+  for (int shape : kSplitShapes) {
+    if (shape >= kKsShapeCount[(int)t]) continue;
+    const KsShape s = kKsShapes[shape];
+    const long tiles = ks_tiles(s, m, n);
+    for (long slots : {2L * cus, (long)cus}) {
+      const long parts = std::min({slots / tiles, kSplitMaxWorkgroups / tiles, k / (32 * c.bk)});
+      if (parts < 2) continue;
+      const double us = ks_time(t, s, tiles * parts, (k + parts - 1) / parts, cus) * (tiles * parts <= cus ? 1.03 : 1) +
+                        5.5 + parts * m * n * es[(int)t] / 2.5e6;
+      if (us < least) {
+        least = us;
+        best = {shape, (int)parts};
+      }
+    }
+  }
+  return best;
+}
+
 // One product on the given shape (an index of kKsShapes), or a group of products with one op pair,
 // alpha and k in one launch; every product must satisfy ks_takes. The result does not depend on
 // the shape, nor on the grouping.
 #define TMM_KS_DECLARE(t, R)                                                   \
   hipError_t launch_ks_##t(const GemmParams<R>& p, int shape, hipStream_t s); \
-  hipError_t launch_ks_##t##_group(const GemmParams<R>* tiles, int count, hipStream_t s);
+  hipError_t launch_ks_##t##_group(const GemmParams<R>* tiles, int count, hipStream_t s); \
+  hipError_t launch_ks_##t##_split(const GemmParams<R>& p, int shape, int parts, void* ws, hipStream_t s);
 TMM_KS_DECLARE(d, double)
 TMM_KS_DECLARE(s, float)
 TMM_KS_DECLARE(z, double)

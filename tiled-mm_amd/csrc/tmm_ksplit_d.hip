@@ -29,4 +29,12 @@ hipError_t launch_ks_d_batched(char opa, char opb, const GemmParams<double>* pro
   return hipGetLastError();
 }
 
+hipError_t launch_ks_d_split(const GemmParams<double>& p, int shape, int parts, void* ws, hipStream_t s) {
+  if (shape == kSplitShapes[0]) return ks::launch_split<ks::TypeD, 1, 1, 4>(p, parts, ws, s);
+  if (shape == kSplitShapes[1]) return ks::launch_split<ks::TypeD, 2, 2, 2>(p, parts, ws, s);
+  if (shape == kSplitShapes[2]) return ks::launch_split<ks::TypeD, 3, 3, 2>(p, parts, ws, s);
+  if (shape == kSplitShapes[3]) return ks::launch_split<ks::TypeD, 4, 4, 2>(p, parts, ws, s);
+  return hipErrorInvalidValue;
+}
+
 }  // namespace tmm

@@ -245,9 +245,18 @@ struct Geometry {
   static constexpr int LDS = RING > JP * COLS16 ? RING : JP * COLS16;
 };
 
-// The C tile at (m0, n0). conj_a / conj_b: negate the imaginary part (op 'C').
-template <typename T, bool A_KC, bool B_KC, int WBM, int WBN, int S>
-__device__ __forceinline__ void tile_at(const GemmParams<typename T::R>& prm, bool conj_a, bool conj_b, int m0, int n0) {
+// A workgroup's share of the inner dimension of a product that is split over workgroups as well.
+template <typename R>
+struct Part {
+  int index, count;
+  R* sums;  // this share's m x n sums, without alpha, beta and C
+};
+
+// The C tile at (m0, n0). conj_a / conj_b: negate the imaginary part (op 'C'). SPLIT: the
+// tile's sums over share part.index of the inner dimension, to part.sums.
+template <typename T, bool A_KC, bool B_KC, int WBM, int WBN, int S, bool SPLIT = false>
+__device__ __forceinline__ void tile_at(const GemmParams<typename T::R>& prm, bool conj_a, bool conj_b, int m0, int n0,
+                                        const Part<typename T::R>& part = {}) {
   typedef typename T::R R;
   typedef Geometry<T, WBM, WBN, S> G;
   typedef Operand<T, A_KC, WBM> OpA;
@@ -263,7 +272,9 @@ __device__ __forceinline__ void tile_at(const GemmParams<typename T::R>& prm, bo
   t.zero();
   // stages read through the ring, and the k range of the step read element by element
   const bool ragged = K % BK != 0 || (!A_KC && M % OpA::KV != 0) || (!B_KC && N % OpB::KV != 0);
-  const int nfull = ragged ? (K - 1) / BK : K / BK;
+  const int nall = ragged ? (K - 1) / BK : K / BK;
+  const int first = SPLIT ? (int)((long)nall * part.index / part.count) : 0;
+  const int nfull = SPLIT ? (int)((long)nall * (part.index + 1) / part.count) - first : nall;
   const int ns = nfull > wave ? (nfull - wave + 3) / 4 : 0;
 
   auto conj = [&](typename TileT::Frags& f) {
@@ -282,8 +293,8 @@ __device__ __forceinline__ void tile_at(const GemmParams<typename T::R>& prm, bo
 
   OpA oa;
   OpB ob;
-  oa.setup(prm.a, prm.lda, m0, M, wave, 4, lane);
-  ob.setup(prm.b, prm.ldb, n0, N, wave, 4, lane);
+  oa.setup(prm.a, prm.lda, m0, M, first + wave, 4, lane);
+  ob.setup(prm.b, prm.ldb, n0, N, first + wave, 4, lane);
   char* ring = lds + wave * (S * G::STAGE);
   auto issue = [&](int slot) {
     oa.issue(ring + slot * G::STAGE);
@@ -297,12 +308,12 @@ __device__ __forceinline__ void tile_at(const GemmParams<typename T::R>& prm, bo
     for (int j = 0; j < WBN; ++j) f.b[j] = OpB::frag(st + WBM * 1024, j, li, lg);
   };
 
-  if (ragged && (nfull & 3) == wave) {
+  if (ragged && (nfull & 3) == wave && (!SPLIT || part.index == part.count - 1)) {
     typename TileT::Frags f;
 #pragma unroll
-    for (int i = 0; i < WBM; ++i) f.a[i] = OpA::frag_global(prm.a, prm.lda, m0, M, nfull * BK, K, i, li, lg);
+    for (int i = 0; i < WBM; ++i) f.a[i] = OpA::frag_global(prm.a, prm.lda, m0, M, nall * BK, K, i, li, lg);
 #pragma unroll
-    for (int j = 0; j < WBN; ++j) f.b[j] = OpB::frag_global(prm.b, prm.ldb, n0, N, nfull * BK, K, j, li, lg);
+    for (int j = 0; j < WBN; ++j) f.b[j] = OpB::frag_global(prm.b, prm.ldb, n0, N, nall * BK, K, j, li, lg);
     conj(f);
     t.template mma<0>(f);
     t.template mma<1>(f);
@@ -356,7 +367,64 @@ __device__ __forceinline__ void tile_at(const GemmParams<typename T::R>& prm, bo
   const R alr = prm.alpha, ali = prm.alpha_im, ber = prm.beta, bei = prm.beta_im;
   const bool acc_prev = prm.accumulate != 0, use_cin = ber != R(0) || (T::CPLX && bei != R(0));
   constexpr int NR = T::CPLX ? 2 : 1;
-  R* part = (R*)lds;
+  // U elements per thread and pass, their C loads in flight together: elements x0 + 256 u of the
+  // `total` from column n0 + col0 on, their sums from sum(element, component)
+  constexpr int U = 4;
+  auto store = [&](int x0, int total, int col0, auto sum) {
+    long at[U];
+    bool ok[U];
+    R prev[U][NR], cin[U][NR];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int x = x0 + 256 * u, gi = m0 + x % BM, gj = n0 + col0 + x / BM;
+      ok[u] = x < total && gi < M && gj < N;
+      at[u] = (long)gi + (long)gj * prm.ldc;
+#pragma unroll
+      for (int c = 0; c < NR; ++c) prev[u][c] = cin[u][c] = R(0);
+    }
+    if (acc_prev) {
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int c = 0; c < NR; ++c)
+          if (ok[u]) prev[u][c] = prm.c[at[u] * NR + c];
+    }
+    if (use_cin) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int x = x0 + 256 * u, gi = m0 + x % BM, gj = n0 + col0 + x / BM;
+#pragma unroll
+        for (int c = 0; c < NR; ++c)
+          if (ok[u]) cin[u][c] = prm.cin[((long)gi + (long)gj * prm.ldcin) * NR + c];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (!ok[u]) continue;
+      R* dst = prm.c + at[u] * NR;
+      const R xr = sum(u, 0);
+      if constexpr (!T::CPLX) {
+        R v = alr * xr;
+        if (acc_prev) v += prev[u][0];
+        if (use_cin) v += ber * cin[u][0];
+        dst[0] = v;
+      } else {
+        const R xi = sum(u, 1);
+        R vr = alr * xr - ali * xi, vi = alr * xi + ali * xr;
+        if (acc_prev) {
+          vr += prev[u][0];
+          vi += prev[u][NR - 1];
+        }
+        if (use_cin) {
+          vr += ber * cin[u][0] - bei * cin[u][NR - 1];
+          vi += ber * cin[u][NR - 1] + bei * cin[u][0];
+        }
+        dst[0] = vr;
+        dst[1] = vi;
+      }
+    }
+  };
+  R* lsum = (R*)lds;
   constexpr int COLS = 16 * G::JP, PART = COLS * BM * NR;  // reals of one wave's part
 #pragma unroll
   for (int jp = 0; jp < WBN; jp += G::JP) {
@@ -368,69 +436,28 @@ __device__ __forceinline__ void tile_at(const GemmParams<typename T::R>& prm, bo
       for (int i = 0; i < WBM; ++i)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          R* q = part + wave * PART + ((jj * 16 + out_col(R(0), lane, r)) * BM + 16 * i + li) * NR;
+          R* q = lsum + wave * PART + ((jj * 16 + out_col(R(0), lane, r)) * BM + 16 * i + li) * NR;
           q[0] = t.acc[0][i][jp + jj][r];
           if constexpr (T::CPLX) q[1] = t.acc[1][i][jp + jj][r];
         }
     }
     __syncthreads();
-    // U elements per thread and pass, their C loads in flight together
-    constexpr int U = 4;
     const int total = min(COLS, BN - 16 * jp) * BM;
-    for (int x0 = threadIdx.x; x0 < total; x0 += 256 * U) {
-      long at[U];
-      bool ok[U];
-      R prev[U][NR], cin[U][NR];
+    if constexpr (SPLIT) {
+      for (int x = threadIdx.x; x < total; x += 256) {
+        const int gi = m0 + x % BM, gj = n0 + 16 * jp + x / BM;
+        if (gi >= M || gj >= N) continue;
+        const R* q = lsum + x * NR;
+        R* dst = part.sums + ((long)gi + (long)gj * M) * NR;
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int x = x0 + 256 * u, gi = m0 + x % BM, gj = n0 + 16 * jp + x / BM;
-        ok[u] = x < total && gi < M && gj < N;
-        at[u] = (long)gi + (long)gj * prm.ldc;
-#pragma unroll
-        for (int c = 0; c < NR; ++c) prev[u][c] = cin[u][c] = R(0);
+        for (int c = 0; c < NR; ++c) dst[c] = (q[c] + q[PART + c]) + (q[2 * PART + c] + q[3 * PART + c]);
       }
-      if (acc_prev) {
-#pragma unroll
-        for (int u = 0; u < U; ++u)
-#pragma unroll
-          for (int c = 0; c < NR; ++c)
-            if (ok[u]) prev[u][c] = prm.c[at[u] * NR + c];
-      }
-      if (use_cin) {
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-          const int x = x0 + 256 * u, gi = m0 + x % BM, gj = n0 + 16 * jp + x / BM;
-#pragma unroll
-          for (int c = 0; c < NR; ++c)
-            if (ok[u]) cin[u][c] = prm.cin[((long)gi + (long)gj * prm.ldcin) * NR + c];
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        if (!ok[u]) continue;
-        const R* q = part + (x0 + 256 * u) * NR;
-        R* dst = prm.c + at[u] * NR;
-        const R xr = (q[0] + q[PART]) + (q[2 * PART] + q[3 * PART]);
-        if constexpr (!T::CPLX) {
-          R v = alr * xr;
-          if (acc_prev) v += prev[u][0];
-          if (use_cin) v += ber * cin[u][0];
-          dst[0] = v;
-        } else {
-          const R xi = (q[1] + q[PART + 1]) + (q[2 * PART + 1] + q[3 * PART + 1]);
-          R vr = alr * xr - ali * xi, vi = alr * xi + ali * xr;
-          if (acc_prev) {
-            vr += prev[u][0];
-            vi += prev[u][NR - 1];
-          }
-          if (use_cin) {
-            vr += ber * cin[u][0] - bei * cin[u][NR - 1];
-            vi += ber * cin[u][NR - 1] + bei * cin[u][0];
-          }
-          dst[0] = vr;
-          dst[1] = vi;
-        }
-      }
+    } else {
+      for (int x0 = threadIdx.x; x0 < total; x0 += 256 * U)
+        store(x0, total, 16 * jp, [&](int u, int c) {
+          const R* q = lsum + (x0 + 256 * u) * NR + c;
+          return (q[0] + q[PART]) + (q[2 * PART] + q[3 * PART]);
+        });
     }
   }
 }
@@ -470,6 +497,80 @@ __global__ __launch_bounds__(256, 2) void gemm_ks_group_kernel(TileGroup<typenam
   int local;
   if (group_member(g, blockIdx.x, 16 * WBM, 16 * WBN, prm, local) < 0) return;
   tile<T, A_KC, B_KC, WBM, WBN, S>(prm, local);
+}
+
+// One product whose tiles are each shared by `parts` workgroups; sums: the m x n sums of each share.
+// Workgroup w takes, in the XCD order of tile_of, one share of the inner dimension after another: the
+// tiles that an XCD runs at one time read the same part of the operands.
+template <typename T, bool A_KC, bool B_KC, int WBM, int WBN, int S>
+__global__ __launch_bounds__(256, 2) void gemm_ks_split_kernel(GemmParams<typename T::R> prm, int parts,
+                                                               typename T::R* __restrict__ sums) {
+  constexpr int BM = 16 * WBM, BN = 16 * WBN;
+  const int nbm = (prm.m + BM - 1) / BM, tiles = nbm * ((prm.n + BN - 1) / BN), all = tiles * parts;
+  const int xcd = blockIdx.x % 8, per = all / 8, rem = all % 8;
+  const int i = xcd * per + min(xcd, rem) + blockIdx.x / 8, share = i / tiles, tile = i % tiles;
+  const Part<typename T::R> part = {share, parts, sums + (long)share * prm.m * prm.n * (T::CPLX ? 2 : 1)};
+  tile_at<T, A_KC, B_KC, WBM, WBN, S, true>(prm, prm.opa == 'C', prm.opb == 'C', tile % nbm * BM, tile / nbm * BN, part);
+}
+
+// C from the shares' sums, added in a fixed order: a workgroup takes 64 elements, its four waves a
+// quarter of the shares each, 8 loads in flight.
+template <typename T>
+__global__ __launch_bounds__(256) void split_sum_kernel(GemmParams<typename T::R> prm, int parts,
+                                                        const typename T::R* __restrict__ sums) {
+  typedef typename T::R R;
+  constexpr int NR = T::CPLX ? 2 : 1, U = 8;
+  __shared__ R quarter[4][64 * NR];
+  const long total = (long)prm.m * prm.n;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const long x = (long)blockIdx.x * 64 + lane;
+  const int p0 = (int)((long)parts * wave / 4), p1 = (int)((long)parts * (wave + 1) / 4);
+  R acc[NR];
+#pragma unroll
+  for (int c = 0; c < NR; ++c) acc[c] = R(0);
+  if (x < total) {
+    for (int p = p0; p < p1; p += U) {
+      R v[U][NR];
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int c = 0; c < NR; ++c) v[u][c] = p + u < p1 ? sums[((long)(p + u) * total + x) * NR + c] : R(0);
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int c = 0; c < NR; ++c) acc[c] += v[u][c];
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < NR; ++c) quarter[wave][lane * NR + c] = acc[c];
+  __syncthreads();
+  if (wave != 0 || x >= total) return;
+#pragma unroll
+  for (int c = 0; c < NR; ++c)
+    acc[c] = (quarter[0][lane * NR + c] + quarter[1][lane * NR + c]) + (quarter[2][lane * NR + c] + quarter[3][lane * NR + c]);
+  const long gi = x % prm.m, gj = x / prm.m;
+  R* dst = prm.c + (gi + gj * prm.ldc) * NR;
+  const R* cin = prm.cin + (gi + gj * prm.ldcin) * NR;
+  if constexpr (!T::CPLX) {
+    R v = prm.alpha * acc[0];
+    if (prm.accumulate) v += dst[0];
+    if (prm.beta != R(0)) v += prm.beta * cin[0];
+    dst[0] = v;
+  } else {
+    const R ar = prm.alpha, ai = prm.alpha_im, br = prm.beta, bi = prm.beta_im;
+    R vr = ar * acc[0] - ai * acc[1], vi = ar * acc[1] + ai * acc[0];
+    if (prm.accumulate) {
+      vr += dst[0];
+      vi += dst[1];
+    }
+    if (br != R(0) || bi != R(0)) {
+      const R cr = cin[0], ci = cin[1];
+      vr += br * cr - bi * ci;
+      vi += br * ci + bi * cr;
+    }
+    dst[0] = vr;
+    dst[1] = vi;
+  }
 }
 
 // Persistent batch: items (problem, tile row, tile column), the first gridDim.x dealt out by
@@ -524,6 +625,22 @@ hipError_t launch_group(const GemmParams<typename T::R>* tiles, int count, hipSt
   else if (akc) hipLaunchKernelGGL((gemm_ks_group_kernel<T, true, false, WBM, WBN, S>), grid, block, 0, s, g);
   else if (bkc) hipLaunchKernelGGL((gemm_ks_group_kernel<T, false, true, WBM, WBN, S>), grid, block, 0, s, g);
   else hipLaunchKernelGGL((gemm_ks_group_kernel<T, false, false, WBM, WBN, S>), grid, block, 0, s, g);
+  return hipGetLastError();
+}
+
+template <typename T, int WBM, int WBN, int S>
+hipError_t launch_split(const GemmParams<typename T::R>& p, int parts, void* ws, hipStream_t s) {
+  const long tiles = ks_tiles(KsShape{WBM, WBN}, p.m, p.n);
+  if (parts < 2 || tiles * parts > kSplitMaxWorkgroups) return hipErrorInvalidValue;
+  const dim3 grid((unsigned)(tiles * parts)), block(256);
+  const bool akc = p.opa != 'N', bkc = p.opb == 'N';
+  typename T::R* sums = (typename T::R*)ws;
+  if (akc && bkc) hipLaunchKernelGGL((gemm_ks_split_kernel<T, true, true, WBM, WBN, S>), grid, block, 0, s, p, parts, sums);
+  else if (akc) hipLaunchKernelGGL((gemm_ks_split_kernel<T, true, false, WBM, WBN, S>), grid, block, 0, s, p, parts, sums);
+  else if (bkc) hipLaunchKernelGGL((gemm_ks_split_kernel<T, false, true, WBM, WBN, S>), grid, block, 0, s, p, parts, sums);
+  else hipLaunchKernelGGL((gemm_ks_split_kernel<T, false, false, WBM, WBN, S>), grid, block, 0, s, p, parts, sums);
+  const dim3 sum_grid((unsigned)(((long)p.m * p.n + 63) / 64));
+  hipLaunchKernelGGL((split_sum_kernel<T>), sum_grid, block, 0, s, p, parts, sums);
   return hipGetLastError();
 }
 

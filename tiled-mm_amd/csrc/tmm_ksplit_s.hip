@@ -18,4 +18,12 @@ hipError_t launch_ks_s_group(const GemmParams<float>* tiles, int count, hipStrea
   return ks::launch_group<ks::TypeS, 4, 4, 2>(tiles, count, s);
 }
 
+hipError_t launch_ks_s_split(const GemmParams<float>& p, int shape, int parts, void* ws, hipStream_t s) {
+  if (shape == kSplitShapes[0]) return ks::launch_split<ks::TypeS, 1, 1, 4>(p, parts, ws, s);
+  if (shape == kSplitShapes[1]) return ks::launch_split<ks::TypeS, 2, 2, 2>(p, parts, ws, s);
+  if (shape == kSplitShapes[2]) return ks::launch_split<ks::TypeS, 3, 3, 2>(p, parts, ws, s);
+  if (shape == kSplitShapes[3]) return ks::launch_split<ks::TypeS, 4, 4, 2>(p, parts, ws, s);
+  return hipErrorInvalidValue;
+}
+
 }  // namespace tmm

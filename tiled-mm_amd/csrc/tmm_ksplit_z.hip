@@ -16,4 +16,11 @@ hipError_t launch_ks_z_group(const GemmParams<double>* tiles, int count, hipStre
   return ks::launch_group<ks::TypeZ, 3, 3, 2>(tiles, count, s);
 }
 
+hipError_t launch_ks_z_split(const GemmParams<double>& p, int shape, int parts, void* ws, hipStream_t s) {
+  if (shape == kSplitShapes[0]) return ks::launch_split<ks::TypeZ, 1, 1, 4>(p, parts, ws, s);
+  if (shape == kSplitShapes[1]) return ks::launch_split<ks::TypeZ, 2, 2, 2>(p, parts, ws, s);
+  if (shape == kSplitShapes[2]) return ks::launch_split<ks::TypeZ, 3, 3, 2>(p, parts, ws, s);
+  return hipErrorInvalidValue;
+}
+
 }  // namespace tmm

@@ -210,6 +210,10 @@ Handle::~Handle() {
       if (ozwork_pending[i]) (void)hipEventSynchronize(ozwork_ev[i]);
       (void)hipEventDestroy(ozwork_ev[i]);
     }
+  if (split_ev) {
+    (void)hipEventSynchronize(split_ev);
+    (void)hipEventDestroy(split_ev);
+  }
   for (auto e : events) (void)hipEventDestroy(e);
   for (auto e : prof_events) (void)hipEventDestroy(e);
   delete threads;
@@ -404,6 +408,63 @@ int launch_mode(Handle& h, int ws, char opa, char opb, int m, int n, int k, cons
   launch(h.dtype, opa, opb, m, n, k, alpha, a, lda, b, ldb, beta, use_beta, cin, ldcin, accumulate, c, ldc, s,
          h.dgemm_variant);
   return 0;
+}
+
+// hipMalloc and its like are allowed while this lives, whatever other streams are capturing.
+struct RelaxedCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
+// Runs a native device call with its tiles shared by several workgroups, if that is the faster way
+// (split_plan). Not under stream capture, where the graph could run beside any later call, and not
+// without memory for the partial sums.
+template <typename R>
+bool launch_split(Handle& h, KsType type, const GemmParams<R>& p, hipStream_t s,
+                  hipError_t (*launch)(const GemmParams<R>&, int, int, void*, hipStream_t)) {
+  if (!ks_takes(p, type >= KsType::Z)) return false;
+  const SplitPlan plan = split_plan(type, p.m, p.n, p.k, h.cus);
+  if (plan.parts < 2) return false;
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &capture) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  if (capture != hipStreamCaptureStatusNone) return false;
+  std::lock_guard<std::mutex> lock(h.split_mu);
+  if (!h.split_ev) {
+    RelaxedCapture relaxed;
+    try {
+      h.split_work.reserve(split_bytes(type));
+    } catch (const Error&) {
+      return false;
+    }
+    hip_check(hipEventCreateWithFlags(&h.split_ev, hipEventDisableTiming), "hipEventCreate");
+  } else {
+    hip_check(hipStreamWaitEvent(s, h.split_ev, 0), "hipStreamWaitEvent (split products)");
+  }
+  hip_check(launch(p, plan.shape, plan.parts, h.split_work.ptr, s), "split GEMM launch");
+  hip_check(hipEventRecord(h.split_ev, s), "hipEventRecord (split products)");
+  return true;
+}
+
+bool launch_split(Handle& h, const GemmCall& c, bool use_beta, hipStream_t s) {
+  if (ozaki_active(h) || h.dgemm_variant != 1 || c.k <= 0) return false;
+  const bool cplx = h.dtype >= 2;
+  auto run = [&](auto zero, KsType type, auto launch) {
+    typedef decltype(zero) R;
+    GemmParams<R> p = make_params<R>(c.opa, c.opb, c.m, c.n, c.k, (const R*)c.alpha, cplx, c.a, c.lda, c.b, c.ldb,
+                                     (const R*)c.beta, use_beta, c.c, c.ldc, false, c.c, c.ldc);
+    p.variant = 1;
+    return launch_split<R>(h, type, p, s, launch);
+  };
+  switch (h.dtype) {
+    case 0: return run(0.0f, KsType::S, launch_ks_s_split);
+    case 1: return run(0.0, KsType::D, launch_ks_d_split);
+    case 2: return run(0.0f, KsType::C, launch_ks_c_split);
+    default: return run(0.0, KsType::Z, launch_ks_z_split);
+  }
 }
 
 bool scalar_is_zero(int dtype, const void* v) {
@@ -1138,6 +1199,10 @@ void gemm_device(Handle& h, const GemmCall& in, hipStream_t s) {
   if (scalar_is_zero(h.dtype, call.alpha)) call.k = 0;  // C = beta*C; A and B are not read
   // In-place C: C_in and C_out are the same matrix, so the beta term reads each element
   // before the same thread overwrites it.
+  if (launch_split(h, call, use_beta, s ? s : h.compute[0])) {
+    h.stats[13] = 0;
+    return;
+  }
   const int np = launch_mode(h, 0, call.opa, call.opb, call.m, call.n, call.k, call.alpha, call.a, call.lda, call.b,
                              call.ldb, call.beta, use_beta, call.c, call.ldc, false, call.c, call.ldc,
                              s ? s : h.compute[0]);

@@ -154,6 +154,12 @@ struct Handle {
   // user waits for it (another stream) and a reallocation synchronises with it first
   std::vector<hipEvent_t> ozwork_ev;
   std::vector<char> ozwork_pending;
+  // partial sums of a device call whose inner dimension is split over workgroups (split_plan): one
+  // buffer, its calls ordered by split_ev on whatever streams they run; split_mu holds from the wait
+  // to the record, so that callers' threads need no order of their own
+  std::mutex split_mu;
+  DeviceBuffer split_work;
+  hipEvent_t split_ev = nullptr;
   std::vector<DeviceBuffer> ozcache;  // scheme II prepared-operand slots, one buffer per compute queue
   DeviceBuffer batch_meta;           // batched path: problem descriptors, work items, counters
   TuneRates rates;
