@@ -1,35 +1,29 @@
-"""The residue of an int32 sum in the epilogue of the INT8 product kernel (residue_of_sum in
-tiled-mm_amd/csrc/tmm_ozaki.hip), modelled in FP32 on the CPU: for every modulus and every value that
-the folded sum t can take (and so for every sum up to 2^30 in magnitude) it must be the exact
-remainder in [0, modulus)."""
+"""The residue of an int32 sum in the epilogue of the INT8 product kernel (residues_of_sums in
+tiled-mm_amd/csrc/tmm_ozaki.hip), modelled in integers on the CPU: for every modulus and sums up to 2^30
+in magnitude it must be congruent to the sum and lie in [0, modulus], where the byte it is stored in
+holds it (modulus 256: [0, 255])."""
 import numpy as np
 import pytest
 
 from crt_model import MODULI
 
 
+def _residue(s, m):
+    magic = -(-2 ** 38 // m)
+    assert magic < 2 ** 31  # a signed 32-bit factor
+    h = (s * magic) >> 32
+    q = (h & 0xffff) >> 6  # 16-bit lanes from here on
+    return ((q * ((-m) & 0xffff) + (s & 0xffff)) & 0xffff) & 0xff
+
+
 @pytest.mark.parametrize("m", MODULI)
-def test_residue_of_every_folded_sum(m):
-    c16 = 65536 % m
-    c16 = c16 - m if c16 > m // 2 else c16
-    assert abs(c16) <= 128
-    top = 16384 * 128 + 65535  # |hi| <= 2^14 for |sum| <= 2^30, lo < 2^16
-    inv = np.float32(1) / np.float32(m)
-    for lo in range(-top, top + 1, 1 << 20):
-        t = np.arange(lo, min(lo + (1 << 20), top + 1))
-        f = t.astype(np.float32)
-        assert np.array_equal(f.astype(np.int64), t)
-        # fma(f, inv, inv / 2): the products and the sum fit 53 bits, one rounding to FP32
-        q = np.floor((f.astype(np.float64) * np.float64(inv) + np.float64(np.float32(0.5) * inv)).astype(np.float32))
-        r = f.astype(np.float64) - q.astype(np.float64) * m
-        assert np.array_equal(r.astype(np.int64), t % m)
-
-
-def test_folding_keeps_the_residue():
-    rng = np.random.default_rng(5)
-    s = np.concatenate([rng.integers(-2 ** 30, 2 ** 30 + 1, 100000), [-2 ** 30, -1, 0, 1, 65535, 65536, 2 ** 30]])
-    for m in MODULI:
-        c16 = 65536 % m
-        c16 = c16 - m if c16 > m // 2 else c16
-        t = (s >> 16) * c16 + (s & 0xffff)
-        assert np.array_equal(t % m, s % m) and np.abs(t).max() <= 16384 * 128 + 65535
+def test_residue_of_a_sum(m):
+    assert 129 <= m <= 256
+    rng = np.random.default_rng(m)
+    top = 2 ** 30
+    near = (np.arange(-top // m, top // m + 1, 997, dtype=np.int64)[:, None] * m + np.arange(-2, 3)).ravel()
+    ends = np.concatenate([np.arange(-top, -top + 5000), np.arange(-5000, 5000), np.arange(top - 5000, top + 1)])
+    for s in (rng.integers(-top, top + 1, 2000000), near[np.abs(near) <= top], ends):
+        r = _residue(s.astype(np.int64), m)
+        assert np.array_equal(r % m, s % m)
+        assert r.min() >= 0 and r.max() <= min(m, 255)

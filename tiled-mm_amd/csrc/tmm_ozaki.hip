@@ -191,8 +191,8 @@ struct CrtProductParams {
   long plane, ldres;
   const int* fa;
   const int* fb;
-  int c16[kCrtMaxModuli];  // 2^16 mod m, balanced
-  float inv[kCrtMaxModuli], mod[kCrtMaxModuli];
+  int magic[kCrtMaxModuli];       // ceil(2^38 / m)
+  unsigned neg_m[kCrtMaxModuli];  // -m
 };
 
 constexpr int OZ_BM = 256, OZ_BN = 256, OZ_BK = 64;
@@ -246,18 +246,32 @@ __device__ __forceinline__ int xcd_range(int w, int n) {
   return xcd * per + min(xcd, rem) + w / 8;
 }
 
-// acc mod m as a float in [0, m), for |acc| <= 2^30 and 2 <= m <= 256: acc = hi 2^16 + lo is
-// congruent to t = hi (2^16 mod m, balanced) + lo, |t| < 2^21.1, and floor((t + 1/2) / m) is exact in
-// FP32: (t + 1/2) / m lies at least 1 / (2m) from an integer, and the error of the product is below
-// |t / m| 2^-23 < 1 / (2m). Eight full-rate instructions with the conversion to a byte; an integer
-// multiply-high and its correction are two quarter-rate ones and five others.
-__device__ __forceinline__ float residue_of_sum(int acc, int c16, float inv, float m) {
-  const int t = __mul24(acc >> 16, c16) + (acc & 0xffff);
-  const float f = (float)t;
-  return fmaf(-floorf(fmaf(f, inv, 0.5f * inv)), m, f);
+// Residues of four sums as the bytes of a word: each congruent to its sum mod m and in [0, m], for
+// |sum| <= 2^30 and 129 <= m <= 256. h = sum M / 2^32 with M = ceil(2^38 / m), q = h / 2^6: sum M / 2^38
+// differs from sum / m by less than 2^30 / 2^38 < 1 / m (not at all for 256), so q is the floored
+// quotient, or one less where a negative sum is a multiple of m (the residue is then m, as good as 0
+// for the reconstruction). Of sum - q m only the low byte is needed, so that part runs on pairs of 16
+// bits. 17 instructions for four sums with the reads of the accumulators; with one wave per SIMD an
+// instruction takes 5.5 cycles and a conversion between integers and floats 8.5, and the FP32 form
+// (fold to 21 bits, convert, fma, floor, fma, convert and pack) took 36 of them, a quarter of the
+// kernel's time at an inner dimension of 2048.
+__device__ __forceinline__ unsigned residues_of_sums(const i32x4& sum, int magic, unsigned neg_m) {
+  typedef unsigned short us2 __attribute__((ext_vector_type(2)));
+  const us2 factor = {(unsigned short)neg_m, (unsigned short)neg_m};
+  unsigned r[2];
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    const int s0 = sum[2 * p], s1 = sum[2 * p + 1];
+    // the low halves of two words
+    const unsigned h = __builtin_amdgcn_perm((unsigned)__mulhi(s1, magic), (unsigned)__mulhi(s0, magic), 0x05040100u);
+    const unsigned s = __builtin_amdgcn_perm((unsigned)s1, (unsigned)s0, 0x05040100u);
+    const us2 q = __builtin_bit_cast(us2, h) >> (unsigned short)6;
+    r[p] = __builtin_bit_cast(unsigned, (us2)(q * factor + __builtin_bit_cast(us2, s)));
+  }
+  return __builtin_amdgcn_perm(r[1], r[0], 0x06040200u);
 }
 
-// Residue epilogue of the product kernel: res[i + j*ldres] = acc mod modulus for the workgroup's
+// Residue epilogue of the product kernel: res[i + j*ldres] = acc mod m for the workgroup's
 // 256x256 tile. The lane holds C(i = m0 + wm*128 + bi*16 + 4*lg + r, j = n0 + wn*128 + bj*16 + li) in
 // acc[bj][bi][r] (B is the loop's first operand), so the four residues of an accumulator are
 // consecutive rows: one word. The words go through the (then idle) LDS ring as a column-major
@@ -268,18 +282,15 @@ constexpr int OZ_RES_STRIDE = 272;
 
 __device__ __forceinline__ void oz_store_residues(const CrtProductParams& prm, int q, const i32x4 (&acc)[8][8], int m0,
                                                   int n0, int wm, int wn, int li, int lg, int8_t* lds) {
-  const int c16 = prm.c16[q];
-  const float inv = prm.inv[q], mod = prm.mod[q];
+  const int magic = prm.magic[q];
+  const unsigned neg_m = prm.neg_m[q];
   uint8_t* T = (uint8_t*)lds;
   __syncthreads();  // every wave is done with the ring
 #pragma unroll
   for (int bj = 0; bj < 8; ++bj)
 #pragma unroll
     for (int bi = 0; bi < 8; ++bi) {
-      unsigned w = 0;
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        w = __builtin_amdgcn_cvt_pk_u8_f32(residue_of_sum(acc[bj][bi][r], c16, inv, mod), r, w);
+      const unsigned w = residues_of_sums(acc[bj][bi], magic, neg_m);
       *(unsigned*)(T + (wn * 128 + bj * 16 + li) * OZ_RES_STRIDE + wm * 128 + bi * 16 + 4 * lg) = w;
     }
   __syncthreads();
@@ -410,8 +421,12 @@ __global__ __launch_bounds__(256, 1) void ozaki_gemm_kernel(OzakiGemmParams prm)
 // layout, a 4-stage ring (128 KB of LDS) and the k-step schedule of gen_crt_loop.py (fragments
 // double-buffered in registers, loads and LDS reads interleaved with the MFMAs, one barrier
 // half-way through each k-step). B is the loop's first operand (see oz_store_residues). A 5-stage
-// ring (160 KB) gave the same rate, the limit being the L2 -> LDS data path (texture data unit busy
-// 83% of cycles).
+// ring (160 KB) gave the same rate.
+// A k-step takes 1090 to 1140 cycles, 1024 of them MFMAs, and a tile some 22000 cycles more (first
+// loads, residues, 64 KB of stores, the next workgroup's start; 26000 before the residues ran on
+// integers). What bounds a long inner dimension is power: the clock falls from 2.7 GHz at 64 to 2.0 at
+// 2048 and 1.85 at 8192. 2048 x 2048 x k, 16 moduli, in us: k = 64 42.3 -> 34.3, 512 61.4 -> 59.0, 2048
+// 122.2 -> 117.4.
 __global__ __launch_bounds__(256, 1) void crt_product_kernel(CrtProductParams prm) {
   constexpr int S = 4;  // the generated loop's ring
   __shared__ __attribute__((aligned(16))) int8_t lds[S * OZ_STAGE];
@@ -679,6 +694,7 @@ namespace {
 
 constexpr int kCrtModuli[kCrtMaxModuli] = {256, 255, 253, 251, 247, 241, 239, 233, 229, 227,
                                            223, 211, 199, 197, 193, 191, 181, 179, 173, 167};
+static_assert(kCrtModuli[kCrtMaxModuli - 1] >= 129, "residues_of_sums: 2^38 / m fits a signed factor");
 
 constexpr long inv_mod(long a, long m) {  // extended Euclid; a and m coprime
   long g = m, x = 0, x1 = 1, a1 = a % m;
@@ -1049,10 +1065,8 @@ hipError_t ozaki2_products(int m, int n, int k, const void* pa, const void* pb, 
   P.fa = (const int*)pa + m;  // operands with a fallback flag skip the products
   P.fb = (const int*)pb + n;
   auto constants = [&P](int at, int modulus) {
-    const int c = 65536 % modulus;
-    P.c16[at] = c > modulus / 2 ? c - modulus : c;
-    P.inv[at] = 1.0f / (float)modulus;
-    P.mod[at] = (float)modulus;
+    P.magic[at] = (int)(((1L << 38) + modulus - 1) / modulus);
+    P.neg_m[at] = (unsigned)-modulus;
   };
   const long ntiles = (mpad / OZ_BM) * (npad / OZ_BN);
   // All moduli in one launch while a modulus has few tiles: alone it leaves CUs idle (2048^3: 64
