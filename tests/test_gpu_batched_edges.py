@@ -53,8 +53,8 @@ def test_batched_tile_edges_exact(torch_gpu, flags):
 @pytest.mark.parametrize("graph", [0, 1])
 @pytest.mark.parametrize("pad,shift", [(0, 0), (0, 1), (1, 0), (2, 1)])
 def test_batched_copies_exact(torch_gpu, pad, shift, graph):
-    """Matrices on both sides of the size that one kernel copies, of the 4096 elements of its pieces,
-    and of 16-byte alignment; contiguous and padded; nothing beyond the matrices is written."""
+    """A batch whose copies run by kernel: matrices on both sides of the 4096 elements of its pieces and
+    of 16-byte alignment; contiguous and padded; nothing beyond the matrices is written."""
     rng = np.random.default_rng(22)
     sizes = [(362, 362, 362), (363, 362, 361), (1, 1, 1), (64, 64, 64), (4095, 3, 5), (4096, 2, 3), (4097, 3, 2),
              (3, 4099, 2), (17, 9, 4101)]

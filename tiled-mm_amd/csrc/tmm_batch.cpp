@@ -4,7 +4,7 @@
 // Tiled-MM src/Tiled-MM/tiled_mm.cpp:492-624, each with its own tiling, copies and a
 // device-wide synchronisation). Here the whole batch is one pipeline:
 //   * the problems are packed into one device arena and cut into G groups of about equal
-//     host-link bytes; group g's H2D copies (small matrices by one kernel, large ones spread over
+//     host-link bytes; group g's H2D copies (one kernel in a batch of small matrices, else spread over
 //     two copy queues), one persistent batched-kernel launch over all C tiles of the group (largest
 //     k first), and its D2H copies run on their own queues, so H2D of group g+1 overlaps the kernel
 //     of group g and the D2H of group g-1;
@@ -33,19 +33,22 @@ struct Prob {
   const double* b;
   double* c;
   double alpha, beta;
-  void *map_a = nullptr, *map_b = nullptr, *map_c = nullptr;  // a, b, c on the device if a kernel copies them
+  void *map_a = nullptr, *map_b = nullptr, *map_c = nullptr;  // a, b, c on the device
   size_t offA, offB, offC;  // arena offsets (elements)
   long rowsA, colsA, rowsB, colsB;
 };
 
-// Page-locked matrices of up to this size are copied by one kernel per group and direction
-// (tmm_copy.hip; its workgroups), larger ones by a DMA command each: below it the command's 10 us
-// outweigh the transfer, above it a kernel's reads over the link slow the tile kernels beside it
-// (their loads wait behind them in the L2; 0.27 ms for a group became 0.5). Calls in us with no
-// kernel copies / up to 256 KB / 1 MB / 4 MB: 48 problems of 64 to 1024 rows and columns 2350 / 2377 /
-// 2284 / 2756, 90 of 64 to 700 with padded columns 4707 / 3870 / 3048 / 3154, 300 of 16 to 128 6620 /
-// 1547 / 1518 / 1519, 200 of 64 to 3000 37770 / 37862 / 37385 / 37880.
-constexpr size_t kKernelCopyBytes = 1u << 20;
+// A batch in page-locked memory is copied by one kernel per group and direction (tmm_copy.hip; its
+// workgroups) while its copies are no larger than this on average, contiguous ones and padded ones,
+// and by a DMA command each otherwise: below it the commands' 10 us (more for a padded matrix)
+// outweigh the transfers, above it a kernel's reads over the link slow the tile kernels beside it
+// (their loads wait behind them in the L2). us per call by DMA / by kernel: contiguous, mean 78 KB
+// 2009 / 936, 432 KB 885 / 790, 703 KB 3070 / 2875, 733 KB 728 / 680, 867 KB 2370 / 2650, 1203 KB 2627 /
+// 3112; padded, 294 KB 2360 / 1250, 570 KB 4640 / 3130, 846 KB 3160 / 2617, 1250 KB 2754 / 2436. Never both
+// in one batch: where the streams share hardware queues, as in a process with other handles, the
+// copy kernels then wait for DMA commands and for each other (867 KB: 2300 in a first handle, 3100
+// to 3800 in later ones).
+constexpr double kKernelCopyBytes = 768 << 10, kKernelCopyPaddedBytes = 1536 << 10;
 constexpr int kCopyInWorkgroups = 64, kCopyOutWorkgroups = 32;
 
 }  // namespace
@@ -119,12 +122,19 @@ void gemm_batched_host(Handle& h, char opa, char opb, int count, const int* m, c
     if (!all_pinned) break;
   }
   shape.pinned = all_pinned;
-  for (Prob& p : P) {  // only the matrices that a kernel copies keep their device address
-    auto small = [&](long rows, long cols) { return rows > 0 && cols > 0 && (size_t)rows * cols * 8 <= kKernelCopyBytes; };
-    if (!all_pinned || !small(p.rowsA, p.colsA)) p.map_a = nullptr;
-    if (!all_pinned || !small(p.rowsB, p.colsB)) p.map_b = nullptr;
-    if (!all_pinned || !small(p.m, p.n)) p.map_c = nullptr;
+  double copy_limit = 0;  // of all copies together (kKernelCopyBytes)
+  bool mapped = all_pinned;
+  for (const Prob& p : P) {
+    auto add = [&](const void* map, long rows, long cols, long ld, int copies) {
+      if (rows <= 0 || cols <= 0) return;
+      mapped = mapped && map;
+      copy_limit += copies * (ld == rows ? kKernelCopyBytes : kKernelCopyPaddedBytes);
+    };
+    add(p.map_a, p.rowsA, p.colsA, p.lda, 1);
+    add(p.map_b, p.rowsB, p.colsB, p.ldb, 1);
+    add(p.map_c, p.m, p.n, p.ldc, p.beta != 0.0 ? 2 : 1);
   }
+  const bool by_kernel = mapped && shape.h2d_bytes + shape.d2h_bytes <= copy_limit;
   BatchConfig cfg = choose_batch_config(h, shape);
   cfg.queues = std::max(1, std::min(cfg.queues, (int)h.compute.size()));
   // emulated problems: one workspace per compute queue (groups alternate over the queues),
@@ -207,25 +217,23 @@ void gemm_batched_host(Handle& h, char opa, char opb, int count, const int* m, c
       }
       return;
     }
+    if (rows <= 0 || cols <= 0) return;
     const long nr = std::min(rows, kCopyItemElems), nc = std::max(1L, kCopyItemElems / nr);
     for (long c = 0; c < cols; c += nc)
       for (long r = 0; r < rows; r += nr)
         copies.push_back(CopyItem{src + r + c * ld_src, dst + r + c * ld_dst, ld_src, ld_dst,
                                   (int)std::min(nr, rows - r), (int)std::min(nc, cols - c)});
   };
-  for (int g = 0; g < G; ++g) {
+  for (int g = 0; g < G && by_kernel; ++g) {
     in_start[g] = (int)copies.size();
     for (int i = gstart[g]; i < gstart[g + 1]; ++i) {
       const Prob& p = P[i];
-      if (p.map_a) add_copies((const double*)p.map_a, p.lda, dev + p.offA, p.rowsA, p.rowsA, p.colsA);
-      if (p.map_b) add_copies((const double*)p.map_b, p.ldb, dev + p.offB, p.rowsB, p.rowsB, p.colsB);
-      if (p.map_c && p.beta != 0.0) add_copies((const double*)p.map_c, p.ldc, dev + p.offC, p.m, p.m, p.n);
+      add_copies((const double*)p.map_a, p.lda, dev + p.offA, p.rowsA, p.rowsA, p.colsA);
+      add_copies((const double*)p.map_b, p.ldb, dev + p.offB, p.rowsB, p.rowsB, p.colsB);
+      if (p.beta != 0.0) add_copies((const double*)p.map_c, p.ldc, dev + p.offC, p.m, p.m, p.n);
     }
     out_start[g] = (int)copies.size();
-    for (int i = gstart[g]; i < gstart[g + 1]; ++i) {
-      const Prob& p = P[i];
-      if (p.map_c) add_copies(dev + p.offC, p.m, (double*)p.map_c, p.ldc, p.m, p.n);
-    }
+    for (int i = gstart[g]; i < gstart[g + 1]; ++i) add_copies(dev + P[i].offC, P[i].m, (double*)P[i].map_c, P[i].ldc, P[i].m, P[i].n);
   }
   in_start[G] = (int)copies.size();
 
@@ -275,9 +283,7 @@ void gemm_batched_host(Handle& h, char opa, char opb, int count, const int* m, c
   // queue's transfer covers the other's. The 512-problem batch (m, n, k log-uniform in [64, 4096],
   // 1536 H2D copies of 4 KB - 130 MB, 64 groups) ran 232-234 ms per call with one H2D queue, 213 ms
   // with two balanced by bytes; a third queue, or a second D2H queue, ran slower.
-  bool dma_in = false;
-  for (const Prob& p : P) dma_in = dma_in || !p.map_a || !p.map_b || (p.beta != 0.0 && !p.map_c);
-  hipStream_t sh2 = dma_in ? h.h2d_aux_stream() : sh;
+  hipStream_t sh2 = by_kernel ? sh : h.h2d_aux_stream();
   std::vector<hipEvent_t> ev_in(G), ev_in2(G), ev_k(G);
   for (int g = 0; g < G; ++g) {
     ev_in[g] = h.event(3 * g);
@@ -305,12 +311,12 @@ void gemm_batched_host(Handle& h, char opa, char opb, int count, const int* m, c
          q ? sh2 : sh);
   };
   auto h2d = [&](const Prob& p) {
-    if (!p.map_a) h2d_copy(dev + p.offA, p.a, p.rowsA, p.colsA, p.lda);
-    if (!p.map_b) h2d_copy(dev + p.offB, p.b, p.rowsB, p.colsB, p.ldb);
-    if (p.beta != 0.0 && !p.map_c) h2d_copy(dev + p.offC, p.c, p.m, p.n, p.ldc);
+    h2d_copy(dev + p.offA, p.a, p.rowsA, p.colsA, p.lda);
+    h2d_copy(dev + p.offB, p.b, p.rowsB, p.colsB, p.ldb);
+    if (p.beta != 0.0) h2d_copy(dev + p.offC, p.c, p.m, p.n, p.ldc);
   };
   auto d2h = [&](const Prob& p, hipStream_t s) {
-    if (p.m && p.n && !p.map_c)
+    if (p.m && p.n)
       copy(p.c, (size_t)p.ldc * 8, dev + p.offC, (size_t)p.m * 8, (size_t)p.m * 8, (size_t)p.n, hipMemcpyDeviceToHost,
            s);
   };
@@ -319,16 +325,17 @@ void gemm_batched_host(Handle& h, char opa, char opb, int count, const int* m, c
     hip_check(hipEventRecord(ev_fork, sh), "hipEventRecord");
     for (hipStream_t q : scs) hip_check(hipStreamWaitEvent(q, ev_fork, 0), "hipStreamWaitEvent");
     hip_check(hipStreamWaitEvent(sd, ev_fork, 0), "hipStreamWaitEvent");
-    if (dma_in) hip_check(hipStreamWaitEvent(sh2, ev_fork, 0), "hipStreamWaitEvent");
+    if (!by_kernel) hip_check(hipStreamWaitEvent(sh2, ev_fork, 0), "hipStreamWaitEvent");
     issued[0] = issued[1] = 0;
     for (int g = 0; g < G; ++g) {
       hipStream_t sg = scs[g % cfg.queues];
       hip_check(launch_copy_items(d_copies + in_start[g], out_start[g] - in_start[g], kCopyInWorkgroups, sh),
                 "batched H2D copy launch");
-      for (int i = gstart[g]; i < gstart[g + 1]; ++i) h2d(P[i]);
+      if (!by_kernel)
+        for (int i = gstart[g]; i < gstart[g + 1]; ++i) h2d(P[i]);
       hip_check(hipEventRecord(ev_in[g], sh), "hipEventRecord");
       hip_check(hipStreamWaitEvent(sg, ev_in[g], 0), "hipStreamWaitEvent");
-      if (dma_in) {
+      if (!by_kernel) {
         hip_check(hipEventRecord(ev_in2[g], sh2), "hipEventRecord");
         hip_check(hipStreamWaitEvent(sg, ev_in2[g], 0), "hipStreamWaitEvent");
       }
@@ -338,7 +345,8 @@ void gemm_batched_host(Handle& h, char opa, char opb, int count, const int* m, c
       hip_check(launch_copy_items(d_copies + out_start[g], in_start[g + 1] - out_start[g], kCopyOutWorkgroups,
                                   sd),
                 "batched D2H copy launch");
-      for (int i = gstart[g]; i < gstart[g + 1]; ++i) d2h(P[i], sd);
+      if (!by_kernel)
+        for (int i = gstart[g]; i < gstart[g + 1]; ++i) d2h(P[i], sd);
     }
     // join back into the H2D queue
     for (size_t q = 0; q < scs.size(); ++q) {
@@ -347,7 +355,7 @@ void gemm_batched_host(Handle& h, char opa, char opb, int count, const int* m, c
     }
     hip_check(hipEventRecord(ev_join_d, sd), "hipEventRecord");
     hip_check(hipStreamWaitEvent(sh, ev_join_d, 0), "hipStreamWaitEvent");
-    if (dma_in) {
+    if (!by_kernel) {
       hip_check(hipEventRecord(ev_join_h2, sh2), "hipEventRecord");
       hip_check(hipStreamWaitEvent(sh, ev_join_h2, 0), "hipStreamWaitEvent");
     }

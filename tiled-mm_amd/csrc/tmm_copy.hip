@@ -3,9 +3,9 @@
 // A DMA command costs about 10 us beside its transfer (64 KB at 6 GB/s, 1 MB at 38), and a batch of
 // small matrices issues three per problem. A kernel reads and writes page-locked memory over the same
 // link at its full rate (64 MB at 56.7 GB/s from 64 workgroups, 55.2 GB/s back from 32; DMA 57.0), so
-// that one launch copies all the small matrices of a group. Bound by the link; a thread keeps 8
-// accesses in flight, 32 KB per workgroup, and 64 workgroups leave the CUs to the tile kernels beside
-// them (256 and more ran slower: 53 GB/s).
+// that one launch copies the matrices of a group. Bound by the link; a thread keeps 8 accesses in
+// flight, 32 KB per workgroup, and 64 workgroups leave the CUs to the tile kernels beside them (256
+// and more ran slower: 53 GB/s).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
