@@ -795,9 +795,11 @@ __device__ __forceinline__ long crt_tiled_offset(int r, int k, int kpad) {
 //   is off by less than 2^-20, and y / m lies at least 1 / (2m) from a half for odd m and is exact
 //   for 256, so y - q m is the balanced residue (128 and -128 are the same byte); adding 1.5 2^52
 //   once more leaves it in the low byte. Five FP64 instructions and 3/4 of a byte permutation, all
-//   full-rate; the integer form's multiply-highs are quarter-rate ones. Bound by memory: 16 moduli of
-// two operands of 2048 x 2048 46 us (4.4 TB/s), of 4096 x 4096 209 us; a launch per operand with the
-// integer form took 87 us at 2048 x 2048.
+//   full-rate; an integer form needs a wider reduction. Bound by memory once the loads of a tile are in
+//   flight together and nothing waits on them one by one: 16 moduli of two operands of 1000 x 1000 16
+//   us, of 2048 x 2048 41 us (4.9 TB/s), of 4096 x 4096 188 us; with a bounds check around every load
+//   and LDS read 20, 46 and 227 us; a launch per operand with the integer form took 87 us at 2048 x
+//   2048.
 struct ResidueDst {
   int bits, kpad;
   long plane;
@@ -809,30 +811,43 @@ __device__ __forceinline__ void residues64(const OperandSrc& o, const ResidueDst
                                            int q0, int q1, double* tile) {
   const int t = threadIdx.x, nks = d.kpad / 64;
   const int r0 = (((block >> 2) / nks) * 4 + (block & 3)) * 64, k0 = (block >> 2) % nks * 64;
+  // all 16 loads in flight, out-of-range ones from the last row and k, before any goes to LDS
+  double v[16] = {};
+  if (o.rows > 0 && o.k > 0) {
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      const int hi = (t >> 6) + 4 * j, lo = t & 63;
+      const int r = min(r0 + (o.kc ? hi : lo), o.rows - 1), kk = min(k0 + (o.kc ? lo : hi), o.k - 1);
+      v[j] = o.p[o.kc ? (long)kk + (long)r * o.ld : (long)r + (long)kk * o.ld];
+    }
+  }
 #pragma unroll
   for (int j = 0; j < 16; ++j) {
     const int hi = (t >> 6) + 4 * j, lo = t & 63;
-    const int rl = o.kc ? hi : lo, kl = o.kc ? lo : hi, r = r0 + rl, kk = k0 + kl;
-    double v = 0.0;
-    if (r < o.rows && kk < o.k) v = o.p[o.kc ? (long)kk + (long)r * o.ld : (long)r + (long)kk * o.ld];
-    tile[rl * kResStride + kl] = v;
+    const int rl = o.kc ? hi : lo, kl = o.kc ? lo : hi;
+    tile[rl * kResStride + kl] = r0 + rl < o.rows && k0 + kl < o.k ? v[j] : 0.0;
   }
   __syncthreads();
   // 4 lanes take a row: a wave's 64 stores of 16 bytes fill 1 KB
   const int rl = t >> 2, g = t & 3, r = r0 + rl;
   const int er = r < o.rows ? o.e[r] : kExpNone;
+  const int shift = er == kExpNone ? 0 : d.bits - er;  // a row without an exponent holds zeros
   double xh[16], xl[16];
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
-    const double v = tile[rl * kResStride + 16 * g + i];
-    const double x = er == kExpNone ? 0.0 : rint(ldexp(v, d.bits - er));
+    const double x = rint(ldexp(tile[rl * kResStride + 16 * g + i], shift));
     xh[i] = rint(x * 0x1p-30);
     xl[i] = fma(-xh[i], 0x1p30, x);
   }
   const double magic = 0x1.8p52;
   int8_t* out = d.out + crt_tiled_offset(r, k0 + 16 * g, d.kpad);
+  double c30_next = cc.c30[q0], inv_next = cc.inv[q0], m_next = cc.m[q0];
   for (int q = q0; q < q1; ++q) {
-    const double c30 = cc.c30[q], inv = cc.inv[q], m = cc.m[q];
+    const double c30 = c30_next, inv = inv_next, m = m_next;
+    const int qn = min(q + 1, q1 - 1);  // the next modulus's constants come in under this one's work
+    c30_next = cc.c30[qn];
+    inv_next = cc.inv[qn];
+    m_next = cc.m[qn];
     unsigned b[16];
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
@@ -1031,11 +1046,10 @@ hipError_t prepare(const PrepareJob* jobs, int count, int k, int nmod, hipStream
   }
   const hipError_t e = launch_exponents(src, count, s);
   if (e != hipSuccess) return e;
-  // Up to 384 workgroups (1.5 per CU) the moduli go to two sets of them, which read the operands
-  // twice but keep more waves in flight: whole emulated products of 500^3 45.6 -> 43.2 us, 700^3 48.9 ->
-  // 46.8; with 512 workgroups 64.4 -> 63.8 (1000^3), with 520 81.2 -> 84.5 (1200 x 1200 x 800), with more
-  // the second read costs up to 10%; four sets gain nothing more.
-  const int all = blocks[0] + blocks[1], parts = all <= 384 ? 2 : 1;
+  // Up to about one workgroup per CU the moduli go to two sets of them, which read the operands twice
+  // but keep more waves in flight: whole emulated products of 500^3 (128 workgroups) 40.7 -> 38.9 us,
+  // 700^3 (264) 45.6 -> 44.5; 850^3 (448) 52.8 -> 54.4, 2048^3 216 -> 224; four sets gain nothing more.
+  const int all = blocks[0] + blocks[1], parts = all <= 288 ? 2 : 1;
   hipLaunchKernelGGL(residues_kernel, dim3(all, parts), dim3(256), 0, s, src[0], dst[0], blocks[0], src[1], dst[1],
                      residue_consts(nmod));
   return hipGetLastError();
