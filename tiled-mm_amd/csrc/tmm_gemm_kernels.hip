@@ -1678,6 +1678,13 @@ Route route(KsType t, const GemmParams<R>& p) {
   if (!ks_takes(p, cplx)) return {pipe ? Route::kPipe : Route::kReal, 0};
   double us = 0;
   const int shape = ks_shape(t, p.m, p.n, p.k, cus, &us);
+  // Two k-contiguous real operands with leading dimensions off 64 bytes: a 64-byte row chunk of a
+  // k-split stage then touches two of the L2's lines, and small tiles load twice as many chunks. FP64 TN
+  // 4832 x 5373, ld 8098 against 8096: k-split 7330 against 6394 us, pipelined 6808 against 6660; ld 6001
+  // against 6008: 5099 against 4719, pipelined 4971; 3000 x 3000 x 8090 6% (pipelined far behind). Complex
+  // operands lose 1%. By the leading dimension alone, so that the route does not hang on addresses.
+  if (!cplx && p.opa != 'N' && p.opb == 'N' && p.lda * (long)sizeof(R) % 64 != 0 && p.ldb * (long)sizeof(R) % 64 != 0)
+    us *= 1 + 0.13 * std::min(1.0, p.k * (double)sizeof(R) / 64000);
   const bool many = t != KsType::Z && tiles >= 12L * cus;
   if (pipe && (many || 0.98 * pipe_time(t, tiles, p.k, cus) <= us)) return {Route::kPipe, 0};
   return {Route::kKs, shape};
