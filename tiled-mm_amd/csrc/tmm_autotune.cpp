@@ -21,7 +21,11 @@
 //   * G in {1, 2, 4, ..., 64}, and one captured hipGraph vs the queues (pinned memory only): this
 //     ROCm's graph executor runs copy nodes one after the other, so with the graph H2D and D2H
 //     add up: T = max(H + D + c/G, C + h + d) without per-group host cost.
-// The persistent grid fills the CUs at the bodies' occupancy (2 workgroups per CU).
+// The persistent grid leaves a quarter of the CUs one of their two places: two workgroups take all the
+// registers of a CU until the group's last item, and copies that run as kernels (the runtime's own for
+// D2H, or tmm_copy.hip's) would wait for them. The 512-problem batch at the end of a process with other
+// handles 227 ms with the full grid, 213 with this one; 48 problems of 64 to 1024 2370-2437 and
+// 2325-2463 us.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -224,7 +228,7 @@ BatchConfig choose_batch_config(Handle& h, const BatchShape& shape) {
   if (std::max({*std::max_element(shape.m.begin(), shape.m.end()), *std::max_element(shape.n.begin(), shape.n.end()),
                 *std::max_element(shape.k.begin(), shape.k.end())}) > (1 << 25))
     best.body = 0;
-  best.workgroups = 2 * cus;
+  best.workgroups = 2 * cus - cus / 4;
   const double rate = best.body ? r.kernel_flops_dlds : r.kernel_flops;
   // native or emulated per problem; the compute total and the largest k of the native items
   const int cnt = (int)shape.m.size();
