@@ -318,7 +318,11 @@ __device__ __forceinline__ void tile_at(const GemmParams<typename T::R>& prm, bo
     t.template mma<0>(f);
     t.template mma<1>(f);
   }
-  if (ns > 0) {
+  // A wave without stages (ns = 0) runs through too: it loads nothing, waits for nothing, reads a slot
+  // whose contents are not used and multiplies none. With a branch around it the sums after the step
+  // above and those after the loop were two sets of registers, and 36 to 516 bytes per lane of
+  // the first spilled wherever the tile has 6 complex or 12 blocks and an operand is row-contiguous.
+  {
 #pragma unroll
     for (int s = 0; s < S; ++s)
       if (s < ns) issue(s);
