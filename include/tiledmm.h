@@ -126,8 +126,9 @@ const char* tmm_last_error(tmm_handle* h);
  * cublas_gemm_wrapper -> {s,d,c,z}gemm (tiled_mm.cpp:181-268). All pointers are device
  * pointers; stream = NULL runs on the handle's first compute stream. Asynchronous. A product with
  * a small C and a long inner dimension adds up partial sums in a buffer of up to 20 MB that the handle
- * allocates at the first one: such calls of one handle run one after the other, whatever their
- * streams (under stream capture they take neither the buffer nor the faster kernels). */
+ * allocates for a stream's first such call and keeps; up to 8 streams at a time have one of their own, beyond that
+ * such calls of one handle also wait for those of another stream (under stream capture they take
+ * neither a buffer nor the kernels that need it). */
 int tmm_device_gemm(tmm_handle* h, char trans_a, char trans_b, int m, int n, int k, const void* alpha,
                     const void* a, int ld_a, const void* b, int ld_b, const void* beta, void* c, int ld_c,
                     void* stream);

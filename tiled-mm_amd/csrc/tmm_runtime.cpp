@@ -210,9 +210,9 @@ Handle::~Handle() {
       if (ozwork_pending[i]) (void)hipEventSynchronize(ozwork_ev[i]);
       (void)hipEventDestroy(ozwork_ev[i]);
     }
-  if (split_ev) {
-    (void)hipEventSynchronize(split_ev);
-    (void)hipEventDestroy(split_ev);
+  for (SplitBuffer& b : split_buffers) {
+    (void)hipEventSynchronize(b.done);
+    (void)hipEventDestroy(b.done);
   }
   for (auto e : events) (void)hipEventDestroy(e);
   for (auto e : prof_events) (void)hipEventDestroy(e);
@@ -417,6 +417,32 @@ struct RelaxedCapture {
   ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
 };
 
+// The buffer of a split call on stream s: the one that the stream's last such call used, or one whose
+// calls have all run, or a new one, or the one used longest ago; null without memory for a first one.
+Handle::SplitBuffer* split_buffer(Handle& h, KsType type, hipStream_t s) {
+  Handle::SplitBuffer *idle = nullptr, *oldest = nullptr;
+  for (Handle::SplitBuffer& b : h.split_buffers) {
+    if (b.stream == s) return &b;
+    if (!oldest || b.used < oldest->used) oldest = &b;
+  }
+  RelaxedCapture relaxed;
+  for (Handle::SplitBuffer& b : h.split_buffers) {
+    if (hipEventQuery(b.done) == hipSuccess) idle = &b;
+    else (void)hipGetLastError();
+  }
+  if (idle) return idle;
+  if (h.split_buffers.size() >= Handle::kSplitBuffers) return oldest;
+  Handle::SplitBuffer fresh;
+  try {
+    fresh.work.reserve(split_bytes(type));
+    hip_check(hipEventCreateWithFlags(&fresh.done, hipEventDisableTiming), "hipEventCreate");
+  } catch (const Error&) {
+    return oldest;
+  }
+  h.split_buffers.push_back(std::move(fresh));
+  return &h.split_buffers.back();
+}
+
 // Runs a native device call with its tiles shared by several workgroups, if that is the faster way
 // (split_plan). Not under stream capture, where the graph could run beside any later call, and not
 // without memory for the partial sums.
@@ -433,19 +459,14 @@ bool launch_split(Handle& h, KsType type, const GemmParams<R>& p, hipStream_t s,
   }
   if (capture != hipStreamCaptureStatusNone) return false;
   std::lock_guard<std::mutex> lock(h.split_mu);
-  if (!h.split_ev) {
-    RelaxedCapture relaxed;
-    try {
-      h.split_work.reserve(split_bytes(type));
-    } catch (const Error&) {
-      return false;
-    }
-    hip_check(hipEventCreateWithFlags(&h.split_ev, hipEventDisableTiming), "hipEventCreate");
-  } else {
-    hip_check(hipStreamWaitEvent(s, h.split_ev, 0), "hipStreamWaitEvent (split products)");
-  }
-  hip_check(launch(p, plan.shape, plan.parts, h.split_work.ptr, s), "split GEMM launch");
-  hip_check(hipEventRecord(h.split_ev, s), "hipEventRecord (split products)");
+  Handle::SplitBuffer* buf = split_buffer(h, type, s);
+  if (!buf) return false;
+  hip_check(hipStreamWaitEvent(s, buf->done, 0), "hipStreamWaitEvent (split products)");
+  buf->stream = s;
+  buf->used = ++h.split_calls;
+  const hipError_t launched = launch(p, plan.shape, plan.parts, buf->work.ptr, s);
+  hip_check(hipEventRecord(buf->done, s), "hipEventRecord (split products)");
+  hip_check(launched, "split GEMM launch");
   return true;
 }
 

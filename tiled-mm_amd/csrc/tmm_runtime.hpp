@@ -154,12 +154,22 @@ struct Handle {
   // user waits for it (another stream) and a reallocation synchronises with it first
   std::vector<hipEvent_t> ozwork_ev;
   std::vector<char> ozwork_pending;
-  // partial sums of a device call whose inner dimension is split over workgroups (split_plan): one
-  // buffer, its calls ordered by split_ev on whatever streams they run; split_mu holds from the wait
-  // to the record, so that callers' threads need no order of their own
+  // partial sums of device calls whose inner dimension is split over workgroups (split_plan): a buffer
+  // per stream that has such calls under way, so that streams do not wait for each other; `done` is recorded
+  // behind the last call in a buffer, and a call waits for it first. Beyond kSplitBuffers busy streams (the
+  // device runs four hardware queues per process, so more than that do not run side by side) the
+  // buffer used longest ago is shared. split_mu holds from the choice to the record, so that callers' threads
+  // need no order of their own
+  struct SplitBuffer {
+    DeviceBuffer work;
+    hipEvent_t done = nullptr;
+    hipStream_t stream = nullptr;
+    long used = 0;  // number of the last call in it
+  };
+  static constexpr size_t kSplitBuffers = 8;
   std::mutex split_mu;
-  DeviceBuffer split_work;
-  hipEvent_t split_ev = nullptr;
+  std::deque<SplitBuffer> split_buffers;
+  long split_calls = 0;
   std::vector<DeviceBuffer> ozcache;  // scheme II prepared-operand slots, one buffer per compute queue
   DeviceBuffer batch_meta;           // batched path: problem descriptors, work items, counters
   TuneRates rates;
