@@ -371,9 +371,9 @@ int tmmh_simulate_gemm(int dtype, char opa, char opb, int m, int n, int k, const
 }
 
 // Blocks and chunks that pipeline_panels makes of the given ones for a product rate of flops_per_s:
-// out: tile_m, tile_n, tile_k, first chunk.
-int tmmh_pipeline_panels(int m, int n, int k, int beta_nonzero, int tm, int tn, int tk, int first_chunk, long budget,
-                         int elem_bytes, double flops_per_s, int* out) {
+// out: tile_m, tile_n, tile_k, first chunk. Returns the products that its estimates walked through.
+long tmmh_pipeline_panels_steps(int m, int n, int k, int beta_nonzero, int tm, int tn, int tk, int first_chunk,
+                                long budget, int elem_bytes, double flops_per_s, int* out) {
   PlanRequest rq;
   rq.m = m;
   rq.n = n;
@@ -384,12 +384,18 @@ int tmmh_pipeline_panels(int m, int n, int k, int beta_nonzero, int tm, int tn, 
   rq.tile_k = tk;
   rq.first_chunk_k = first_chunk;
   if (budget > 0) rq.pool_budget_elems = (size_t)budget;
-  pipeline_panels(rq, elem_bytes, 64, 8,
-                  [&](long a, long b, long c) { return 2.0 * a * (double)b * c / flops_per_s; });
+  const long steps = pipeline_panels(rq, elem_bytes, 64, 8, [&](long a, long b, long c) {
+    return 2.0 * a * (double)b * c / flops_per_s;
+  });
   out[0] = rq.tile_m;
   out[1] = rq.tile_n;
   out[2] = rq.tile_k;
   out[3] = rq.first_chunk_k;
+  return steps;
+}
+int tmmh_pipeline_panels(int m, int n, int k, int beta_nonzero, int tm, int tn, int tk, int first_chunk, long budget,
+                         int elem_bytes, double flops_per_s, int* out) {
+  tmmh_pipeline_panels_steps(m, n, k, beta_nonzero, tm, tn, tk, first_chunk, budget, elem_bytes, flops_per_s, out);
   return 0;
 }
 

@@ -295,21 +295,39 @@ Plan make_plan(const PlanRequest& rq) {
 
 namespace {
 // Estimated seconds of a call with rq's blocks: make_plan's order of copies and products (one group,
-// one compute queue), each queue working through its own in order.
-double call_seconds(const PlanRequest& rq, int es, const std::function<double(long, long, long)>& gemm_s) {
+// one compute queue), each queue working through its own in order. Returns `limit` as soon as it is known
+// that the call takes no less. steps: grows by the products walked through.
+double call_seconds(const PlanRequest& rq, int es, const std::function<double(long, long, long)>& gemm_s, double limit,
+                    long& steps) {
   const double kByte = es / 56e9, kCopy = 10e-6, kLaunch = 8e-6, kWake = 15e-6, kThreads = 60e-6;
   const int tm = std::min(rq.tile_m, rq.m), tn = std::min(rq.tile_n, rq.n);
   const int nm = (rq.m + tm - 1) / tm, nn = (rq.n + tn - 1) / tn;
+  const long blocks = (long)nm * nn;
   std::vector<int> kb(1, 0);
   if (rq.first_chunk_k > 0 && rq.first_chunk_k < rq.tile_k && rq.k > rq.tile_k) kb.push_back(rq.first_chunk_k);
   while (kb.back() < rq.k) kb.push_back((int)std::min<long>((long)kb.back() + rq.tile_k, rq.k));
   const int chunks = (int)kb.size() - 1;
+  std::vector<double> tile_s(chunks);
+  double left = 0;  // seconds of the products of the chunks to come
+  const double m = rq.m, n = rq.n, tiles = m / tm * (n / tn);
+  for (int c = 0; c < chunks; ++c) {
+    const int kc = kb[c + 1] - kb[c];
+    tile_s[c] = c > 0 && kc == kb[c] - kb[c - 1] ? tile_s[c - 1] : gemm_s(tm, tn, kc);
+    left += tile_s[c] * tiles + blocks * kLaunch;
+  }
+  // Neither queue of copies can take less than its own work, nor can the products (1e-9: the order of the sums).
+  const double tail = kWake + (blocks * chunks > 1 ? kThreads : 0.0), least = limit * (1 + 1e-9) - tail;
+  const double all_in = ((m + n) * rq.k + (rq.beta_nonzero ? m * n : 0)) * kByte +
+                        ((double)(nm + nn) * chunks + (rq.beta_nonzero ? blocks : 0)) * kCopy;
+  if (std::max({all_in, m * n * kByte + blocks * kCopy, left}) >= least) return limit;
   const auto order = shell_order(nm, nn);
   std::vector<double> a(nm), b(nn), cin(order.size(), 0.0);
   double in = 0, mul = 0, out = 0;
   for (int c = 0; c < chunks; ++c) {
+    if (mul + left >= least) return limit;
+    left -= tile_s[c] * tiles + blocks * kLaunch;
+    steps += blocks;
     const int kc = kb[c + 1] - kb[c];
-    const double tile_s = gemm_s(tm, tn, kc);
     std::fill(a.begin(), a.end(), -1.0);
     std::fill(b.begin(), b.end(), -1.0);
     for (size_t p = 0; p < order.size(); ++p) {
@@ -320,23 +338,24 @@ double call_seconds(const PlanRequest& rq, int es, const std::function<double(lo
       if (rq.beta_nonzero && c == (chunks == 1 ? 0 : 1 + (int)((long)p * (chunks - 1) / (long)order.size())))
         cin[p] = in += rows * cols * kByte + kCopy;
       mul = std::max({mul, a[i], b[j], c == chunks - 1 ? cin[p] : 0.0});
-      mul += tile_s * (rows / tm) * (cols / tn) + kLaunch;
+      mul += tile_s[c] * (rows / tm) * (cols / tn) + kLaunch;
       if (c == chunks - 1) out = std::max(out, mul + kWake) + rows * cols * kByte + kCopy;
     }
   }
-  return out + (order.size() * chunks > 1 ? kThreads : 0.0);
+  return out + (blocks * chunks > 1 ? kThreads : 0.0);
 }
 }  // namespace
 
-void pipeline_panels(PlanRequest& rq, int elem_bytes, int align, int k_align,
+long pipeline_panels(PlanRequest& rq, int elem_bytes, int align, int k_align,
                      const std::function<double(long, long, long)>& gemm_s) {
   const double m = rq.m, n = rq.n, k = rq.k, es = elem_bytes;
   const double bytes_in = es * (m * k + k * n + (rq.beta_nonzero ? m * n : 0)), bytes_out = es * m * n;
-  if (rq.k <= 0 || bytes_in + bytes_out < 8e6) return;
+  if (rq.k <= 0 || bytes_in + bytes_out < 8e6) return 0;
   const double whole = gemm_s(rq.tile_m, rq.tile_n, rq.k) * (m / rq.tile_m) * (n / rq.tile_n);
-  if (whole > 2 * std::max(bytes_in, bytes_out) / 56e9) return;
+  if (whole > 2 * std::max(bytes_in, bytes_out) / 56e9) return 0;
   const PlanRequest base = rq;
-  double least = 0.97 * call_seconds(base, elem_bytes, gemm_s);
+  long steps = 0;
+  double least = 0.97 * call_seconds(base, elem_bytes, gemm_s, HUGE_VAL, steps);
   auto edge = [align](int ext, int tile, int cut) {  // cut 1: the present blocks
     if (cut == 1) return tile;
     const long parts = (long)((ext + tile - 1) / tile) * cut;
@@ -361,7 +380,7 @@ void pipeline_panels(PlanRequest& rq, int elem_bytes, int align, int k_align,
         const double tk = std::min<double>(r.tile_k, k);
         const double pool = 2 * tk * (nm * r.tile_m + nn * r.tile_n) + (rq.beta_nonzero ? 2 : 1) * nm * nn * (double)r.tile_m * r.tile_n;
         if (pool > (double)rq.pool_budget_elems) continue;
-        const double t = call_seconds(r, elem_bytes, gemm_s);
+        const double t = call_seconds(r, elem_bytes, gemm_s, least, steps);
         if (t < least) {
           least = t;
           rq = r;
@@ -369,6 +388,7 @@ void pipeline_panels(PlanRequest& rq, int elem_bytes, int align, int k_align,
       }
     }
   }
+  return steps;
 }
 
 int operand_producer(const Plan& P, size_t gemm, Mat mat) {

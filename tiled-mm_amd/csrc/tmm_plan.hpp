@@ -107,8 +107,11 @@ Plan make_plan(const PlanRequest& rq);
 // rq: the request with its present blocks (tile_*, first_chunk_k), which stay where no cut gains 3%,
 // where the products take more than twice the link's time (both ends are then a small part), and in
 // calls of less than 8 MB, whose copies cost more apart than together. align: granularity of the cuts;
-// k_align: of the chunks.
-void pipeline_panels(PlanRequest& rq, int elem_bytes, int align, int k_align,
+// k_align: of the chunks. Returns the number of products that the estimates walked through. A cut is only
+// walked through while the work of each queue on its own leaves it a chance: the search runs on the caller's
+// thread in every call (DGEMM 10000^3 in 5120 x 5120 blocks 104 us; 2000 x 2000 x 100000 in k tiles of 1024, where no cut
+// can gain, 87 us, 2.3 ms when every cut was walked through).
+long pipeline_panels(PlanRequest& rq, int elem_bytes, int align, int k_align,
                      const std::function<double(long, long, long)>& gemm_s);
 
 // Index of the H2D op that filled the A (mat == Mat::A) or B operand block a GEMM op reads, or
