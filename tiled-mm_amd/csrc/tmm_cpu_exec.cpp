@@ -399,4 +399,7 @@ int tmmh_pipeline_panels(int m, int n, int k, int beta_nonzero, int tm, int tn, 
   return 0;
 }
 
+// Bytes of a staging piece of a call that moves call_bytes through the staging slots in one direction.
+long tmmh_stage_piece(long call_bytes, int whole) { return (long)stage_piece((size_t)call_bytes, whole != 0); }
+
 }  // extern "C"

@@ -114,6 +114,21 @@ Plan make_plan(const PlanRequest& rq);
 long pipeline_panels(PlanRequest& rq, int elem_bytes, int align, int k_align,
                      const std::function<double(long, long, long)>& gemm_s);
 
+// Pageable memory passes through page-locked staging slots in pieces: of a slot's size at most, and a part of the
+// bytes that the call moves that way (at least 8 MiB) in a smaller call, so that packing, DMA and scatter of
+// its pieces overlap (63 MB in and 45 MB out as three pieces: 3.3 ms, most of it one after the other). 1/64 where C is
+// one block by the call's tiles (whole; also once that is cut): nothing is scattered there before the last product.
+// 1/8 where C is several: packing and scattering then run together and share the host's threads, for which every
+// piece waits once more. ms with pieces of a slot / 1/8 / 1/64: DGEMM with a C read 9000 x 8800 x 2000 in four blocks
+// 24.4 / 24.7 / 28.0, 20000 x 8000 x 3000 in eight 45.9 / 46.0 / 52.2, ZGEMM 6100 x 6100 x 1000 in four 22.7 / 22.6 / 24.2;
+// one block: DGEMM 4000^3 12.2 / 11.8 / 11.1, 2000^3 - / 3.2 / 3.0, SGEMM 6000 x 3000 x 20000 - / 17.9 / 16.7.
+constexpr size_t kStageBytes = 128u << 20;
+constexpr size_t kStageMinPiece = 8u << 20;
+constexpr size_t stage_piece(size_t call_bytes, bool whole) {
+  const size_t part = call_bytes / (whole ? 64 : 8);
+  return part < kStageMinPiece ? kStageMinPiece : part > kStageBytes ? kStageBytes : part;
+}
+
 // Index of the H2D op that filled the A (mat == Mat::A) or B operand block a GEMM op reads, or
 // -1 when none of its dependencies did (the operand then has no identity to share).
 int operand_producer(const Plan& P, size_t gemm, Mat mat);

@@ -588,13 +588,7 @@ struct Scatterer {
 // scheme II DGEMM TN 40000^3 (host-link bound): 0.90-0.99 s per call with 6 x 64 MiB, 0.834 s with
 // 6 x 128 MiB, 0.838 with 4 x 256, 0.841 with 12 x 64, 0.825 with 12 x 128; the native call
 // (kernel bound) ran 1.856-1.862 s with every ring.
-// A piece is at most a slot, and 1/64 of the call's bytes (at least 8 MiB) in a smaller call, so that
-// packing, the DMA and the scatter of its pieces overlap (63 MB in and 45 MB out as three pieces:
-// 3.3 ms, most of it one after the other).
-constexpr size_t kStageBytes = 128u << 20;
-constexpr size_t kStageMinPiece = 8u << 20;
 constexpr int kStageSlots = 8;
-size_t stage_piece(size_t call_bytes) { return std::min(kStageBytes, std::max(kStageMinPiece, call_bytes / 64)); }
 
 // Cross-thread state of one plan execution (one thread per copy queue, the caller's thread for
 // the GEMMs). Every op is "marked" once it has been enqueued and, when another queue depends on
@@ -636,7 +630,8 @@ struct ExecSync {
   }
 };
 
-void execute_plan(Handle& h, const Plan& P, const GemmCall& call, const bool pinned[3], bool use_beta) {
+// whole: C is one block by the call's tiles (stage_piece).
+void execute_plan(Handle& h, const Plan& P, const GemmCall& call, const bool pinned[3], bool use_beta, bool whole) {
   const int es = h.elem_bytes;
   const size_t nops = P.ops.size();
   std::vector<char> need(nops, 0);
@@ -658,7 +653,7 @@ void execute_plan(Handle& h, const Plan& P, const GemmCall& call, const bool pin
 
   const bool any_pageable_in = !pinned[0] || !pinned[1] || (use_beta && !pinned[2]);
   const bool pageable_out = call.copy_back && !pinned[2];
-  const size_t piece_in = stage_piece(P.h2d_elems * es), piece_out = stage_piece(P.d2h_elems * es);
+  const size_t piece_in = stage_piece(P.h2d_elems * es, whole), piece_out = stage_piece(P.d2h_elems * es, whole);
   if (any_pageable_in) h.stage_in.ensure(kStageSlots, kStageBytes);
   if (pageable_out) h.stage_out.ensure(kStageSlots, kStageBytes);
   ThreadPool* tp = (any_pageable_in || pageable_out) ? &h.pool_threads() : nullptr;
@@ -1191,7 +1186,7 @@ void gemm_host(Handle& h, const GemmCall& in) {
     h.fullc_elems = need;
   }
 
-  execute_plan(h, P, call, pinned, use_beta);
+  execute_plan(h, P, call, pinned, use_beta, tm >= call.m && tn >= call.n);
 
   int ngemm = 0;
   for (auto& op : P.ops) ngemm += op.kind == OpKind::GEMM;
