@@ -1147,9 +1147,15 @@ void gemm_host(Handle& h, const GemmCall& in) {
     }
     rq.pool_budget_elems = budget / es;
   }
-  // calls to which the host link matters: smaller blocks (native products; the emulation shares
-  // prepared operands between whole blocks)
-  if (h.coarsen && call.copy_back && !ozaki_active(h) && h.first_chunk < 0) {
+  // Calls to which the host link matters: smaller blocks (native products; the emulation shares
+  // prepared operands between whole blocks). Not where a C of several blocks is read from pageable memory:
+  // it is packed, and scattered, by the host's threads at the same time, and for those smaller blocks are more and
+  // narrower pieces, which the estimate does not know. ms with / without smaller blocks, pageable, medians of three
+  // processes: DGEMM 9000 x 8800 x 2000 27 / 24.8, 20000 x 8000 x 3000 53 / 46, ZGEMM 6100 x 6100 x 1000 23 / 22.2, SGEMM 9000 x
+  // 8800 x 2000 16.2 / 14.5; without the C read they gain (DGEMM 10000 x 10000 x 4000 22 / 26), and with one block
+  // (8000 x 8000 x 2000 25 / 31).
+  const bool pageable_cin_blocks = use_beta && !pinned[2] && (tm < call.m || tn < call.n);
+  if (h.coarsen && call.copy_back && !ozaki_active(h) && h.first_chunk < 0 && !pageable_cin_blocks) {
     const KsType type = h.dtype == 0 ? KsType::S : h.dtype == 1 ? KsType::D : h.dtype == 2 ? KsType::C : KsType::Z;
     const int cus = h.cus;
     pipeline_panels(rq, es, 64, kstep, [type, cus](long m, long n, long k) {
