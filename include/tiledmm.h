@@ -230,7 +230,9 @@ int tmm_get_option(tmm_handle* h, int option, long* value);
 
 /* Statistics of the last host-to-host call, for measurement:
  *   stats[0] h2d bytes, [1] d2h bytes, [2] tile GEMM launches, [3] tile_m, [4] tile_n,
- *   [5] tile_k, [6] k-chunks, [7] wall seconds of the call, [8] 1 if A,B,C were all pinned;
+ *   [5] tile_k, [6] k-chunks (the blocks of C and the k-chunks that the call ran on; with
+ *   TMM_OPT_COARSEN the blocks are smaller than the tiles where the host link matters),
+ *   [7] wall seconds of the call, [8] 1 if A,B,C were all pinned;
  *   with TMM_OPT_PROFILE: [9] summed tile-GEMM kernel seconds, [10] launches timed, [11] their
  *   flops, [12] longest launch in seconds; [13] INT8 operations of the Ozaki path (2mnk per slice
  *   product); [14] 1 if the last batched call ran as one hipGraph, [15] its group count; with

@@ -37,3 +37,12 @@ def test_blocks_with_a_pageable_c_read_are_not_cut(torch_gpu, pinned_ab, pinned_
     assert st["k_chunks"] == 1
     assert (st["gemm_launches"] > BLOCKS) == cut, st
     assert cut or st["gemm_launches"] == BLOCKS, st
+
+
+@pytest.mark.parametrize("coarsen", [0, 1])
+@pytest.mark.parametrize("pinned", [False, True])
+def test_statistics_report_the_blocks_that_ran(torch_gpu, pinned, coarsen):
+    st = _call(pinned, pinned, 0.0, coarsen)
+    blocks = -(-M // int(st["tile_m"])) * -(-N // int(st["tile_n"]))
+    assert st["gemm_launches"] == blocks * st["k_chunks"], st
+    assert blocks > BLOCKS, st  # without coarsening 2 x 2 tiles, with it cut blocks

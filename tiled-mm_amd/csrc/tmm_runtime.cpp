@@ -1091,7 +1091,6 @@ void gemm_host(Handle& h, const GemmCall& in) {
     tn = align_edge(call.n, tn, align_n);
   }
 
-  const int block_m = tm, block_n = tn;
   PlanRequest rq;
   rq.opa = call.opa;
   rq.opb = call.opb;
@@ -1199,8 +1198,8 @@ void gemm_host(Handle& h, const GemmCall& in) {
   h.stats[0] = (double)P.h2d_elems * es;
   h.stats[1] = (double)P.d2h_elems * es;
   h.stats[2] = ngemm;
-  h.stats[3] = std::min(block_m, call.m);
-  h.stats[4] = std::min(block_n, call.n);
+  h.stats[3] = P.tile_m;
+  h.stats[4] = P.tile_n;
   h.stats[5] = P.tile_k;
   h.stats[6] = P.nTk;
   h.stats[7] = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
