@@ -245,6 +245,10 @@ int tmm_get_option(tmm_handle* h, int option, long* value);
  *   read and written once per operand use). n <= 24. */
 int tmm_last_call_stats(tmm_handle* h, double* stats, int n);
 
+/* How the handle's last tmm_device_gemm shared its tiles, for tests and measurement: *parts workgroups
+ * per tile of *edge rows and columns; 1 and 0 for a product that was not split. */
+int tmm_last_device_split(tmm_handle* h, int* edge, int* parts);
+
 #ifdef __cplusplus
 }
 #endif

@@ -359,4 +359,11 @@ int tmm_last_call_stats(tmm_handle* h, double* stats, int n) {
   return TMM_SUCCESS;
 }
 
+int tmm_last_device_split(tmm_handle* h, int* edge, int* parts) {
+  if (!h || !edge || !parts) return TMM_ERR_INVALID_ARG;
+  *edge = h->impl->last_split_edge;
+  *parts = h->impl->last_split_parts;
+  return TMM_SUCCESS;
+}
+
 }  // extern "C"

@@ -467,6 +467,8 @@ bool launch_split(Handle& h, KsType type, const GemmParams<R>& p, hipStream_t s,
   const hipError_t launched = launch(p, plan.shape, plan.parts, buf->work.ptr, s);
   hip_check(hipEventRecord(buf->done, s), "hipEventRecord (split products)");
   hip_check(launched, "split GEMM launch");
+  h.last_split_edge = 16 * kKsShapes[plan.shape].m;
+  h.last_split_parts = plan.parts;
   return true;
 }
 
@@ -1218,6 +1220,8 @@ void gemm_device(Handle& h, const GemmCall& in, hipStream_t s) {
   if (call.m == 0 || call.n == 0) return;
   const bool use_beta = !scalar_is_zero(h.dtype, call.beta);
   if (scalar_is_zero(h.dtype, call.alpha)) call.k = 0;  // C = beta*C; A and B are not read
+  h.last_split_edge = 0;
+  h.last_split_parts = 1;
   // In-place C: C_in and C_out are the same matrix, so the beta term reads each element
   // before the same thread overwrites it.
   if (launch_split(h, call, use_beta, s ? s : h.compute[0])) {

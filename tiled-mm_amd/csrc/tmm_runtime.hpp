@@ -170,6 +170,7 @@ struct Handle {
   std::mutex split_mu;
   std::deque<SplitBuffer> split_buffers;
   long split_calls = 0;
+  std::atomic<int> last_split_edge{0}, last_split_parts{1};  // of the last device call: tile edge, workgroups per tile
   std::vector<DeviceBuffer> ozcache;  // scheme II prepared-operand slots, one buffer per compute queue
   DeviceBuffer batch_meta;           // batched path: problem descriptors, work items, counters
   TuneRates rates;

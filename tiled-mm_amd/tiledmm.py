@@ -64,6 +64,7 @@ def load():
         lib.tmm_set_option.argtypes = [vp, i, ctypes.c_long]
         lib.tmm_get_option.argtypes = [vp, i, ctypes.POINTER(ctypes.c_long)]
         lib.tmm_last_call_stats.argtypes = [vp, ctypes.POINTER(d), i]
+        lib.tmm_last_device_split.argtypes = [vp, ctypes.POINTER(i), ctypes.POINTER(i)]
         lib.tmm_full_c_device_ptr.argtypes = [vp, ctypes.POINTER(vp), ctypes.POINTER(ctypes.c_size_t)]
         lib.tmm_tile_buffer.argtypes = [vp, i, i, ctypes.POINTER(vp), ctypes.POINTER(ctypes.c_size_t)]
         lib.tmm_get_stream.argtypes = [vp, i, ctypes.POINTER(vp)]
@@ -193,6 +194,12 @@ class Handle:
                 "batch_graph", "batch_groups", "group_launches", "group_kernel_s", "group_flops", "host_c_written", "batch_body", "batch_queues",
                 "batch_emulated", "group_bytes"]
         return dict(zip(keys, list(arr)))
+
+    def last_device_split(self):
+        """(tile edge, workgroups per tile) of the last device_gemm; (0, 1) if it was not split."""
+        edge, parts = ctypes.c_int(), ctypes.c_int()
+        self._check(load().tmm_last_device_split(self._h, ctypes.byref(edge), ctypes.byref(parts)))
+        return edge.value, parts.value
 
     def gemm_batched(self, ta, tb, ms, ns, ks, alphas, As, ldas, Bs, ldbs, betas, Cs, ldcs):
         """Batched host-to-host DGEMM (tmm_dgemm_batched); As/Bs/Cs: lists of arrays or pointers."""
