@@ -1676,6 +1676,11 @@ Route route(KsType t, const GemmParams<R>& p) {
   const bool chunks_ok = ks_chunks_ok<R>(cplx, p.opa != 'N', p.m, p.lda) && ks_chunks_ok<R>(cplx, p.opb == 'N', p.n, p.ldb);
   const bool pipe = tiles >= 2L * cus && chunks_ok;
   if (!ks_takes(p, cplx)) return {pipe ? Route::kPipe : Route::kReal, 0};
+  if (short_inner(t, p.m, p.n, p.k, cus)) {
+    const bool reads_c = p.accumulate || p.beta != R(0) || (cplx && p.beta_im != R(0));
+    const ShortKernel x = short_kernel(t, p.m, p.n, p.k, reads_c, cus);
+    return {x == ShortKernel::Pipe ? Route::kPipe : x == ShortKernel::Real ? Route::kReal : Route::kKs, kShortShape};
+  }
   double us = 0;
   const int shape = ks_shape(t, p.m, p.n, p.k, cus, &us);
   // Two k-contiguous real operands with leading dimensions off 64 bytes: a 64-byte row chunk of a

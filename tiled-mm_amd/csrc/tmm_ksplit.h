@@ -96,6 +96,42 @@ inline double product_time(KsType t, long m, long n, long k, int cus) {
   return tiles >= 2L * cus ? std::min(us, pipe_time(t, tiles, k, cus)) : us;
 }
 
+// Products with a short inner dimension and more than two 32 x 32 tiles per CU (no side within one of 16): the times above count a tile's
+// first loads and its C once per product, which is right for a long inner dimension or few tiles; here they
+// are most of the work of every tile. Kernel by kernel, in us: a product, every round of its tiles over
+// the CUs, and each k of a round. Fitted to 50 products per type without and 50 with a C that is read, from 399 x 4207 to
+// 6874 x 1710 with k from 1 on (4 to 16% rms); the choice they lead to is 0.5 to 2.5% behind the fastest kernel on
+// average (complex double with a C read 4%). With the times above 16 x 16 tiles were taken for the shortest: in us, with
+// these / with those, SGEMM 2000 x 2000 x 1 9.8 / 27, 6000 x 6000 x 1 36 / 160; DGEMM 2000 x 2000 x 1 12.3 / 28, x 64
+// 19.6 / 24.4, 6000 x 6000 x 8 67 / 89; ZGEMM 6000 x 6000 x 64 308 / 419; CGEMM 2000 x 2000 x 64 25 / 31.
+struct ShortCost {
+  double product, round, k;
+};
+enum class ShortKernel { Ks32, Pipe, Real };  // 32 x 32 k-split, pipelined, register-staged tiles
+constexpr int kShortMaxK[4] = {128, 256, 128, 128};
+constexpr int kShortShape = 3;  // 32 x 32 in kKsShapes
+inline bool short_inner(KsType t, long m, long n, long k, int cus) {
+  return k <= kShortMaxK[(int)t] && m > 16 && n > 16 && ks_tiles(kKsShapes[kShortShape], m, n) > 2L * cus;
+}
+// reads_c: beta or an accumulation reads C, which the large tiles do with too little in flight: only complex double's
+// (64 x 64) can win then.
+inline ShortKernel short_kernel(KsType t, long m, long n, long k, bool reads_c, int cus) {
+  constexpr ShortCost ks[4] = {{3.9, 0.70, 0.0068}, {3.8, 0.63, 0.0036}, {4.0, 1.06, 0.0266}, {3.6, 0.79, 0.0136}};
+  constexpr ShortCost pipe[4] = {{8.9, 8.3, 0.118}, {5.5, 3.4, 0.057}, {3.2, 2.6, 0.106}, {4.6, 6.1, 0.220}};
+  constexpr ShortCost real_d = {4.3, 6.6, 0.128};  // stores its C faster than the pipelined kernel
+  constexpr ShortCost ks_zc = {3.3, 1.67, 0.026}, pipe_zc = {5.5, 5.8, 0.1035};
+  if (reads_c && t != KsType::Z) return ShortKernel::Ks32;
+  auto time = [&](const ShortCost& c, long edge) {
+    const long rounds = (((m + edge - 1) / edge) * ((n + edge - 1) / edge) + cus - 1) / cus;
+    return c.product + rounds * (c.round + k * c.k);
+  };
+  const double a = time(reads_c ? ks_zc : ks[(int)t], 32);
+  const double b = time(reads_c ? pipe_zc : pipe[(int)t], t == KsType::Z ? 64 : 128);
+  if (t == KsType::D && time(real_d, 128) < std::min(a, b)) return ShortKernel::Real;
+  // complex float's pipelined times scatter most: 10% in hand
+  return b < (t == KsType::C ? 0.9 : 1.0) * a ? ShortKernel::Pipe : ShortKernel::Ks32;
+}
+
 // Whether an operand's 16-byte row chunks reach over the end of at most one column (a chunk of 4
 // floats over the end of a column, or of two complex floats, of a leading dimension below its size).
 template <typename R>
