@@ -18,7 +18,7 @@
 //   * the compute queue count (1 or 2): with 2, consecutive groups' kernels may overlap, which
 //     hides the last partial wave of each group (modelled as one tile of the group's largest k per
 //     group);
-//   * G in {1, 2, 4, ..., 64}, and one captured hipGraph vs the queues (pinned memory only): this
+//   * G in {1, 2, 4, ..., 64}, and one captured hipGraph vs the queues (pinned memory copied by DMA only): this
 //     ROCm's graph executor runs copy nodes one after the other, so with the graph H2D and D2H
 //     add up: T = max(H + D + c/G, C + h + d) without per-group host cost.
 // The persistent grid leaves a quarter of the CUs one of their two places: two workgroups take all the
@@ -256,7 +256,9 @@ BatchConfig choose_batch_config(Handle& h, const BatchShape& shape) {
   // a group's last partial wave: about one tile of the largest k on one workgroup's share
   const double edge = batched_tile(best.body), tail = 2.0 * edge * edge * (double)kmax / (rate / (2.0 * cus));
   const double hsum = shape.h2d_bytes / r.h2d_Bps, dsum = shape.d2h_bytes / r.d2h_Bps;
-  const bool graph_ok = shape.pinned && h.batch_graph != 0, graph_only = graph_ok && h.batch_graph == 1;
+  // the graph's model is that of its copy nodes; a batch that can be copied by kernels runs on the queues
+  const bool graph_ok = shape.pinned && (h.batch_graph == 1 || (h.batch_graph != 0 && !shape.kernel_copies));
+  const bool graph_only = graph_ok && h.batch_graph == 1;
   for (int G = 1; G <= 64; G *= 2) {
     if (G > std::max(1, shape.count)) break;
     for (int q = 1; q <= 2; ++q) {

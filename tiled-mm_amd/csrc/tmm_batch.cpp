@@ -47,7 +47,9 @@ struct Prob {
 // 3112; padded, 294 KB 2360 / 1250, 570 KB 4640 / 3130, 846 KB 3160 / 2617, 1250 KB 2754 / 2436. Never both
 // in one batch: where the streams share hardware queues, as in a process with other handles, the
 // copy kernels then wait for DMA commands and for each other (867 KB: 2300 in a first handle, 3100
-// to 3800 in later ones).
+// to 3800 in later ones). Nor in a captured graph, whose copies are memory copy nodes: the graph saves nothing
+// once a group is three launches (200 problems of 16 to 100: 987 us a call with the graph to choose from, 1019 on the
+// queues).
 constexpr double kKernelCopyBytes = 768 << 10, kKernelCopyPaddedBytes = 1536 << 10;
 constexpr int kCopyInWorkgroups = 64, kCopyOutWorkgroups = 32;
 
@@ -134,8 +136,9 @@ void gemm_batched_host(Handle& h, char opa, char opb, int count, const int* m, c
     add(p.map_b, p.rowsB, p.colsB, p.ldb, 1);
     add(p.map_c, p.m, p.n, p.ldc, p.beta != 0.0 ? 2 : 1);
   }
-  const bool by_kernel = mapped && shape.h2d_bytes + shape.d2h_bytes <= copy_limit;
+  shape.kernel_copies = mapped && shape.h2d_bytes + shape.d2h_bytes <= copy_limit;
   BatchConfig cfg = choose_batch_config(h, shape);
+  const bool by_kernel = shape.kernel_copies && !cfg.use_graph;
   cfg.queues = std::max(1, std::min(cfg.queues, (int)h.compute.size()));
   // emulated problems: one workspace per compute queue (groups alternate over the queues),
   // reserved before any capture

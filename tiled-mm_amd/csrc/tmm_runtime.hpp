@@ -95,6 +95,7 @@ struct BatchShape {
   int count = 0;
   double flops = 0, h2d_bytes = 0, d2h_bytes = 0;
   bool pinned = false;
+  bool kernel_copies = false;  // small enough for copies by kernel, unless the call runs as a graph
   std::vector<int> m, n, k;  // per problem
 };
 struct BatchConfig {
