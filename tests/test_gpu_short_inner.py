@@ -12,9 +12,9 @@ from test_gpu_ragged import CODES, _ops
 pytestmark = pytest.mark.gpu
 
 
-# one k, whole and partial k-steps, both sides of the longest short one; sizes of less than one 128 x 128 tile per
+# one k, whole and partial k-steps, both sides of each type's longest short one; sizes of less than one 128 x 128 tile per
 # CU, one, and several
-@pytest.mark.parametrize("k", [1, 8, 33, 64, 128, 129, 256, 257])
+@pytest.mark.parametrize("k", [1, 8, 33, 64, 128, 129, 160, 161, 256, 257, 512, 513])
 @pytest.mark.parametrize("m,n", [(897, 705), (2001, 1999), (3003, 2817)])
 @pytest.mark.parametrize("dtype", list(CODES), ids=["s", "d", "c", "z"])
 def test_short_inner_dimension_exact(torch_gpu, dtype, m, n, k):

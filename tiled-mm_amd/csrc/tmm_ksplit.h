@@ -103,12 +103,13 @@ inline double product_time(KsType t, long m, long n, long k, int cus) {
 // 6874 x 1710 with k from 1 on (4 to 16% rms); the choice they lead to is 0.5 to 2.5% behind the fastest kernel on
 // average (complex double with a C read 4%). With the times above 16 x 16 tiles were taken for the shortest: in us, with
 // these / with those, SGEMM 2000 x 2000 x 1 9.8 / 27, 6000 x 6000 x 1 36 / 160; DGEMM 2000 x 2000 x 1 12.3 / 28, x 64
-// 19.6 / 24.4, 6000 x 6000 x 8 67 / 89; ZGEMM 6000 x 6000 x 64 308 / 419; CGEMM 2000 x 2000 x 64 25 / 31.
+// 19.6 / 24.4, 6000 x 6000 x 8 67 / 89; ZGEMM 6000 x 6000 x 64 308 / 419; CGEMM 2000 x 2000 x 64 25 / 31; near the upper
+// end SGEMM 3073 x 6846 x 309 139 / 169, DGEMM 4258 x 1250 x 144 41 / 50, ZGEMM 3941 x 5734 x 187 531 / 587.
 struct ShortCost {
   double product, round, k;
 };
 enum class ShortKernel { Ks32, Pipe, Real };  // 32 x 32 k-split, pipelined, register-staged tiles
-constexpr int kShortMaxK[4] = {128, 256, 128, 128};
+constexpr int kShortMaxK[4] = {160, 512, 256, 128};  // above, the times further up choose as well or better
 constexpr int kShortShape = 3;  // 32 x 32 in kKsShapes
 inline bool short_inner(KsType t, long m, long n, long k, int cus) {
   return k <= kShortMaxK[(int)t] && m > 16 && n > 16 && ks_tiles(kKsShapes[kShortShape], m, n) > 2L * cus;
