@@ -129,8 +129,7 @@ inline ShortKernel short_kernel(KsType t, long m, long n, long k, bool reads_c, 
   const double a = time(reads_c ? ks_zc : ks[(int)t], 32);
   const double b = time(reads_c ? pipe_zc : pipe[(int)t], t == KsType::Z ? 64 : 128);
   if (t == KsType::D && time(real_d, 128) < std::min(a, b)) return ShortKernel::Real;
-  // complex float's pipelined times scatter most: 10% in hand
-  return b < (t == KsType::C ? 0.9 : 1.0) * a ? ShortKernel::Pipe : ShortKernel::Ks32;
+  return b < a ? ShortKernel::Pipe : ShortKernel::Ks32;
 }
 
 // Whether an operand's 16-byte row chunks reach over the end of at most one column (a chunk of 4
