@@ -181,7 +181,8 @@ int tmm_synchronize(tmm_handle* h);
  *                        chooses between capturing the call's copies and launches into one
  *                        hipGraph (no per-group host overhead; the graph runs its copies one
  *                        after the other) and enqueueing them on the three queues (H2D and D2H
- *                        overlap); 1 always the graph; 0 never.
+ *                        overlap; always, where the matrices are small enough to be copied by
+ *                        kernels); 1 always the graph; 0 never.
  *   TMM_OPT_BATCH_BODY   tmm_dgemm_batched tile body: -1 (default) the autotuner's choice (the faster
  *                        one measured), 0 register-staged LDS double buffer, 1 direct-to-LDS rings with the inner
  *                        dimension split over the waves. A batch with a dimension above 2^25 runs on 0.
@@ -203,11 +204,14 @@ int tmm_synchronize(tmm_handle* h);
  *                        own products, as for native calls. Same results.
  *   TMM_OPT_DGEMM_KERNEL tile kernels of every element type: 1 (default) = direct global->LDS
  *                        loads: small tiles that split the inner dimension over a workgroup's
- *                        waves, or, with at least two workgroup tiles per CU and where they are
- *                        estimated to be faster, software-pipelined 128 x 128 tiles (complex
- *                        double 64 x 64; FP64 128 x 256 from 2^27 elements of C on); 0 = LDS
- *                        double buffer filled through registers (the kernel that variant 1 also
- *                        uses for k = 0 and for leading dimensions beyond 256 MB). */
+ *                        waves, or software-pipelined 128 x 128 tiles (complex double 64 x 64;
+ *                        FP64 128 x 256 from 2^27 elements of C on), whichever is estimated to be
+ *                        faster (the pipelined ones with at least two per CU or a short inner
+ *                        dimension); 0 = LDS double buffer filled through registers. Variant 1 uses
+ *                        that one for k = 0, for some FP64 products with a short inner dimension,
+ *                        for FP32 with a row-contiguous operand of leading dimension 1 or 2 and a
+ *                        row count off 4, and for leading dimensions beyond 256 MB where there are
+ *                        fewer than two pipelined tiles per CU. */
 enum {
   TMM_OPT_COARSEN = 1,
   TMM_OPT_FIRST_CHUNK = 2,

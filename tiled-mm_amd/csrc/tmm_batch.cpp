@@ -44,7 +44,8 @@ struct Prob {
 // outweigh the transfers, above it a kernel's reads over the link slow the tile kernels beside it
 // (their loads wait behind them in the L2). us per call by DMA / by kernel: contiguous, mean 78 KB
 // 2009 / 936, 432 KB 885 / 790, 703 KB 3070 / 2875, 733 KB 728 / 680, 867 KB 2370 / 2650, 1203 KB 2627 /
-// 3112; padded, 294 KB 2360 / 1250, 570 KB 4640 / 3130, 846 KB 3160 / 2617, 1250 KB 2754 / 2436. Never both
+// 3112; padded, 294 KB 2360 / 1250, 570 KB 4640 / 3130, 846 KB 3160 / 2617, 1250 KB 2754 / 2436 (the kernel still ahead:
+// where it falls behind was not measured, the limit is set by analogy). Never both
 // in one batch: where the streams share hardware queues, as in a process with other handles, the
 // copy kernels then wait for DMA commands and for each other (867 KB: 2300 in a first handle, 3100
 // to 3800 in later ones). Nor in a captured graph, whose copies are memory copy nodes: the graph saves nothing

@@ -1653,7 +1653,8 @@ long grid_tiles(int m, int n, int bm, int bn) { return (long)((m + bm - 1) / bm)
 
 // Which kernels a product runs on: a function of the product alone, so that a grouped launch gives
 // each of its products the bits of a launch of its own.
-//   kReal  register-staged (variant 0, k = 0, an extreme leading dimension);
+//   kReal  register-staged (variant 0, k = 0; what the other two do not take: ks_chunks_ok, and
+//          leading dimensions beyond 256 MB below two pipelined tiles per CU; some short k);
 //   kKs    the small tiles that split k over a workgroup's waves, of shape `shape`;
 //   kPipe  the pipelined 128 x 128 (complex double: 64 x 64) tiles, for which there must be two per
 //          CU, where the estimated times say so. Their times lie within a few percent of each
@@ -1690,6 +1691,12 @@ Route route(KsType t, const GemmParams<R>& p) {
   // operands lose 1%. By the leading dimension alone, so that the route does not hang on addresses.
   if (!cplx && p.opa != 'N' && p.opb == 'N' && p.lda * (long)sizeof(R) % 64 != 0 && p.ldb * (long)sizeof(R) % 64 != 0)
     us *= 1 + 0.13 * std::min(1.0, p.k * (double)sizeof(R) / 64000);
+  // The largest complex double products of one k-contiguous and one row-contiguous operand: the 48 x 48 tiles lead by
+  // 2 to 4% below (NN 12000 x 12000 x 16000 258 ms against 265, 24000 x 24000 x 8000 521 against 523), and fall behind above
+  // (16000 x 16000 x 32000 951 against 935, 24000 x 24000 x 16000 1072 against 1046, x 32000 2171 against 2092); TT likewise. With
+  // operands of one kind they lead throughout (TN 24000 x 24000 x 16000 1022 against 1053).
+  const bool mixed = (p.opa != 'N') != (p.opb == 'N');
+  if (t == KsType::Z && pipe && mixed && (double)p.m * p.n * p.k > 6e12) return {Route::kPipe, 0};
   const bool many = t != KsType::Z && tiles >= 12L * cus;
   if (pipe && (many || 0.98 * pipe_time(t, tiles, p.k, cus) <= us)) return {Route::kPipe, 0};
   return {Route::kKs, shape};
