@@ -1865,15 +1865,19 @@ hipError_t launch_many(const Kernels<R>& k, const GemmParams<R>* tiles, int coun
   if (count > kDgemmGroupMax) return hipErrorInvalidValue;
   GemmParams<R> pipe[kDgemmGroupMax], ks[kDgemmGroupMax];
   int npipe = 0, nks = 0;
+  long ks_group_tiles = 0;  // at least the grid: group tiles are 48 x 48 (complex) or larger, products start on multiples of 8
   hipError_t e = hipSuccess;
   for (int t = 0; t < count && e == hipSuccess; ++t) {
     const Route::Kind kind = route(k.type, tiles[t]).kind;
-    if (kind == Route::kKs) ks[nks++] = tiles[t];
-    else if (kind == Route::kPipe) pipe[npipe++] = tiles[t];
+    if (kind == Route::kKs) {
+      ks[nks++] = tiles[t];
+      ks_group_tiles += ks_tiles(KsShape{3, 3}, tiles[t].m, tiles[t].n) + 7;
+    } else if (kind == Route::kPipe) pipe[npipe++] = tiles[t];
     else e = launch_one(k, tiles[t], s);
   }
   if (e == hipSuccess && npipe > 0) e = k.pipe_group(pipe, npipe, s);
-  if (e == hipSuccess && nks > 0) e = nks == 1 ? launch_one(k, ks[0], s) : k.ks_group(ks, nks, s);
+  if (nks > 1 && ks_group_tiles <= kKsMaxTiles) return e == hipSuccess ? k.ks_group(ks, nks, s) : e;
+  for (int t = 0; t < nks && e == hipSuccess; ++t) e = launch_one(k, ks[t], s);
   return e;
 }
 

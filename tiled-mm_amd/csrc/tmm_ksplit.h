@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <limits>
 
 #include "tmm_kernels.h"
 
@@ -74,13 +75,19 @@ inline double pipe_time(KsType t, long tiles, long k, int cus) {
 
 inline long ks_tiles(KsShape s, long m, long n) { return ((m + 16 * s.m - 1) / (16 * s.m)) * ((n + 16 * s.n - 1) / (16 * s.n)); }
 
-// Fastest shape for an m x n x k product, and its time in us.
+// Tiles of one launch: a grid holds fewer than 2^32 threads, 256 per tile. The largest C's that fit the device have more
+// small tiles than that (131072 x 131072, 69 GB in FP32, has 2^24 of 32 x 32; so has a C of 2^29 x 1 in 32 x 16).
+constexpr long kKsMaxTiles = (1L << 24) - 1;
+
+// Fastest shape for an m x n x k product, and its time in us (infinite if none has few enough tiles).
 inline int ks_shape(KsType t, long m, long n, long k, int cus, double* us) {
   int best = 0;
-  double least = 0;
+  double least = std::numeric_limits<double>::infinity();
   for (int i = 0; i < kKsShapeCount[(int)t]; ++i) {
-    const double x = ks_time(t, kKsShapes[i], ks_tiles(kKsShapes[i], m, n), k, cus);
-    if (i == 0 || x < least) {
+    const long tiles = ks_tiles(kKsShapes[i], m, n);
+    if (tiles > kKsMaxTiles) continue;
+    const double x = ks_time(t, kKsShapes[i], tiles, k, cus);
+    if (x < least) {
       least = x;
       best = i;
     }
@@ -113,7 +120,8 @@ enum class ShortKernel { Ks32, Pipe, Real };  // 32 x 32 k-split, pipelined, reg
 constexpr int kShortMaxK[4] = {160, 512, 256, 128};  // above, the times further up choose as well or better
 constexpr int kShortShape = 3;  // 32 x 32 in kKsShapes
 inline bool short_inner(KsType t, long m, long n, long k, int cus) {
-  return k <= kShortMaxK[(int)t] && m > 16 && n > 16 && ks_tiles(kKsShapes[kShortShape], m, n) > 2L * cus;
+  const long tiles = ks_tiles(kKsShapes[kShortShape], m, n);
+  return k <= kShortMaxK[(int)t] && m > 16 && n > 16 && tiles > 2L * cus && tiles <= kKsMaxTiles;
 }
 // reads_c: beta or an accumulation reads C, which the large tiles do with too little in flight: only complex double's
 // (64 x 64) can win then.
