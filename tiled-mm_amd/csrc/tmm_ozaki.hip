@@ -91,12 +91,15 @@ __device__ __forceinline__ void exponents16(const OperandSrc& o, int block, int*
   }
 }
 
-// Exponents of two operands, the second's workgroups behind the first's.
+// Exponents of two operands, the second's workgroups behind the first's. A grid holds fewer than 2^32 threads in one
+// dimension, which 2^26 rows exceed: from kExpGridX workgroups on they go on in the second one.
+constexpr int kExpGridX = 1 << 20;
 __global__ __launch_bounds__(1024) void exponents_kernel(OperandSrc a, OperandSrc b) {
   __shared__ int lds[256];
-  const int na = (a.rows + kExpRows - 1) / kExpRows;
-  if ((int)blockIdx.x < na) exponents16(a, blockIdx.x, lds);
-  else exponents16(b, blockIdx.x - na, lds);
+  const int w = (int)(blockIdx.y * gridDim.x + blockIdx.x);
+  const int na = (a.rows + kExpRows - 1) / kExpRows, nb = (b.rows + kExpRows - 1) / kExpRows;
+  if (w < na) exponents16(a, w, lds);
+  else if (w - na < nb) exponents16(b, w - na, lds);
 }
 
 // *flag from the operand's exponents, by one workgroup. Inf and NaN have frexp-exponent 1025, so an
@@ -522,7 +525,10 @@ hipError_t launch_exponents(const OperandSrc* o, int count, hipStream_t s) {
   OperandSrc none{};
   const OperandSrc& b = count > 1 ? o[1] : none;
   const int blocks = (o[0].rows + kExpRows - 1) / kExpRows + (b.rows + kExpRows - 1) / kExpRows;
-  if (blocks > 0) hipLaunchKernelGGL(exponents_kernel, dim3(blocks), dim3(1024), 0, s, o[0], b);
+  if (blocks > 0) {
+    const dim3 grid(std::min(blocks, kExpGridX), (blocks + kExpGridX - 1) / kExpGridX);
+    hipLaunchKernelGGL(exponents_kernel, grid, dim3(1024), 0, s, o[0], b);
+  }
   return hipGetLastError();
 }
 }  // namespace
